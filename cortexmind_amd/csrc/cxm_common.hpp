@@ -200,6 +200,58 @@ __device__ __forceinline__ void st4_stream(float *p, float4 v) {
     __builtin_nontemporal_store(f32x4{v.x, v.y, v.z, v.w}, reinterpret_cast<f32x4 *>(p));
 }
 
+// The same accesses at 4-byte alignment: gfx950 takes a dwordx4 access at
+// any dword address, so a ragged row (length not a multiple of 4, or a base
+// that is not 16-byte aligned) keeps 128-bit loads and stores.  A wave's
+// 1 KiB then touches nine 128-byte lines instead of eight.
+typedef float f32x4u __attribute__((ext_vector_type(4), aligned(4)));
+template <bool AL>
+__device__ __forceinline__ float4 ld4_any(const float *p) {
+    if constexpr (AL) return ld4(p);
+    const f32x4u v = *reinterpret_cast<const f32x4u *>(p);
+    return make_float4(v.x, v.y, v.z, v.w);
+}
+template <bool AL>
+__device__ __forceinline__ float4 ld4_any_stream(const float *p) {
+    if constexpr (AL) return ld4_stream(p);
+    const f32x4u v = __builtin_nontemporal_load(reinterpret_cast<const f32x4u *>(p));
+    return make_float4(v.x, v.y, v.z, v.w);
+}
+// Stores of a ragged row are temporal: neighbouring waves share the line at
+// their seam, and L2 merges the two halves.
+template <bool AL>
+__device__ __forceinline__ void st4_any_stream(float *p, float4 v) {
+    if constexpr (AL) st4_stream(p, v);
+    else *reinterpret_cast<f32x4u *>(p) = f32x4u{v.x, v.y, v.z, v.w};
+}
+
+// Float4 number i of a run of n floats at 4-byte alignment, n >= 4 or at
+// least 4 - n floats of the same row before it: the load goes to offset
+// tail_off (whole float4s at 4 i, everything past them at the last four
+// floats of the run), so every lane's load is in bounds and none needs a
+// branch; tail_keep then replaces the components that belong to another
+// float4 (or to none) by `pad`.
+__device__ __forceinline__ int tail_off(int i, int n) { return 4 * i < n - 4 ? 4 * i : n - 4; }
+__device__ __forceinline__ float4 tail_keep(float4 v, int i, int off, float4 pad) {
+    const int d = 4 * i - off;  // components below d belong to earlier float4s
+    v.x = d > 0 ? pad.x : v.x;
+    v.y = d > 1 ? pad.y : v.y;
+    v.z = d > 2 ? pad.z : v.z;
+    v.w = d > 3 ? pad.w : v.w;
+    return v;
+}
+// Stores float4 i of such a run: whole, or the components of the tail.
+__device__ __forceinline__ void tail_store(float *p, float4 v, int i, int off) {
+    const int d = 4 * i - off;
+    if (d <= 0) {
+        st4_any_stream<false>(p + off, v);
+    } else if (d < 4) {
+        if (d <= 1) p[off + 1] = v.y;
+        if (d <= 2) p[off + 2] = v.z;
+        p[off + 3] = v.w;
+    }
+}
+
 // Direct global-to-LDS load of 16 bytes per lane (global_load_lds_dwordx4):
 // lane L's 16 bytes at gsrc land at LDS byte lds + 16 L (lds wave-uniform,
 // placed in M0).  Issued through inline asm so that the compiler's wait
@@ -393,6 +445,19 @@ __device__ __forceinline__ Pow2 readlane(Pow2 p, int lane) {
     return {readlane(p.s1, lane), readlane(p.s2, lane)};
 }
 
+// The value of lane ^ 16 (within each half of the wave; ds_swizzle's xor
+// mode: and-mask 0x1f, xor-mask 0x10).
+__device__ __forceinline__ int swap16(int v) { return __builtin_amdgcn_ds_swizzle(v, (0x10 << 10) | 0x1f); }
+__device__ __forceinline__ float swap16(float v) {
+    return __builtin_bit_cast(float, swap16(__builtin_bit_cast(int, v)));
+}
+__device__ __forceinline__ ArgPair swap16(ArgPair p) { return {swap16(p.v), swap16(p.i)}; }
+__device__ __forceinline__ double swap16(double v) {
+    const unsigned long long u = __builtin_bit_cast(unsigned long long, v);
+    return dbl_from(swap16(static_cast<int>(u)), swap16(static_cast<int>(u >> 32)));
+}
+__device__ __forceinline__ Pow2 swap16(Pow2 p) { return {swap16(p.s1), swap16(p.s2)}; }
+
 // Reduce across the 64 lanes of a wave; every lane gets the result.
 // Must be called with all 64 lanes active.
 template <class Op>
@@ -404,6 +469,23 @@ __device__ __forceinline__ typename Op::T wave_reduce(typename Op::T v) {
     typename Op::T r = Op::combine(Op::combine(readlane(v, 0), readlane(v, 16)),
                                    Op::combine(readlane(v, 32), readlane(v, 48)));
     return r;
+}
+
+// Reduce across groups of G lanes (G a power of two from 4); every lane of
+// a group gets its group's result.  All 64 lanes must be active.
+template <class Op, int G>
+__device__ __forceinline__ typename Op::T group_reduce(typename Op::T v) {
+    if constexpr (G == kWave) {
+        return wave_reduce<Op>(v);
+    } else {
+        static_assert(G == 4 || G == 8 || G == 16 || G == 32, "group of 4 to 32 lanes");
+        v = Op::combine(v, dpp<kQuadXor1>(v));
+        v = Op::combine(v, dpp<kQuadXor2>(v));
+        if constexpr (G >= 8) v = Op::combine(v, dpp<kRowHalfMirror>(v));
+        if constexpr (G >= 16) v = Op::combine(v, dpp<kRowMirror>(v));
+        if constexpr (G >= 32) v = Op::combine(v, swap16(v));
+        return v;
+    }
 }
 
 // Reduce across a workgroup of NT threads; the result is valid in every

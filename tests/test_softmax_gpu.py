@@ -327,3 +327,27 @@ def test_in_place(hip, orc, shape, same_path, log):
         check_bwd(sep, dy_h, got, ref, log)
         if same_path:
             assert np.array_equal(got.view(np.uint32), want.view(np.uint32)), alias
+
+
+@pytest.mark.parametrize("c", [1, 2, 3, 4, 5, 15, 17, 32, 33, 63, 65, 128, 131, 256, 257, 514, 1000, 1025, 2047, 2050,
+                               4096, 4097, 9001])
+def test_xent_row_widths(hip, orc, c):
+    """Every lanes-per-row form of the loss at the edges of its range, with
+    row counts that leave its last workgroup partly empty and (261 rows of
+    the widest forms) that need the two-level ticket.  dlogits: rounding of
+    exp, sum, quotient and product, within 1e-5 of each row's values."""
+    for b in (1, 5, 261):
+        g = SplitMix64(0x7E57 + 31 * c + b)
+        logits, labels = g.normal((b, c), 0.0, 3.0), g.randint(b, c)
+        dl_, dlab, dloss, ddl = dev(logits), dev(labels), empty((1,)), empty((b, c))
+        engine.train.softmax_xent(dl_, dlab, dloss, ddl, b, c)
+        z = logits.astype(np.float64)
+        z = z - z.max(axis=1, keepdims=True)
+        p = np.exp(z)
+        ls = np.log(p.sum(axis=1))
+        p /= p.sum(axis=1, keepdims=True)
+        rows = np.arange(b)
+        loss = np.mean(ls - z[rows, labels])
+        p[rows, labels] -= 1.0
+        assert abs(dloss.numpy()[0] - loss) <= 1e-5 * max(abs(loss), 1e-3)
+        assert np.all(np.abs(ddl.numpy() - p / b) <= 1e-5 * (np.abs(p) + np.exp(z)) / b + 1e-30)
