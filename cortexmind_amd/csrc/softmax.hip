@@ -13,8 +13,10 @@
 // which s is summed differs.
 //
 // Kernel families by row length:
-//  * wave per row, row in registers (cols <= 4096, cols % 4 == 0): one pass
-//    over HBM, DPP wave reductions, no LDS;
+//  * rows in registers (4 <= cols <= 4096): 4 to 64 lanes per row, one pass
+//    over HBM, DPP reductions, no LDS; ragged rows (cols not a multiple of
+//    4, or bases not 16-byte aligned) run the same kernels with dword-aligned
+//    128-bit accesses;
 //  * long rows (up to 64 segments of 8192, up to 8192 rows): one pass, each
 //    workgroup holds a segment in registers and the workgroups of a row
 //    exchange partials through device memory (see the single-pass section);
@@ -22,7 +24,8 @@
 //    (max m_b, sum_b exp(x - m_b)) [forward] or to its partial dot product
 //    [backward]; pass 2 combines the row's partials in segment order
 //    (S = sum_b s_b * exp(m_b - M)), re-reads its segment and writes;
-//  * any shape or alignment: wave per row, three sweeps over the row.
+//  * what is left (fewer than 4 columns; long ragged rows without scratch):
+//    wave per row, three sweeps over the row.
 // The running max starts from -FLT_MAX, as reduce::max does, so an
 // all -inf row (or segment) never forms (-inf) - (-inf).
 #include <atomic>
@@ -68,27 +71,46 @@ __device__ __forceinline__ float exp_lsm(float y) { return exp2f(y * 1.442695040
 
 // ------------------------------------------------- wave per row, registers
 
-// NV float4 per lane: cols <= 256 * NV.  WPB rows (one per wave) per workgroup.
-template <int NV, bool LOG, int WPB = kWavesPerBlock>
-__global__ __launch_bounds__(WPB * kWave) void k_sm_fwd_wave(const float *__restrict__ x,
-                                                             float *__restrict__ y, size_t rows,
-                                                             size_t cols) {
-    const size_t row = static_cast<size_t>(blockIdx.x) * WPB + threadIdx.x / kWave;
-    if (row >= rows) return;  // whole waves leave together
-    const int lane = threadIdx.x & (kWave - 1);
+// G lanes per row, NV float4 per lane: cols <= 4 G NV; a 128-thread
+// workgroup takes 128 / G rows (measured on [512, 1024] as 3.35 us per launch
+// against 3.5-3.8 us with four or eight waves per workgroup: more workgroups
+// spread the rows over more CUs).  AL: 16-byte aligned rows (G = 64 only);
+// otherwise dword-aligned 128-bit accesses with a masked tail (tail_off).
+// The ragged forms replaced three sweeps of dword loads by a wave per row:
+// [5000, 1003] forward and backward 36.4 -> 20.4 us (20 bytes per element: 4.9 TB/s).  Rows of up to 128 columns share a
+// wave, which a wave each left mostly idle.
+constexpr int kSmThreads = 128;
+template <int G, int NV, bool LOG, bool AL>
+__global__ __launch_bounds__(kSmThreads) void k_sm_fwd_rows(const float *__restrict__ x, float *__restrict__ y,
+                                                            size_t rows, size_t cols) {
+    static_assert(G == kWave || !AL, "narrow rows take the dword-aligned form");
+    const size_t r = static_cast<size_t>(blockIdx.x) * (kSmThreads / G) + threadIdx.x / G;
+    if (G == kWave && r >= rows) return;  // whole waves leave together
+    const size_t row = r < rows ? r : rows - 1;  // lanes past the last row re-read it
+    const int lane = threadIdx.x % G;
     const float *__restrict__ xr = x + row * cols;
     float *__restrict__ yr = y + row * cols;
     const size_t c4 = cols / 4;
+    const float4 ninf = make_float4(-INFINITY, -INFINITY, -INFINITY, -INFINITY);
     float4 v[NV];
+    int off[NV];
 #pragma unroll
     for (int k = 0; k < NV; ++k) {
-        const size_t i = static_cast<size_t>(k) * kWave + lane;
-        v[k] = i < c4 ? ld4_stream(xr + 4 * i) : make_float4(-INFINITY, -INFINITY, -INFINITY, -INFINITY);
+        if constexpr (AL) {
+            const size_t i = static_cast<size_t>(k) * G + lane;
+            v[k] = i < c4 ? ld4_stream(xr + 4 * i) : ninf;
+        } else {
+            off[k] = tail_off(k * G + lane, static_cast<int>(cols));
+            v[k] = ld4_any_stream<false>(xr + off[k]);
+        }
     }
     float m = kLowest;
 #pragma unroll
-    for (int k = 0; k < NV; ++k) m = vmax(vmax(vmax(vmax(m, v[k].x), v[k].y), v[k].z), v[k].w);
-    m = wave_reduce<MaxOp>(m);
+    for (int k = 0; k < NV; ++k) {
+        if constexpr (!AL) v[k] = tail_keep(v[k], k * G + lane, off[k], ninf);
+        m = vmax(vmax(vmax(vmax(m, v[k].x), v[k].y), v[k].z), v[k].w);
+    }
+    m = group_reduce<MaxOp, G>(m);
     float s = 0.0f;
 #pragma unroll
     for (int k = 0; k < NV; ++k) {
@@ -100,65 +122,80 @@ __global__ __launch_bounds__(WPB * kWave) void k_sm_fwd_wave(const float *__rest
             s += (v[k].x + v[k].y) + (v[k].z + v[k].w);
         }
     }
-    s = wave_reduce<SumOp>(s);
-    if constexpr (LOG) {
-        const float ls = logf(s);
+    s = group_reduce<SumOp, G>(s);
+    if (G != kWave && r >= rows) return;
+    const float ls = LOG ? logf(s) : 0.0f;
+    const float inv = LOG ? 0.0f : 1.0f / s;  // e * rn(1/s): one rounding from e / s
 #pragma unroll
-        for (int k = 0; k < NV; ++k) {
-            const size_t i = static_cast<size_t>(k) * kWave + lane;
-            if (i < c4)
-                st4_stream(yr + 4 * i, make_float4(v[k].x - ls, v[k].y - ls, v[k].z - ls, v[k].w - ls));
-        }
-    } else {
-        const float inv = 1.0f / s;  // e * rn(1/s): one rounding from e / s
-#pragma unroll
-        for (int k = 0; k < NV; ++k) {
-            const size_t i = static_cast<size_t>(k) * kWave + lane;
-            if (i < c4) st4_stream(yr + 4 * i, make_float4(v[k].x * inv, v[k].y * inv, v[k].z * inv, v[k].w * inv));
+    for (int k = 0; k < NV; ++k) {
+        float4 o;
+        if constexpr (LOG) o = make_float4(v[k].x - ls, v[k].y - ls, v[k].z - ls, v[k].w - ls);
+        else o = make_float4(v[k].x * inv, v[k].y * inv, v[k].z * inv, v[k].w * inv);
+        if constexpr (AL) {
+            const size_t i = static_cast<size_t>(k) * G + lane;
+            if (i < c4) st4_stream(yr + 4 * i, o);
+        } else {
+            tail_store(yr, o, k * G + lane, off[k]);
         }
     }
 }
 
+// dx of four elements from y, dy and the row's sum r.
+template <bool LOG>
+__device__ __forceinline__ float4 sm_dx4(float4 y, float4 g, float r) {
+    if constexpr (LOG)
+        return make_float4(g.x - exp_lsm(y.x) * r, g.y - exp_lsm(y.y) * r, g.z - exp_lsm(y.z) * r,
+                           g.w - exp_lsm(y.w) * r);
+    return make_float4(y.x * (g.x - r), y.y * (g.y - r), y.z * (g.z - r), y.w * (g.w - r));
+}
+
 // Backward from the saved output: softmax dx = y*(dy - sum(dy*y)),
 // log-softmax dx = dy - exp(y)*sum(dy).
-template <int NV, bool LOG, int WPB = kWavesPerBlock>
-__global__ __launch_bounds__(WPB * kWave) void k_sm_bwd_wave(const float *__restrict__ y,
-                                                             const float *__restrict__ dy,
-                                                             float *__restrict__ dx, size_t rows,
-                                                             size_t cols) {
-    const size_t row = static_cast<size_t>(blockIdx.x) * WPB + threadIdx.x / kWave;
-    if (row >= rows) return;
-    const int lane = threadIdx.x & (kWave - 1);
-    const size_t off = row * cols;
+template <int G, int NV, bool LOG, bool AL>
+__global__ __launch_bounds__(kSmThreads) void k_sm_bwd_rows(const float *__restrict__ y, const float *__restrict__ dy,
+                                                            float *__restrict__ dx, size_t rows, size_t cols) {
+    static_assert(G == kWave || !AL, "narrow rows take the dword-aligned form");
+    const size_t rw = static_cast<size_t>(blockIdx.x) * (kSmThreads / G) + threadIdx.x / G;
+    if (G == kWave && rw >= rows) return;
+    const size_t row = rw < rows ? rw : rows - 1;
+    const int lane = threadIdx.x % G;
+    const size_t base = row * cols;
     const size_t c4 = cols / 4;
     const float4 zero = make_float4(0.f, 0.f, 0.f, 0.f);
     float4 yv[NV], gv[NV];
+    int off[NV];
 #pragma unroll
     for (int k = 0; k < NV; ++k) {
-        const size_t i = static_cast<size_t>(k) * kWave + lane;
-        yv[k] = i < c4 ? ld4_stream(y + off + 4 * i) : zero;
-        gv[k] = i < c4 ? ld4_stream(dy + off + 4 * i) : zero;
+        if constexpr (AL) {
+            const size_t i = static_cast<size_t>(k) * G + lane;
+            yv[k] = i < c4 ? ld4_stream(y + base + 4 * i) : zero;
+            gv[k] = i < c4 ? ld4_stream(dy + base + 4 * i) : zero;
+        } else {
+            off[k] = tail_off(k * G + lane, static_cast<int>(cols));
+            yv[k] = ld4_any_stream<false>(y + base + off[k]);
+            gv[k] = ld4_any_stream<false>(dy + base + off[k]);
+        }
     }
     float r = 0.0f;
 #pragma unroll
     for (int k = 0; k < NV; ++k) {
+        if constexpr (!AL) {
+            yv[k] = tail_keep(yv[k], k * G + lane, off[k], zero);
+            gv[k] = tail_keep(gv[k], k * G + lane, off[k], zero);
+        }
         if constexpr (LOG) r += (gv[k].x + gv[k].y) + (gv[k].z + gv[k].w);
         else r += (gv[k].x * yv[k].x + gv[k].y * yv[k].y) + (gv[k].z * yv[k].z + gv[k].w * yv[k].w);
     }
-    r = wave_reduce<SumOp>(r);
+    r = group_reduce<SumOp, G>(r);
+    if (G != kWave && rw >= rows) return;
 #pragma unroll
     for (int k = 0; k < NV; ++k) {
-        const size_t i = static_cast<size_t>(k) * kWave + lane;
-        if (i >= c4) continue;
-        float4 o;
-        if constexpr (LOG) {
-            o.x = gv[k].x - exp_lsm(yv[k].x) * r; o.y = gv[k].y - exp_lsm(yv[k].y) * r;
-            o.z = gv[k].z - exp_lsm(yv[k].z) * r; o.w = gv[k].w - exp_lsm(yv[k].w) * r;
+        if constexpr (AL) {
+            const size_t i = static_cast<size_t>(k) * G + lane;
+            if (i < c4) st4_stream(dx + base + 4 * i, sm_dx4<LOG>(yv[k], gv[k], r));
         } else {
-            o.x = yv[k].x * (gv[k].x - r); o.y = yv[k].y * (gv[k].y - r);
-            o.z = yv[k].z * (gv[k].z - r); o.w = yv[k].w * (gv[k].w - r);
+            tail_store(dx + base, sm_dx4<LOG>(yv[k], gv[k], r), k * G + lane, off[k]);
         }
-        st4_stream(dx + off + 4 * i, o);
     }
 }
 
@@ -170,6 +207,34 @@ constexpr int kSegNV = 4;
 struct MS {
     float m, s;
 };
+
+// A segment of `left` floats to the row's end, at most `cap` of them: float4
+// number i of it loaded (missing components as `pad`) and stored.  AL: a
+// whole number of aligned float4s.  Otherwise any length and dword alignment;
+// a segment of fewer than 4 floats reaches back into the row's previous
+// segment for its masked load (rows are longer than one segment).
+template <bool AL>
+struct SegRun {
+    int n;
+    __device__ SegRun(size_t left, size_t cap) : n(static_cast<int>(left < cap ? left : cap)) {}
+    template <bool STREAM>
+    __device__ float4 load(const float *p, int i, float4 pad) const {
+        if constexpr (AL) {
+            if (4 * i >= n) return pad;
+            return STREAM ? ld4_stream(p + 4 * i) : ld4(p + 4 * i);
+        }
+        const int off = tail_off(i, n);
+        return tail_keep(STREAM ? ld4_any_stream<false>(p + off) : ld4_any<false>(p + off), i, off, pad);
+    }
+    __device__ void store(float *p, float4 v, int i) const {
+        if constexpr (AL) {
+            if (4 * i < n) st4_stream(p + 4 * i, v);
+        } else {
+            tail_store(p, v, i, tail_off(i, n));
+        }
+    }
+};
+
 // Pass 1 forward: per (row, segment) the segment max m_b and
 // s_b = sum exp(x - m_b).  A segment is NV float4 per thread, streamed in
 // chunks of 4 float4 with the next chunk's loads in flight while the
@@ -177,7 +242,7 @@ struct MS {
 // online rescaling s = s*exp(m - m') + sum exp(x - m') of Milakov and
 // Gimelshein (2018).  Then a block max, one rescale per thread, and a block
 // sum.  grid = rows * segs.
-template <int NV>
+template <int NV, bool AL>
 __global__ __launch_bounds__(kBlock) void k_sm_fwd_part(const float *__restrict__ x, size_t cols,
                                                         unsigned segs, MS *__restrict__ part) {
     constexpr size_t L = kBlock * 4 * NV;
@@ -187,23 +252,17 @@ __global__ __launch_bounds__(kBlock) void k_sm_fwd_part(const float *__restrict_
     const size_t row = blockIdx.x / segs;
     const unsigned seg = blockIdx.x - static_cast<unsigned>(row) * segs;
     const float *__restrict__ xs = x + row * cols + static_cast<size_t>(seg) * L;
-    const size_t n4 = (cols - static_cast<size_t>(seg) * L) / 4;  // float4 left in the row
+    const SegRun<AL> run(cols - static_cast<size_t>(seg) * L, L);
     const float4 ninf = make_float4(-INFINITY, -INFINITY, -INFINITY, -INFINITY);
     float4 cur[C], nxt[C];
 #pragma unroll
-    for (int k = 0; k < C; ++k) {
-        const size_t i = static_cast<size_t>(k) * kBlock + threadIdx.x;
-        cur[k] = i < n4 ? ld4(xs + 4 * i) : ninf;
-    }
+    for (int k = 0; k < C; ++k) cur[k] = run.template load<false>(xs, k * kBlock + threadIdx.x, ninf);
     float m = kLowest, s = 0.0f;
 #pragma unroll
     for (int c = 0; c < NV / C; ++c) {
         if (c + 1 < NV / C) {
 #pragma unroll
-            for (int k = 0; k < C; ++k) {
-                const size_t i = static_cast<size_t>((c + 1) * C + k) * kBlock + threadIdx.x;
-                nxt[k] = i < n4 ? ld4(xs + 4 * i) : ninf;
-            }
+            for (int k = 0; k < C; ++k) nxt[k] = run.template load<false>(xs, ((c + 1) * C + k) * kBlock + threadIdx.x, ninf);
         }
         float mc = m;
 #pragma unroll
@@ -239,7 +298,7 @@ __device__ __forceinline__ MS combine_row(const MS *__restrict__ p, unsigned seg
 // rounding, and saves the per-element division.  Chunks of 4 float4 per
 // thread, the next chunk's loads in flight while the current one is
 // written.
-template <int NV, bool LOG>
+template <int NV, bool LOG, bool AL>
 __global__ __launch_bounds__(kBlock) void k_sm_fwd_apply(const float *__restrict__ x,
                                                          float *__restrict__ y, size_t cols,
                                                          unsigned segs, const MS *__restrict__ part) {
@@ -250,13 +309,11 @@ __global__ __launch_bounds__(kBlock) void k_sm_fwd_apply(const float *__restrict
     const size_t row = blockIdx.x / segs;
     const unsigned seg = blockIdx.x - static_cast<unsigned>(row) * segs;
     const size_t base = row * cols + static_cast<size_t>(seg) * L;
-    const size_t n4 = (cols - static_cast<size_t>(seg) * L) / 4;
+    const SegRun<AL> run(cols - static_cast<size_t>(seg) * L, L);
+    const float4 zero = make_float4(0.f, 0.f, 0.f, 0.f);
     float4 cur[C], nxt[C];
 #pragma unroll
-    for (int k = 0; k < C; ++k) {
-        const size_t i = static_cast<size_t>(k) * kBlock + threadIdx.x;
-        if (i < n4) cur[k] = ld4_stream(x + base + 4 * i);
-    }
+    for (int k = 0; k < C; ++k) cur[k] = run.template load<true>(x + base, k * kBlock + threadIdx.x, zero);
     const MS t = combine_row(part + row * segs, segs, lds);
     const float ls = LOG ? logf(t.s) : 0.0f;
     const float inv = LOG ? 0.0f : 1.0f / t.s;
@@ -264,15 +321,11 @@ __global__ __launch_bounds__(kBlock) void k_sm_fwd_apply(const float *__restrict
     for (int c = 0; c < NV / C; ++c) {
         if (c + 1 < NV / C) {
 #pragma unroll
-            for (int k = 0; k < C; ++k) {
-                const size_t i = static_cast<size_t>((c + 1) * C + k) * kBlock + threadIdx.x;
-                if (i < n4) nxt[k] = ld4_stream(x + base + 4 * i);
-            }
+            for (int k = 0; k < C; ++k)
+                nxt[k] = run.template load<true>(x + base, ((c + 1) * C + k) * kBlock + threadIdx.x, zero);
         }
 #pragma unroll
         for (int k = 0; k < C; ++k) {
-            const size_t i = static_cast<size_t>(c * C + k) * kBlock + threadIdx.x;
-            if (i >= n4) continue;
             float4 z;
             z.x = cur[k].x - t.m; z.y = cur[k].y - t.m; z.z = cur[k].z - t.m; z.w = cur[k].w - t.m;
             float4 o;
@@ -281,7 +334,7 @@ __global__ __launch_bounds__(kBlock) void k_sm_fwd_apply(const float *__restrict
             } else {
                 o = make_float4(expf(z.x) * inv, expf(z.y) * inv, expf(z.z) * inv, expf(z.w) * inv);
             }
-            st4_stream(y + base + 4 * i, o);
+            run.store(y + base, o, (c * C + k) * kBlock + threadIdx.x);
         }
 #pragma unroll
         for (int k = 0; k < C; ++k) cur[k] = nxt[k];
@@ -289,7 +342,7 @@ __global__ __launch_bounds__(kBlock) void k_sm_fwd_apply(const float *__restrict
 }
 
 // Pass 1 backward: per (row, segment) partial of sum(dy*y) or sum(dy).
-template <int NV, bool LOG>
+template <int NV, bool LOG, bool AL>
 __global__ __launch_bounds__(kBlock) void k_sm_bwd_part(const float *__restrict__ y,
                                                         const float *__restrict__ dy, size_t cols,
                                                         unsigned segs, float *__restrict__ part) {
@@ -298,14 +351,13 @@ __global__ __launch_bounds__(kBlock) void k_sm_bwd_part(const float *__restrict_
     const size_t row = blockIdx.x / segs;
     const unsigned seg = blockIdx.x - static_cast<unsigned>(row) * segs;
     const size_t base = row * cols + static_cast<size_t>(seg) * L;
-    const size_t n4 = (cols - static_cast<size_t>(seg) * L) / 4;
+    const SegRun<AL> run(cols - static_cast<size_t>(seg) * L, L);
+    const float4 zero = make_float4(0.f, 0.f, 0.f, 0.f);
     float4 g[NV], yy[NV];
 #pragma unroll
     for (int k = 0; k < NV; ++k) {
-        const size_t i = static_cast<size_t>(k) * kBlock + threadIdx.x;
-        const bool in = i < n4;
-        g[k] = in ? ld4(dy + base + 4 * i) : make_float4(0.f, 0.f, 0.f, 0.f);
-        if constexpr (!LOG) yy[k] = in ? ld4(y + base + 4 * i) : make_float4(0.f, 0.f, 0.f, 0.f);
+        g[k] = run.template load<false>(dy + base, k * kBlock + threadIdx.x, zero);
+        if constexpr (!LOG) yy[k] = run.template load<false>(y + base, k * kBlock + threadIdx.x, zero);
     }
     float r = 0.0f;
 #pragma unroll
@@ -317,7 +369,7 @@ __global__ __launch_bounds__(kBlock) void k_sm_bwd_part(const float *__restrict_
     if (threadIdx.x == 0) part[blockIdx.x] = r;
 }
 
-template <int NV, bool LOG>
+template <int NV, bool LOG, bool AL>
 __global__ __launch_bounds__(kBlock) void k_sm_bwd_apply(const float *__restrict__ y,
                                                          const float *__restrict__ dy,
                                                          float *__restrict__ dx, size_t cols,
@@ -331,30 +383,16 @@ __global__ __launch_bounds__(kBlock) void k_sm_bwd_apply(const float *__restrict
     for (unsigned b = threadIdx.x; b < segs; b += kBlock) r += part[row * segs + b];
     r = block_reduce<SumOp, kBlock>(r, lds);
     const size_t base = row * cols + static_cast<size_t>(seg) * L;
-    const size_t n4 = (cols - static_cast<size_t>(seg) * L) / 4;
+    const SegRun<AL> run(cols - static_cast<size_t>(seg) * L, L);
+    const float4 zero = make_float4(0.f, 0.f, 0.f, 0.f);
     float4 yy[NV], g[NV];
 #pragma unroll
     for (int k = 0; k < NV; ++k) {
-        const size_t i = static_cast<size_t>(k) * kBlock + threadIdx.x;
-        if (i < n4) {
-            yy[k] = ld4_stream(y + base + 4 * i);
-            g[k] = ld4_stream(dy + base + 4 * i);
-        }
+        yy[k] = run.template load<true>(y + base, k * kBlock + threadIdx.x, zero);
+        g[k] = run.template load<true>(dy + base, k * kBlock + threadIdx.x, zero);
     }
 #pragma unroll
-    for (int k = 0; k < NV; ++k) {
-        const size_t i = static_cast<size_t>(k) * kBlock + threadIdx.x;
-        if (i >= n4) continue;
-        float4 o;
-        if constexpr (LOG) {
-            o.x = g[k].x - exp_lsm(yy[k].x) * r; o.y = g[k].y - exp_lsm(yy[k].y) * r;
-            o.z = g[k].z - exp_lsm(yy[k].z) * r; o.w = g[k].w - exp_lsm(yy[k].w) * r;
-        } else {
-            o.x = yy[k].x * (g[k].x - r); o.y = yy[k].y * (g[k].y - r);
-            o.z = yy[k].z * (g[k].z - r); o.w = yy[k].w * (g[k].w - r);
-        }
-        st4_stream(dx + base + 4 * i, o);
-    }
+    for (int k = 0; k < NV; ++k) run.store(dx + base, sm_dx4<LOG>(yy[k], g[k], r), k * kBlock + threadIdx.x);
 }
 
 // ------------------------------------------- single pass, long rows
@@ -462,29 +500,43 @@ __device__ __forceinline__ unsigned long long x_gather(const unsigned long long 
     return __ballot(miss);
 }
 
-// Loading the thread's NV float4 of a segment of n4 >= 1 float4: x_issue
-// issues every load as straight-line code (an index past the end re-reads
-// the segment's last float4), x_pad then overwrites those with `pad`.
+// Loading the thread's NV float4 of a segment of n4 >= 1 float4 (n >= 1
+// floats when !AL): x_issue issues every load as straight-line code (an index
+// past the end re-reads the segment's last float4, or last four floats),
+// x_pad then overwrites what is not the segment's with `pad`.
 // Loads under a per-load branch were compiled with a wait for each pair of
 // loads at the branch's end, which halved the bytes in flight; all of a
 // kernel's x_issue calls come before its first x_pad.
-template <int NV>
-__device__ __forceinline__ unsigned x_last(size_t n4) {
+// `last`: the last float4's number (AL), or the float count (!AL).
+template <int NV, bool AL>
+__device__ __forceinline__ unsigned x_last(size_t left) {
+    if constexpr (!AL) return static_cast<unsigned>(left < kBlock * NV * 4 ? left : kBlock * NV * 4);
+    const size_t n4 = left / 4;
     return static_cast<unsigned>(n4 < kBlock * NV ? n4 : kBlock * NV) - 1u;
 }
-template <int NV>
+template <int NV, bool AL>
 __device__ __forceinline__ void x_issue(float4 (&v)[NV], const float *p, unsigned last) {
 #pragma unroll
     for (int k = 0; k < NV; ++k) {
         const unsigned i = k * kBlock + threadIdx.x;
-        v[k] = ld4_stream_at(p, 16u * (i < last ? i : last));
+        if constexpr (AL) {
+            v[k] = ld4_stream_at(p, 16u * (i < last ? i : last));
+        } else {  // from 4 floats before the segment, so that the 32-bit byte offset is never negative
+            const unsigned o = static_cast<unsigned>(tail_off(i, last) + 4) * 4u;
+            v[k] = ld4_any_stream<false>(reinterpret_cast<const float *>(reinterpret_cast<const char *>(p - 4) + o));
+        }
     }
 }
-template <int NV>
+template <int NV, bool AL>
 __device__ __forceinline__ void x_pad(float4 (&v)[NV], unsigned last, float4 pad) {
 #pragma unroll
     for (int k = 0; k < NV; ++k) {
-        if (k * kBlock + threadIdx.x > last) v[k] = pad;
+        const unsigned i = k * kBlock + threadIdx.x;
+        if constexpr (AL) {
+            if (i > last) v[k] = pad;
+        } else {
+            v[k] = tail_keep(v[k], i, tail_off(i, last), pad);
+        }
     }
 }
 
@@ -500,7 +552,7 @@ __device__ __forceinline__ float dot4(float r, float4 g, float4 y) {
 
 // Forward.  Softmax keeps e = exp(x - m_t) (m_t the thread's max) and writes
 // e * (exp(m_t - M) * (1/S)); log-softmax keeps x and writes (x - M) - log S.
-template <bool LOG>
+template <bool LOG, bool AL>
 __global__ __launch_bounds__(kBlock) void k_sm_fwd_x(const float *__restrict__ x, float *__restrict__ y,
                                                      size_t cols, unsigned segs, unsigned *hdr,
                                                      unsigned long long *slots, unsigned limit,
@@ -518,13 +570,13 @@ __global__ __launch_bounds__(kBlock) void k_sm_fwd_x(const float *__restrict__ x
     unsigned *h = hdr + row * kCtr;
     const unsigned tag = x_epoch(h) + 1;  // every wave: a load behind a branch would be waited for at its end
     const float *__restrict__ xr = x + static_cast<size_t>(row) * cols;
-    const size_t n4 = (cols - static_cast<size_t>(seg) * kXSeg) / 4;
+    const size_t left = cols - static_cast<size_t>(seg) * kXSeg;
     const float4 ninf = make_float4(-INFINITY, -INFINITY, -INFINITY, -INFINITY);
     float4 v[NV];
-    const unsigned last = x_last<NV>(n4);
-    x_issue(v, xr + seg * kXSeg, last);
+    const unsigned last = x_last<NV, AL>(left);
+    x_issue<NV, AL>(v, xr + seg * kXSeg, last);
     __builtin_amdgcn_sched_barrier(0);
-    x_pad(v, last, ninf);
+    x_pad<NV, AL>(v, last, ninf);
     float mt = kLowest;
 #pragma unroll
     for (int k = 0; k < NV; ++k) mt = max4(mt, v[k]);
@@ -557,19 +609,13 @@ __global__ __launch_bounds__(kBlock) void k_sm_fwd_x(const float *__restrict__ x
     for (unsigned long long miss = s_miss; miss; miss &= miss - 1) {
         const unsigned b = static_cast<unsigned>(__builtin_ctzll(miss));
         const float *xb = xr + b * kXSeg;
-        const size_t nb = (cols - static_cast<size_t>(b) * kXSeg) / 4;
+        const SegRun<AL> run(cols - static_cast<size_t>(b) * kXSeg, kXSeg);
         float m = kLowest;
 #pragma unroll 1
-        for (int k = 0; k < NV; ++k) {
-            const size_t i = static_cast<size_t>(k) * kBlock + threadIdx.x;
-            m = max4(m, i < nb ? ld4(xb + 4 * i) : ninf);
-        }
+        for (int k = 0; k < NV; ++k) m = max4(m, run.template load<false>(xb, k * kBlock + threadIdx.x, ninf));
         float s = 0.0f;
 #pragma unroll 1
-        for (int k = 0; k < NV; ++k) {
-            const size_t i = static_cast<size_t>(k) * kBlock + threadIdx.x;
-            s += sum4(exp4(i < nb ? ld4(xb + 4 * i) : ninf, m));
-        }
+        for (int k = 0; k < NV; ++k) s += sum4(exp4(run.template load<false>(xb, k * kBlock + threadIdx.x, ninf), m));
         const float M1 = block_reduce<MaxOp, kBlock>(m, lds);
         const float S1 = block_reduce<SumOp, kBlock>(s * expf(m - M1), lds);
         if (threadIdx.x == 0) {
@@ -583,22 +629,18 @@ __global__ __launch_bounds__(kBlock) void k_sm_fwd_x(const float *__restrict__ x
     const float S =
         block_reduce<SumOp, kBlock>(has ? part[1][threadIdx.x] * expf(part[0][threadIdx.x] - M) : 0.0f, lds);
     float *__restrict__ ys = y + static_cast<size_t>(row) * cols + seg * kXSeg;
+    const SegRun<AL> out(left, kXSeg);
     if constexpr (LOG) {
         const float ls = logf(S);
 #pragma unroll
-        for (int k = 0; k < NV; ++k) {
-            const size_t i = static_cast<size_t>(k) * kBlock + threadIdx.x;
-            if (i < n4)
-                st4_stream(ys + 4 * i, make_float4((v[k].x - M) - ls, (v[k].y - M) - ls, (v[k].z - M) - ls,
-                                                   (v[k].w - M) - ls));
-        }
+        for (int k = 0; k < NV; ++k)
+            out.store(ys, make_float4((v[k].x - M) - ls, (v[k].y - M) - ls, (v[k].z - M) - ls, (v[k].w - M) - ls),
+                      k * kBlock + threadIdx.x);
     } else {
         const float f = expf(mt - M) * (1.0f / S);
 #pragma unroll
-        for (int k = 0; k < NV; ++k) {
-            const size_t i = static_cast<size_t>(k) * kBlock + threadIdx.x;
-            if (i < n4) st4_stream(ys + 4 * i, make_float4(v[k].x * f, v[k].y * f, v[k].z * f, v[k].w * f));
-        }
+        for (int k = 0; k < NV; ++k)
+            out.store(ys, make_float4(v[k].x * f, v[k].y * f, v[k].z * f, v[k].w * f), k * kBlock + threadIdx.x);
     }
     if (threadIdx.x == 0) x_leave(h, ticket, segs, tag);
 #ifdef CXM_TIMELINE
@@ -609,7 +651,7 @@ __global__ __launch_bounds__(kBlock) void k_sm_fwd_x(const float *__restrict__ x
 
 // Backward: partial r_b = sum(dy*y) or sum(dy) per segment, r = sum_b r_b
 // in segment order, then dx as the wave kernel writes it.
-template <bool LOG>
+template <bool LOG, bool AL>
 __global__ __launch_bounds__(kBlock) void k_sm_bwd_x(const float *__restrict__ y, const float *__restrict__ dy,
                                                      float *__restrict__ dx, size_t cols, unsigned segs,
                                                      unsigned *hdr, unsigned long long *slots,
@@ -625,15 +667,15 @@ __global__ __launch_bounds__(kBlock) void k_sm_bwd_x(const float *__restrict__ y
     const unsigned tag = x_epoch(h) + 1;  // every wave: a load behind a branch would be waited for at its end
     const size_t rbase = static_cast<size_t>(row) * cols;
     const size_t base = rbase + seg * kXSeg;
-    const size_t n4 = (cols - static_cast<size_t>(seg) * kXSeg) / 4;
+    const size_t left = cols - static_cast<size_t>(seg) * kXSeg;
     const float4 zero = make_float4(0.f, 0.f, 0.f, 0.f);
     float4 yv[NV], gv[NV];
-    const unsigned last = x_last<NV>(n4);
-    x_issue(yv, y + base, last);
-    x_issue(gv, dy + base, last);
+    const unsigned last = x_last<NV, AL>(left);
+    x_issue<NV, AL>(yv, y + base, last);
+    x_issue<NV, AL>(gv, dy + base, last);
     __builtin_amdgcn_sched_barrier(0);
-    x_pad(yv, last, zero);
-    x_pad(gv, last, zero);
+    x_pad<NV, AL>(yv, last, zero);
+    x_pad<NV, AL>(gv, last, zero);
     float r = 0.0f;
 #pragma unroll
     for (int k = 0; k < NV; ++k) r = LOG ? r + sum4(gv[k]) : dot4(r, gv[k], yv[k]);
@@ -655,35 +697,22 @@ __global__ __launch_bounds__(kBlock) void k_sm_bwd_x(const float *__restrict__ y
     for (unsigned long long miss = s_miss; miss; miss &= miss - 1) {
         const unsigned b = static_cast<unsigned>(__builtin_ctzll(miss));
         const size_t bb = rbase + b * kXSeg;
-        const size_t nb = (cols - static_cast<size_t>(b) * kXSeg) / 4;
+        const SegRun<AL> run(cols - static_cast<size_t>(b) * kXSeg, kXSeg);
         float q = 0.0f;
 #pragma unroll 1
         for (int k = 0; k < NV; ++k) {
-            const size_t i = static_cast<size_t>(k) * kBlock + threadIdx.x;
-            const bool in = i < nb;
-            const float4 g = in ? ld4(dy + bb + 4 * i) : zero;
+            const float4 g = run.template load<false>(dy + bb, k * kBlock + threadIdx.x, zero);
             if constexpr (LOG) q = q + sum4(g);
-            else q = dot4(q, g, in ? ld4(y + bb + 4 * i) : zero);
+            else q = dot4(q, g, run.template load<false>(y + bb, k * kBlock + threadIdx.x, zero));
         }
         const float q1 = block_reduce<SumOp, kBlock>(q, lds);
         if (threadIdx.x == 0) part[0][b] = q1;
     }
     __syncthreads();
     const float R = block_reduce<SumOp, kBlock>(threadIdx.x < segs ? part[0][threadIdx.x] : 0.0f, lds);
+    const SegRun<AL> out(left, kXSeg);
 #pragma unroll
-    for (int k = 0; k < NV; ++k) {
-        const size_t i = static_cast<size_t>(k) * kBlock + threadIdx.x;
-        if (i >= n4) continue;
-        float4 o;
-        if constexpr (LOG) {
-            o.x = gv[k].x - exp_lsm(yv[k].x) * R; o.y = gv[k].y - exp_lsm(yv[k].y) * R;
-            o.z = gv[k].z - exp_lsm(yv[k].z) * R; o.w = gv[k].w - exp_lsm(yv[k].w) * R;
-        } else {
-            o.x = yv[k].x * (gv[k].x - R); o.y = yv[k].y * (gv[k].y - R);
-            o.z = yv[k].z * (gv[k].z - R); o.w = yv[k].w * (gv[k].w - R);
-        }
-        st4_stream(dx + base + 4 * i, o);
-    }
+    for (int k = 0; k < NV; ++k) out.store(dx + base, sm_dx4<LOG>(yv[k], gv[k], R), k * kBlock + threadIdx.x);
     if (threadIdx.x == 0) x_leave(h, ticket, segs, tag);
 #ifdef CXM_TIMELINE
     __syncthreads();
@@ -912,32 +941,43 @@ inline hipStream_t hs(cxm_stream_t s) { return reinterpret_cast<hipStream_t>(s);
 
 constexpr size_t kWaveRowMax = 256 * 16;  // wave-per-row kernel holds up to 4096 columns
 
-// Two rows (waves) per workgroup: measured on [512, 1024] as 3.35 us per
-// launch against 3.5-3.8 us with four or eight rows per workgroup (more
-// workgroups spread the rows over more CUs).
-constexpr int kSmWpb = 2;
-
-template <bool LOG>
-int sm_fwd_wave(const float *x, float *y, size_t rows, size_t cols, hipStream_t s) {
-    const dim3 grid(ceil_div(rows, kSmWpb)), block(kSmWpb * kWave);
-    const size_t nv = (cols + 255) / 256;
-    if (nv <= 1) hipLaunchKernelGGL((k_sm_fwd_wave<1, LOG, kSmWpb>), grid, block, 0, s, x, y, rows, cols);
-    else if (nv <= 2) hipLaunchKernelGGL((k_sm_fwd_wave<2, LOG, kSmWpb>), grid, block, 0, s, x, y, rows, cols);
-    else if (nv <= 4) hipLaunchKernelGGL((k_sm_fwd_wave<4, LOG, kSmWpb>), grid, block, 0, s, x, y, rows, cols);
-    else if (nv <= 8) hipLaunchKernelGGL((k_sm_fwd_wave<8, LOG, kSmWpb>), grid, block, 0, s, x, y, rows, cols);
-    else hipLaunchKernelGGL((k_sm_fwd_wave<16, LOG, kSmWpb>), grid, block, 0, s, x, y, rows, cols);
+// Lanes per row and float4 per lane by the row's float4 count (the last one
+// partial when ragged): rows of at most 32 float4 share a wave.
+template <bool LOG, bool AL>
+int sm_fwd_rows(const float *x, float *y, size_t rows, size_t cols, hipStream_t s) {
+    const size_t v4 = (cols + 3) / 4;
+#define CXM_SM(G, NV, A)                                                                                          \
+    hipLaunchKernelGGL((k_sm_fwd_rows<G, NV, LOG, A>), dim3(ceil_div(rows, kSmThreads / G)), dim3(kSmThreads), 0, s, \
+                       x, y, rows, cols)
+    if (v4 <= 4) CXM_SM(4, 1, false);
+    else if (v4 <= 8) CXM_SM(8, 1, false);
+    else if (v4 <= 16) CXM_SM(16, 1, false);
+    else if (v4 <= 32) CXM_SM(32, 1, false);
+    else if (v4 <= 64) CXM_SM(64, 1, AL);
+    else if (v4 <= 128) CXM_SM(64, 2, AL);
+    else if (v4 <= 256) CXM_SM(64, 4, AL);
+    else if (v4 <= 512) CXM_SM(64, 8, AL);
+    else CXM_SM(64, 16, AL);
+#undef CXM_SM
     return launch_status();
 }
 
-template <bool LOG>
-int sm_bwd_wave(const float *y, const float *dy, float *dx, size_t rows, size_t cols, hipStream_t s) {
-    const dim3 grid(ceil_div(rows, kSmWpb)), block(kSmWpb * kWave);
-    const size_t nv = (cols + 255) / 256;
-    if (nv <= 1) hipLaunchKernelGGL((k_sm_bwd_wave<1, LOG, kSmWpb>), grid, block, 0, s, y, dy, dx, rows, cols);
-    else if (nv <= 2) hipLaunchKernelGGL((k_sm_bwd_wave<2, LOG, kSmWpb>), grid, block, 0, s, y, dy, dx, rows, cols);
-    else if (nv <= 4) hipLaunchKernelGGL((k_sm_bwd_wave<4, LOG, kSmWpb>), grid, block, 0, s, y, dy, dx, rows, cols);
-    else if (nv <= 8) hipLaunchKernelGGL((k_sm_bwd_wave<8, LOG, kSmWpb>), grid, block, 0, s, y, dy, dx, rows, cols);
-    else hipLaunchKernelGGL((k_sm_bwd_wave<16, LOG, kSmWpb>), grid, block, 0, s, y, dy, dx, rows, cols);
+template <bool LOG, bool AL>
+int sm_bwd_rows(const float *y, const float *dy, float *dx, size_t rows, size_t cols, hipStream_t s) {
+    const size_t v4 = (cols + 3) / 4;
+#define CXM_SM(G, NV, A)                                                                                          \
+    hipLaunchKernelGGL((k_sm_bwd_rows<G, NV, LOG, A>), dim3(ceil_div(rows, kSmThreads / G)), dim3(kSmThreads), 0, s, \
+                       y, dy, dx, rows, cols)
+    if (v4 <= 4) CXM_SM(4, 1, false);
+    else if (v4 <= 8) CXM_SM(8, 1, false);
+    else if (v4 <= 16) CXM_SM(16, 1, false);
+    else if (v4 <= 32) CXM_SM(32, 1, false);
+    else if (v4 <= 64) CXM_SM(64, 1, AL);
+    else if (v4 <= 128) CXM_SM(64, 2, AL);
+    else if (v4 <= 256) CXM_SM(64, 4, AL);
+    else if (v4 <= 512) CXM_SM(64, 8, AL);
+    else CXM_SM(64, 16, AL);
+#undef CXM_SM
     return launch_status();
 }
 
@@ -972,6 +1012,7 @@ void x_stagger_for(int pct, size_t rows, unsigned segs, size_t bytes_in, unsigne
     *quanta = static_cast<unsigned>(total / (groups - 1));
 }
 
+template <bool AL>
 int sm_fwd_x(const float *x, float *y, size_t rows, size_t cols, int log_mode, cxm_stream_t st) {
     const unsigned segs = static_cast<unsigned>((cols + kXSeg - 1) / kXSeg);
     Exchange xc;
@@ -982,14 +1023,15 @@ int sm_fwd_x(const float *x, float *y, size_t rows, size_t cols, int log_mode, c
     unsigned g, q;
     x_stagger_for(g_x_stagger_pct.load(std::memory_order_relaxed), rows, segs, rows * cols * sizeof(float), &g, &q);
     if (log_mode)
-        hipLaunchKernelGGL(k_sm_fwd_x<true>, grid, dim3(kBlock), 0, hs(st), x, y, cols, segs, xc.hdr, xc.slots, lim,
+        hipLaunchKernelGGL((k_sm_fwd_x<true, AL>), grid, dim3(kBlock), 0, hs(st), x, y, cols, segs, xc.hdr, xc.slots, lim,
                            g, q);
     else
-        hipLaunchKernelGGL(k_sm_fwd_x<false>, grid, dim3(kBlock), 0, hs(st), x, y, cols, segs, xc.hdr, xc.slots,
+        hipLaunchKernelGGL((k_sm_fwd_x<false, AL>), grid, dim3(kBlock), 0, hs(st), x, y, cols, segs, xc.hdr, xc.slots,
                            lim, g, q);
     return launch_status();
 }
 
+template <bool AL>
 int sm_bwd_x(const float *y, const float *dy, float *dx, size_t rows, size_t cols, int log_mode,
              cxm_stream_t st) {
     const unsigned segs = static_cast<unsigned>((cols + kXSeg - 1) / kXSeg);
@@ -999,15 +1041,15 @@ int sm_bwd_x(const float *y, const float *dy, float *dx, size_t rows, size_t col
     const dim3 grid(segs, static_cast<unsigned>(rows));  // rows <= kXRowsMax
     const unsigned lim = exchange_wait_limit();
     if (log_mode)
-        hipLaunchKernelGGL(k_sm_bwd_x<true>, grid, dim3(kBlock), 0, hs(st), y, dy, dx, cols, segs, xc.hdr, xc.slots,
+        hipLaunchKernelGGL((k_sm_bwd_x<true, AL>), grid, dim3(kBlock), 0, hs(st), y, dy, dx, cols, segs, xc.hdr, xc.slots,
                            lim);
     else
-        hipLaunchKernelGGL(k_sm_bwd_x<false>, grid, dim3(kBlock), 0, hs(st), y, dy, dx, cols, segs, xc.hdr,
+        hipLaunchKernelGGL((k_sm_bwd_x<false, AL>), grid, dim3(kBlock), 0, hs(st), y, dy, dx, cols, segs, xc.hdr,
                            xc.slots, lim);
     return launch_status();
 }
 
-template <int NV>
+template <int NV, bool AL>
 int sm_fwd_split(const float *x, float *y, size_t rows, size_t cols, int log_mode, cxm_stream_t st) {
     constexpr size_t L = kBlock * 4 * NV;
     const size_t segs = (cols + L - 1) / L;
@@ -1018,18 +1060,18 @@ int sm_fwd_split(const float *x, float *y, size_t rows, size_t cols, int log_mod
     MS *part = static_cast<MS *>(ws.scratch);
     const dim3 grid(static_cast<unsigned>(rows * segs));
     hipStream_t s = hs(st);
-    hipLaunchKernelGGL(k_sm_fwd_part<NV>, grid, dim3(kBlock), 0, s, x, cols, static_cast<unsigned>(segs), part);
+    hipLaunchKernelGGL((k_sm_fwd_part<NV, AL>), grid, dim3(kBlock), 0, s, x, cols, static_cast<unsigned>(segs), part);
     if ((rc = launch_status())) return rc;
     if (log_mode)
-        hipLaunchKernelGGL((k_sm_fwd_apply<NV, true>), grid, dim3(kBlock), 0, s, x, y, cols,
+        hipLaunchKernelGGL((k_sm_fwd_apply<NV, true, AL>), grid, dim3(kBlock), 0, s, x, y, cols,
                            static_cast<unsigned>(segs), part);
     else
-        hipLaunchKernelGGL((k_sm_fwd_apply<NV, false>), grid, dim3(kBlock), 0, s, x, y, cols,
+        hipLaunchKernelGGL((k_sm_fwd_apply<NV, false, AL>), grid, dim3(kBlock), 0, s, x, y, cols,
                            static_cast<unsigned>(segs), part);
     return launch_status();
 }
 
-template <int NV>
+template <int NV, bool AL>
 int sm_bwd_split(const float *y, const float *dy, float *dx, size_t rows, size_t cols, int log_mode,
                  cxm_stream_t st) {
     constexpr size_t L = kBlock * 4 * NV;
@@ -1043,13 +1085,13 @@ int sm_bwd_split(const float *y, const float *dy, float *dx, size_t rows, size_t
     hipStream_t s = hs(st);
     const unsigned sg = static_cast<unsigned>(segs);
     if (log_mode) {
-        hipLaunchKernelGGL((k_sm_bwd_part<NV, true>), grid, dim3(kBlock), 0, s, y, dy, cols, sg, part);
+        hipLaunchKernelGGL((k_sm_bwd_part<NV, true, AL>), grid, dim3(kBlock), 0, s, y, dy, cols, sg, part);
         if ((rc = launch_status())) return rc;
-        hipLaunchKernelGGL((k_sm_bwd_apply<NV, true>), grid, dim3(kBlock), 0, s, y, dy, dx, cols, sg, part);
+        hipLaunchKernelGGL((k_sm_bwd_apply<NV, true, AL>), grid, dim3(kBlock), 0, s, y, dy, dx, cols, sg, part);
     } else {
-        hipLaunchKernelGGL((k_sm_bwd_part<NV, false>), grid, dim3(kBlock), 0, s, y, dy, cols, sg, part);
+        hipLaunchKernelGGL((k_sm_bwd_part<NV, false, AL>), grid, dim3(kBlock), 0, s, y, dy, cols, sg, part);
         if ((rc = launch_status())) return rc;
-        hipLaunchKernelGGL((k_sm_bwd_apply<NV, false>), grid, dim3(kBlock), 0, s, y, dy, dx, cols, sg, part);
+        hipLaunchKernelGGL((k_sm_bwd_apply<NV, false, AL>), grid, dim3(kBlock), 0, s, y, dy, dx, cols, sg, part);
     }
     return launch_status();
 }
@@ -1076,16 +1118,24 @@ int softmax_fwd(const float *x, float *y, size_t rows, size_t cols, int log_mode
     if (bad_alias(y, x, bytes)) return CXM_E_INVALID;
     hipStream_t s = hs(st);
     const bool vec = cols % 4 == 0 && aligned16(x) && aligned16(y);
-    if (!vec) {
-        const dim3 grid(ceil_div(rows, kWavesPerBlock));
-        if (log_mode) hipLaunchKernelGGL(k_sm_fwd_any<true>, grid, dim3(kBlock), 0, s, x, y, rows, cols);
-        else hipLaunchKernelGGL(k_sm_fwd_any<false>, grid, dim3(kBlock), 0, s, x, y, rows, cols);
-        return launch_status();
+    if (cols >= 4 && !use_split(cols)) {
+        if (vec) return log_mode ? sm_fwd_rows<true, true>(x, y, rows, cols, s) : sm_fwd_rows<false, true>(x, y, rows, cols, s);
+        return log_mode ? sm_fwd_rows<true, false>(x, y, rows, cols, s) : sm_fwd_rows<false, false>(x, y, rows, cols, s);
     }
-    if (!use_split(cols))
-        return log_mode ? sm_fwd_wave<true>(x, y, rows, cols, s) : sm_fwd_wave<false>(x, y, rows, cols, s);
-    if (use_x(rows, cols) && x != y) return sm_fwd_x(x, y, rows, cols, log_mode, st);
-    return sm_fwd_split<kSegNV>(x, y, rows, cols, log_mode, st);
+    if (vec) {
+        if (use_x(rows, cols) && x != y) return sm_fwd_x<true>(x, y, rows, cols, log_mode, st);
+        return sm_fwd_split<kSegNV, true>(x, y, rows, cols, log_mode, st);
+    }
+    if (cols >= 4) {
+        const int rc = use_x(rows, cols) && x != y ? sm_fwd_x<false>(x, y, rows, cols, log_mode, st)
+                                                   : sm_fwd_split<kSegNV, false>(x, y, rows, cols, log_mode, st);
+        if (rc == CXM_OK) return rc;
+        (void)hipGetLastError();  // no scratch to be had (a capturing stream's first call): the form without
+    }
+    const dim3 grid(ceil_div(rows, kWavesPerBlock));
+    if (log_mode) hipLaunchKernelGGL(k_sm_fwd_any<true>, grid, dim3(kBlock), 0, s, x, y, rows, cols);
+    else hipLaunchKernelGGL(k_sm_fwd_any<false>, grid, dim3(kBlock), 0, s, x, y, rows, cols);
+    return launch_status();
 }
 
 int softmax_bwd(const float *y, const float *dy, float *dx, size_t rows, size_t cols, int log_mode,
@@ -1097,17 +1147,28 @@ int softmax_bwd(const float *y, const float *dy, float *dx, size_t rows, size_t 
     if (bad_alias(dx, y, bytes) || bad_alias(dx, dy, bytes)) return CXM_E_INVALID;
     hipStream_t s = hs(st);
     const bool vec = cols % 4 == 0 && aligned16(y) && aligned16(dy) && aligned16(dx);
-    if (!vec) {
-        const dim3 grid(ceil_div(rows, kWavesPerBlock));
-        if (log_mode) hipLaunchKernelGGL(k_sm_bwd_any<true>, grid, dim3(kBlock), 0, s, y, dy, dx, rows, cols);
-        else hipLaunchKernelGGL(k_sm_bwd_any<false>, grid, dim3(kBlock), 0, s, y, dy, dx, rows, cols);
-        return launch_status();
+    if (cols >= 4 && !use_split(cols)) {
+        if (vec)
+            return log_mode ? sm_bwd_rows<true, true>(y, dy, dx, rows, cols, s)
+                            : sm_bwd_rows<false, true>(y, dy, dx, rows, cols, s);
+        return log_mode ? sm_bwd_rows<true, false>(y, dy, dx, rows, cols, s)
+                        : sm_bwd_rows<false, false>(y, dy, dx, rows, cols, s);
     }
-    if (!use_split(cols))
-        return log_mode ? sm_bwd_wave<true>(y, dy, dx, rows, cols, s)
-                        : sm_bwd_wave<false>(y, dy, dx, rows, cols, s);
-    if (use_x(rows, cols) && dx != y && dx != dy) return sm_bwd_x(y, dy, dx, rows, cols, log_mode, st);
-    return sm_bwd_split<kSegNV>(y, dy, dx, rows, cols, log_mode, st);
+    const bool apart = dx != y && dx != dy;
+    if (vec) {
+        if (use_x(rows, cols) && apart) return sm_bwd_x<true>(y, dy, dx, rows, cols, log_mode, st);
+        return sm_bwd_split<kSegNV, true>(y, dy, dx, rows, cols, log_mode, st);
+    }
+    if (cols >= 4) {
+        const int rc = use_x(rows, cols) && apart ? sm_bwd_x<false>(y, dy, dx, rows, cols, log_mode, st)
+                                                  : sm_bwd_split<kSegNV, false>(y, dy, dx, rows, cols, log_mode, st);
+        if (rc == CXM_OK) return rc;
+        (void)hipGetLastError();  // as in the forward
+    }
+    const dim3 grid(ceil_div(rows, kWavesPerBlock));
+    if (log_mode) hipLaunchKernelGGL(k_sm_bwd_any<true>, grid, dim3(kBlock), 0, s, y, dy, dx, rows, cols);
+    else hipLaunchKernelGGL(k_sm_bwd_any<false>, grid, dim3(kBlock), 0, s, y, dy, dx, rows, cols);
+    return launch_status();
 }
 
 }  // namespace

@@ -351,3 +351,62 @@ def test_xent_row_widths(hip, orc, c):
         p[rows, labels] -= 1.0
         assert abs(dloss.numpy()[0] - loss) <= 1e-5 * max(abs(loss), 1e-3)
         assert np.all(np.abs(ddl.numpy() - p / b) <= 1e-5 * (np.abs(p) + np.exp(z)) / b + 1e-30)
+
+
+RAGGED = [4, 5, 7, 8, 15, 17, 31, 33, 61, 64, 67, 125, 130, 255, 257, 511, 1003, 1026, 2049, 4093, 4097, 8191, 8193, 8194,
+          16387, 40001, 524289]
+
+
+@pytest.mark.parametrize("cols", RAGGED)
+@pytest.mark.parametrize("off", [0, 1])
+def test_ragged_and_narrow_rows(hip, cols, off):
+    """Rows whose length is a multiple of nothing, or whose base is only
+    4-byte aligned: the dword-aligned forms at the edges of their ranges
+    (lanes per row, float4 per lane, segments of the long rows with a last
+    segment of 1 to 3 floats, the two-pass form beyond 524288 columns),
+    against float64, in buffers whose floats before and after the result
+    must stay as they were."""
+    if cols % 4 == 0 and cols > 128 and off == 0:
+        pytest.skip("the aligned form")
+    rows = 3 if cols > 4096 else 131
+    g = SplitMix64(0x4A66 + cols)
+    x, dyv = g.normal((rows, cols), 0.0, 4.0), g.normal((rows, cols))
+    x[0, cols // 2] = -np.inf
+    n = rows * cols
+
+    def guarded():
+        v = dev(np.full(n + 8 + off, 7.0, np.float32), 4 + off)
+        v.shape, v.size = (rows, cols), n
+        return v
+
+    def check_guard(v):
+        full = v.base.numpy()
+        s = (v.ptr - v.base.ptr) // 4
+        assert np.all(full[:s][4 + off:] == 7.0) and np.all(full[s + n:] == 7.0)
+        return full[s:s + n].reshape(rows, cols)
+
+    for log in (False, True):
+        y = guarded()
+        engine.softmax.forward(dev(x, off), y, rows, cols, log=log)
+        got = check_guard(y)
+        check_fwd(x, got, f64_fwd(x, log).astype(np.float32), log)
+        yb = np.where(np.isfinite(got), got, np.float32(-1e30))
+        dx = guarded()
+        engine.softmax.backward(dev(yb, off), dev(dyv, off), dx, rows, cols, log=log)
+        check_bwd(yb, dyv, check_guard(dx), f64_bwd(yb, dyv, log), log)
+
+
+@pytest.mark.parametrize("cols", [8194, 40001])
+def test_ragged_single_pass_recompute_is_bit_identical(hip, cols):
+    """As test_single_pass_recompute_is_bit_identical for ragged rows."""
+    x, dyv = SplitMix64(cols).normal((5, cols), 0.0, 8.0), SplitMix64(cols + 1).normal((5, cols))
+    outs = []
+    for polls in (1 << 16, 0):
+        old = _wait_limit(polls)
+        try:
+            ys = [fwd(x, False), fwd(x, True)]
+            outs.append(ys + [bwd(ys[0], dyv, False), bwd(ys[1], dyv, True)])
+        finally:
+            _wait_limit(old)
+    for a, b in zip(*outs):
+        assert np.array_equal(a.view(np.uint32), b.view(np.uint32))
