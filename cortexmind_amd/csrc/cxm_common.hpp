@@ -546,13 +546,15 @@ __device__ __forceinline__ Pow2 ld_dev(const Pow2 *p) {
             __builtin_bit_cast(double, __hip_atomic_load(u + 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT))};
 }
 
+constexpr unsigned kPartGroup = 16;
+
 // Combines n partials p[0], p[stride], ..., p[(n-1)*stride] into `a` in
 // index order.  The device-coherent loads go out 16 at a time so their
 // latencies overlap (one at a time, a 64-partial combine costs ~30 us).
 template <class Op>
 __device__ __forceinline__ typename Op::T combine_partials(const typename Op::T *p, unsigned n,
                                                            size_t stride, typename Op::T a) {
-    constexpr unsigned G = 16;
+    constexpr unsigned G = kPartGroup;
     for (unsigned c0 = 0; c0 < n; c0 += G) {
         typename Op::T v[G];
 #pragma unroll

@@ -19,6 +19,9 @@
 //    slice and a chunk of the reduced rows; each thread keeps one float4 of
 //    columns, the four waves take interleaved rows and meet in LDS.  Chunks
 //    are combined in chunk order by the last workgroup of the column tile.
+//    Narrow slices (see kFlatInner) are read flat instead (k_cols_flat): every
+//    thread's float4s lie a whole number of rows apart, so it keeps four
+//    columns whatever the row length.
 #include <atomic>
 #include <mutex>
 #include <type_traits>
@@ -542,6 +545,47 @@ __global__ __launch_bounds__(kBlock) void k_rows(const float *__restrict__ x, si
     }
 }
 
+// Short rows, 4 <= dim <= 4 G NV: G lanes per row (several rows per wave up to
+// 128 floats), NV float4 per lane at dword alignment, all in flight together;
+// no LDS, no barrier.  The last loads are clamped to the row's last four
+// floats (tail_off): the floats they repeat change nothing for max, min and
+// the arg forms; for the sums they are replaced by what adds nothing.
+// A workgroup per row kept one row's few loads in flight per CU slot and
+// spent its time in the block reduction: sum over [32450, 384] 19.4 -> 9.3 us,
+// [262144, 8] 128 -> 3.9 us, [5000, 1003] 6.0 -> 4.7 us.
+template <class Op, int G, int NV>
+__global__ __launch_bounds__(kBlock) void k_rows_short(const float *__restrict__ x, size_t rows, int dim,
+                                                       OutDesc out) {
+    using T = typename Op::T;
+    constexpr bool kRepeats = std::is_same_v<T, ArgPair> || std::is_base_of_v<MaxOp, Op> || std::is_base_of_v<MinOp, Op>;
+    const size_t r = static_cast<size_t>(blockIdx.x) * (kBlock / G) + threadIdx.x / G;
+    if (G == kWave && r >= rows) return;  // whole waves leave together
+    const size_t row = r < rows ? r : rows - 1;  // lanes past the last row re-read it
+    const int lane = threadIdx.x % G;
+    const float *__restrict__ xr = x + row * dim;
+    float4 v[NV];
+    int off[NV];
+#pragma unroll
+    for (int k = 0; k < NV; ++k) {
+        off[k] = tail_off(k * G + lane, dim);
+        v[k] = ld4_any_stream<false>(xr + off[k]);
+    }
+    float k0 = 0.0f;
+    if constexpr (Op::kShift) k0 = xr[0];
+    const float4 k4 = make_float4(k0, k0, k0, k0);
+    __builtin_amdgcn_sched_barrier(0);
+    T acc[4] = {Op::identity(), Op::identity(), Op::identity(), Op::identity()};
+#pragma unroll
+    for (int k = 0; k < NV; ++k) {
+        if constexpr (!kRepeats) v[k] = tail_keep(v[k], k * G + lane, off[k], k4);
+        fold4<Op>(acc, v[k], off[k], 1, k4);
+    }
+    if (lane == 0) first_nan_fix<Op>(acc[0], v[0].x);
+    T a = Op::combine(Op::combine(acc[0], acc[1]), Op::combine(acc[2], acc[3]));
+    a = group_reduce<Op, G>(a);
+    if (lane == 0 && r < rows) write_out<Op>(out, row, a);
+}
+
 // Rows whose base is not 4-byte aligned: element by element, one
 // workgroup per row.
 template <class Op>
@@ -567,21 +611,24 @@ __global__ __launch_bounds__(kBlock) void k_rows_bytes(const float *__restrict__
 
 constexpr int kColTile = 256;  // columns per workgroup
 
-// NW waves per workgroup.  Vector path: a wave covers the 256 columns with
-// one float4 per lane and wave w takes rows r0+w, r0+w+NW, ...; scalar
-// path: thread t owns column t%256 and rows r0+t/256, step NW/4.  The
-// per-slot results meet in LDS and threads 0..255 combine them in slot
-// order.  Workgroup b -> (chunk, tile, outer slice), chunk fastest: the
-// chunks of one tile are adjacent in launch order, so its combine runs
-// while later tiles still stream.
-template <class Op, bool VEC, int UNR, int NW, bool FAST = false>
+// NW waves per workgroup.  A wave covers the 256 columns with one float4 per
+// lane and wave w takes rows r0+w, r0+w+NW, ...  AL: 16-byte aligned rows
+// (inner a multiple of 4).  Otherwise (inner >= 4) dword-aligned loads; the
+// last lanes of a slice's last tile read its last four columns and keep the
+// ones that are theirs.  The per-wave results meet in LDS and threads 0..255
+// combine them in wave order.  Workgroup b -> (chunk, tile, outer slice),
+// chunk fastest: the chunks of one tile are adjacent in launch order, so its
+// combine runs while later tiles still stream.  Rows past the last whole
+// batch of UNR go out as one batch too, its loads clamped to the chunk's last
+// row and only its own rows folded (one at a time, each waited a memory
+// round trip for the last).
+template <class Op, bool AL, int UNR, int NW, bool FAST = false>
 __global__ __launch_bounds__(NW * kWave) void k_cols(const float *__restrict__ x, size_t dim,
-                                                     size_t inner, unsigned ntiles, unsigned chunks,
+                                                     size_t inner, unsigned ntiles, unsigned width, unsigned chunks,
                                                      size_t rows_per_chunk, typename Op::T *__restrict__ part,
                                                      unsigned *__restrict__ counters, OutDesc out) {
     using T = typename Op::T;
-    constexpr int NSLOT = VEC ? NW : NW / 4;
-    __shared__ T lds[NSLOT][kColTile];
+    __shared__ T lds[NW][kColTile];
     __shared__ int flag;
 
     // FAST launches a (chunks, tiles, outer) grid: no index arithmetic ahead
@@ -608,84 +655,100 @@ __global__ __launch_bounds__(NW * kWave) void k_cols(const float *__restrict__ x
     const size_t r0 = chunk * rows_per_chunk;
     const size_t r1 = r0 + rows_per_chunk < dim ? r0 + rows_per_chunk : dim;
 
-    if constexpr (VEC) {
-        const int lane = tid & (kWave - 1);
-        const int w = tid / kWave;
-        const size_t col = static_cast<size_t>(tile) * kColTile + lane * 4;
-        T acc[4] = {Op::identity(), Op::identity(), Op::identity(), Op::identity()};
-        // FAST (whole tiles, a chunk under 2^31 bytes): no column bound to
-        // branch on, so every operand is at hand from the start -- behind
-        // the branch the compiler fetched the input pointer in a second
-        // round of kernel-argument loads after the index arithmetic, a
-        // scalar-cache miss in every workgroup (one per CU here)
-        if (FAST || col < inner) {
-            const float *__restrict__ xc = xo + col;
-            float4 k4 = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
-            if constexpr (Op::kShift) k4 = ld4(xc);
-            if constexpr (FAST) {
-                // the chunk as a uniform base and 32-bit byte offsets: one
-                // address register per load instead of two
-                const float *__restrict__ cb = xo + r0 * inner + static_cast<size_t>(tile) * kColTile;
-                const unsigned rowb = static_cast<unsigned>(inner * sizeof(float)), nr = static_cast<unsigned>(r1 - r0);
-                const unsigned c16 = static_cast<unsigned>(lane * 16);
-                // row offsets as a per-lane column offset plus uniform row
-                // offsets (the wave index made uniform, so the products are
-                // scalar): a multiply per load had put 16 quarter-rate vector
-                // multiplies between the index arithmetic and the first load
-                const unsigned wu = __builtin_amdgcn_readfirstlane(static_cast<unsigned>(w));
-                const unsigned step = NW * rowb;
-                unsigned r = wu, ro = wu * rowb + c16;
-                for (; r + (UNR - 1) * NW < nr; r += UNR * NW, ro += UNR * step) {
-                    float4 v[UNR];
+    const int lane = tid & (kWave - 1);
+    const int w = tid / kWave;
+    const unsigned tw = FAST ? static_cast<unsigned>(kColTile) : width;  // columns per tile
+    const size_t col = static_cast<size_t>(tile) * tw + lane * 4;
+    const bool in = FAST || (lane * 4u < tw && col < inner);
+    // !AL: columns [pos, pos + 4) are read, of which the first d are another lane's
+    const size_t pos = AL || col + 4 <= inner ? col : inner - 4;
+    const int d = in ? static_cast<int>(col - pos) : 4;
+    T acc[4] = {Op::identity(), Op::identity(), Op::identity(), Op::identity()};
+    // FAST and AL (whole tiles, a chunk under 2^31 bytes): no column bound to
+    // branch on, so every operand is at hand from the start -- behind
+    // the branch the compiler fetched the input pointer in a second
+    // round of kernel-argument loads after the index arithmetic, a
+    // scalar-cache miss in every workgroup (one per CU here)
+    if (in) {
+        const float *__restrict__ xc = xo + pos;
+        float4 k4 = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+        if constexpr (Op::kShift) k4 = ld4_any<AL>(xc);
+        if constexpr (FAST) {
+            // the chunk as a uniform base and 32-bit byte offsets: one
+            // address register per load instead of two
+            const float *__restrict__ cb = xo + r0 * inner + static_cast<size_t>(tile) * kColTile;
+            const unsigned rowb = static_cast<unsigned>(inner * sizeof(float)), nr = static_cast<unsigned>(r1 - r0);
+            const unsigned c16 = static_cast<unsigned>(lane * 16);
+            // row offsets as a per-lane column offset plus uniform row
+            // offsets (the wave index made uniform, so the products are
+            // scalar): a multiply per load had put 16 quarter-rate vector
+            // multiplies between the index arithmetic and the first load
+            const unsigned wu = __builtin_amdgcn_readfirstlane(static_cast<unsigned>(w));
+            const unsigned step = NW * rowb;
+            unsigned r = wu, ro = wu * rowb + c16;
+            for (; r + (UNR - 1) * NW < nr; r += UNR * NW, ro += UNR * step) {
+                float4 v[UNR];
 #pragma unroll
-                    for (int u = 0; u < UNR; ++u) v[u] = ld4_stream_at(cb, ro + u * step);
-                    // all UNR loads leave before any is folded: left alone, the
-                    // scheduler interleaved the folds to stay at 64 registers
-                    // and kept 5-6 loads in flight (one 16-wave workgroup per
-                    // CU leaves room for 128); streaming 12.1 -> 11.8 us at C2
-                    __builtin_amdgcn_sched_barrier(0);
+                for (int u = 0; u < UNR; ++u) v[u] = ld4_stream_at(cb, ro + u * step);
+                // all UNR loads leave before any is folded: left alone, the
+                // scheduler interleaved the folds to stay at 64 registers
+                // and kept 5-6 loads in flight (one 16-wave workgroup per
+                // CU leaves room for 128); streaming 12.1 -> 11.8 us at C2
+                __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-                    for (int u = 0; u < UNR; ++u) fold4<Op>(acc, v[u], static_cast<int>(r0 + r + u * NW), 0, k4);
-                }
-                for (; r < nr; r += NW, ro += step) fold4<Op>(acc, ld4_stream_at(cb, ro), static_cast<int>(r0 + r), 0, k4);
-            } else {
-                size_t r = r0 + w;
-                for (; r + (UNR - 1) * NW < r1; r += UNR * NW) {
-                    float4 v[UNR];
-#pragma unroll
-                    for (int u = 0; u < UNR; ++u) v[u] = ld4_stream(xc + (r + u * NW) * inner);
-#pragma unroll
-                    for (int u = 0; u < UNR; ++u) fold4<Op>(acc, v[u], static_cast<int>(r + u * NW), 0, k4);
-                }
-                for (; r < r1; r += NW) fold4<Op>(acc, ld4_stream(xc + r * inner), static_cast<int>(r), 0, k4);
+                for (int u = 0; u < UNR; ++u) fold4<Op>(acc, v[u], static_cast<int>(r0 + r + u * NW), 0, k4);
             }
-            if constexpr (std::is_same_v<T, ArgPair>) {
-                if (r0 == 0 && w == 0) {  // row 0 of these four columns
-                    const float4 x0 = ld4(xc);
-                    first_nan_fix<Op>(acc[0], x0.x);
-                    first_nan_fix<Op>(acc[1], x0.y);
-                    first_nan_fix<Op>(acc[2], x0.z);
-                    first_nan_fix<Op>(acc[3], x0.w);
-                }
+            if (r < nr) {
+                float4 v[UNR];
+                const unsigned lo = (nr - 1) * rowb + c16;
+#pragma unroll
+                for (int u = 0; u < UNR; ++u) v[u] = ld4_stream_at(cb, r + u * NW < nr ? ro + u * step : lo);
+                __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+                for (int u = 0; u < UNR; ++u)
+                    if (r + u * NW < nr) fold4<Op>(acc, v[u], static_cast<int>(r0 + r + u * NW), 0, k4);
+            }
+        } else {
+            // rows from the wave's first one, made uniform: scalar products
+            size_t r = r0 + __builtin_amdgcn_readfirstlane(static_cast<unsigned>(w));
+            const size_t step = NW * inner;
+            for (; r + (UNR - 1) * NW < r1; r += UNR * NW) {
+                float4 v[UNR];
+                const size_t ro = r * inner;
+#pragma unroll
+                for (int u = 0; u < UNR; ++u) v[u] = ld4_any_stream<AL>(xc + (ro + u * step));
+                __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+                for (int u = 0; u < UNR; ++u) fold4<Op>(acc, v[u], static_cast<int>(r + u * NW), 0, k4);
+            }
+            if (r < r1) {
+                float4 v[UNR];
+                const size_t ro = r * inner, lo = (r1 - 1) * inner;
+#pragma unroll
+                for (int u = 0; u < UNR; ++u) v[u] = ld4_any_stream<AL>(xc + (r + u * NW < r1 ? ro + u * step : lo));
+                __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+                for (int u = 0; u < UNR; ++u)
+                    if (r + u * NW < r1) fold4<Op>(acc, v[u], static_cast<int>(r + u * NW), 0, k4);
             }
         }
+        if constexpr (std::is_same_v<T, ArgPair>) {
+            if (r0 == 0 && w == 0) {  // row 0 of these four columns
+                const float4 x0 = ld4_any<AL>(xc);
+                first_nan_fix<Op>(acc[0], x0.x);
+                first_nan_fix<Op>(acc[1], x0.y);
+                first_nan_fix<Op>(acc[2], x0.z);
+                first_nan_fix<Op>(acc[3], x0.w);
+            }
+        }
+    }
+    if constexpr (AL) {
 #pragma unroll
         for (int c = 0; c < 4; ++c) lds[w][lane * 4 + c] = acc[c];
     } else {
-        const int c = tid % kColTile, ph = tid / kColTile;
-        const size_t col = static_cast<size_t>(tile) * kColTile + c;
-        T mine = Op::identity();
-        if (col < inner) {
-            float k = 0.0f;
-            if constexpr (Op::kShift) k = xo[col];
-            for (size_t r = r0 + ph; r < r1; r += NSLOT) {
-                float v = xo[r * inner + col];
-                if constexpr (Op::kShift) v = v - k;
-                mine = Op::accum(mine, v, static_cast<int>(r));
-            }
-            if (r0 == 0 && ph == 0) first_nan_fix<Op>(mine, xo[col]);
-        }
-        lds[ph][c] = mine;
+#pragma unroll
+        for (int c = 0; c < 4; ++c)
+            if (c >= d) lds[w][lane * 4 + c - d] = acc[c];
     }
     __syncthreads();
     tl_mark(kTlColsArg, 1);
@@ -694,21 +757,41 @@ __global__ __launch_bounds__(NW * kWave) void k_cols(const float *__restrict__ x
     if (owner) {
         mine = lds[0][tid];
 #pragma unroll
-        for (int k = 1; k < NSLOT; ++k) mine = Op::combine(mine, lds[k][tid]);
+        for (int k = 1; k < NW; ++k) mine = Op::combine(mine, lds[k][tid]);
     }
-    const size_t col = static_cast<size_t>(tile) * kColTile + tid;
+    const size_t oc = static_cast<size_t>(tile) * tw + tid;
+    const bool put = owner && (FAST || (tid < static_cast<int>(tw) && oc < inner));
     if (chunks == 1) {
-        if (owner && (FAST || col < inner)) write_out<Op>(out, o * inner + col, mine);
+        if (put) write_out<Op>(out, o * inner + oc, mine);
         return;
     }
     const size_t slot = (o * ntiles + tile) * chunks;
     if (owner) st_dev(&part[(slot + chunk) * kColTile + tid], mine);
-    const bool last = last_block_ticket(ctr(counters, o * ntiles + tile), chunks, &flag);
-    tl_mark(kTlColsArg, 2);
-    if (!last) return;
-    if (owner) {
-        const T a = combine_partials<Op>(part + slot * kColTile + tid, chunks, kColTile, Op::identity());
-        if (FAST || col < inner) write_out<Op>(out, o * inner + col, a);
+    const size_t t = o * ntiles + tile;
+    if (chunks <= kTicketGroups) {
+        const bool last = last_block_ticket(ctr(counters, t), chunks, &flag);
+        tl_mark(kTlColsArg, 2);
+        if (!last) return;
+        if (put) {
+            const T a = combine_partials<Op>(part + slot * kColTile + tid, chunks, kColTile, Op::identity());
+            write_out<Op>(out, o * inner + oc, a);
+        }
+    } else {
+        // Two levels: the last workgroup of each group of kPartGroup chunks
+        // combines its group's partials, the last group's the groups'.  One
+        // workgroup reading all of 256 chunks (256 KiB through one CU) took
+        // 7 us longer than of 128; this takes a second ticket.
+        const unsigned groups = (chunks + kPartGroup - 1) / kPartGroup, g = chunk / kPartGroup;
+        const unsigned size = (g + 1) * kPartGroup <= chunks ? kPartGroup : chunks - g * kPartGroup;
+        unsigned *cg = ctr(counters, t * (kTicketGroups + 1));
+        T *top = part + static_cast<size_t>(gridDim.x) * gridDim.y * gridDim.z * kColTile + t * kTicketGroups * kColTile;
+        if (!last_block_ticket(ctr(cg, g), size, &flag)) return;
+        if (owner)
+            st_dev(&top[g * kColTile + tid],
+                   combine_partials<Op>(part + (slot + g * kPartGroup) * kColTile + tid, size, kColTile, Op::identity()));
+        if (!last_block_ticket(ctr(cg, kTicketGroups), groups, &flag)) return;
+        if (put)
+            write_out<Op>(out, o * inner + oc, combine_partials<Op>(top + tid, groups, kColTile, Op::identity()));
     }
     tl_mark(kTlColsArg, 3);
 }
@@ -770,6 +853,147 @@ __global__ __launch_bounds__(16 * kWave) void k_cols_whole(const float *__restri
     tl_mark(kTlCols, 3);
 }
 
+// Narrow slices (kFlatInner) read flat.  A slice is one run of len = dim * inner
+// floats; a workgroup's first `act` threads take consecutive float4s and step by
+// act, with 4 act a whole number of rows, so each of a thread's four
+// components stays in one column ((4 tid + c) % inner) for good: coalesced
+// 128-bit loads at any inner, every lane at work, where a 256-column tile of
+// k_cols left 256 - inner columns' lanes idle and an inner that is not a
+// multiple of 4 read one dword per lane at a time.  Batches of UNR loads; the
+// last one is clamped to the run's end and shifted into place.  Columns
+// meet in LDS by halving (entry e belongs to column e % inner).  Chunks of a
+// slice are combined in a fixed order by its last workgroup.  Measured (sum,
+// us, against tiles of dword loads): [4096, 10] 7.0 -> 5.0, [100000, 10] 27.0
+// -> 5.7, [262144, 4] 24.7 -> 5.7, [160, 404, 3] 8.5 -> 3.8.
+template <class Op>
+__device__ __forceinline__ void lds_fold_cols(typename Op::T *lds, unsigned groups, unsigned inner, unsigned nt) {
+    __syncthreads();
+    while (groups > 1) {
+        const unsigned half = (groups + 1) / 2, n = (groups - half) * inner;
+        for (unsigned e = threadIdx.x; e < n; e += nt) lds[e] = Op::combine(lds[e], lds[e + half * inner]);
+        __syncthreads();
+        groups = half;
+    }
+}
+
+template <class Op, int NT, int UNR>
+__global__ __launch_bounds__(NT) void k_cols_flat(const float *__restrict__ x, unsigned inner, unsigned act,
+                                                  size_t len, unsigned chunks, size_t chunk_floats,
+                                                  typename Op::T *__restrict__ part, unsigned *__restrict__ counters,
+                                                  OutDesc out) {
+    using T = typename Op::T;
+    __shared__ T lds[4 * NT];
+    __shared__ int flag;
+    const unsigned tid = threadIdx.x;
+    const unsigned o = blockIdx.x / chunks, chunk = blockIdx.x - o * chunks;
+    const float *__restrict__ xo = x + static_cast<size_t>(o) * len;
+    const size_t f0 = chunk * chunk_floats;
+    const size_t f1 = f0 + chunk_floats < len ? f0 + chunk_floats : len;
+    const unsigned rps = 4 * act / inner;  // rows per step
+    const bool on = tid < act;
+    T acc[4] = {Op::identity(), Op::identity(), Op::identity(), Op::identity()};
+    unsigned rc[4];
+    float kc[4] = {0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+    for (int c = 0; c < 4; ++c) {
+        const unsigned e = 4 * tid + c;
+        rc[c] = e / inner;  // row within a step
+        if constexpr (Op::kShift) kc[c] = on ? xo[e - rc[c] * inner] : 0.0f;
+    }
+    if (on) {
+        unsigned row = static_cast<unsigned>(f0 / inner);  // first row of the current step (arg indices fit 31 bits)
+        const unsigned step = 16u * act;  // bytes
+        size_t f = f0;
+        for (; f + static_cast<size_t>(UNR) * 4 * act <= f1; f += static_cast<size_t>(UNR) * 4 * act) {
+            float4 v[UNR];
+            const char *cb = reinterpret_cast<const char *>(xo + f);
+#pragma unroll
+            for (int u = 0; u < UNR; ++u)
+                v[u] = ld4_any_stream<false>(reinterpret_cast<const float *>(cb + (16u * tid + u * step)));
+            __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+            for (int u = 0; u < UNR; ++u) {
+                const float e[4] = {v[u].x, v[u].y, v[u].z, v[u].w};
+#pragma unroll
+                for (int c = 0; c < 4; ++c)
+                    acc[c] = Op::accum(acc[c], Op::kShift ? e[c] - kc[c] : e[c], static_cast<int>(row + u * rps + rc[c]));
+            }
+            row += UNR * rps;
+        }
+        if (f < f1) {  // fewer than UNR whole steps: loads clamped to the run's last four floats
+            const int n = static_cast<int>(f1 - f);
+            float4 v[UNR];
+            const float *cb = xo + f;
+#pragma unroll
+            for (int u = 0; u < UNR; ++u) v[u] = ld4_any_stream<false>(cb + tail_off(static_cast<int>(tid + u * act), n));
+            __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+            for (int u = 0; u < UNR; ++u) {
+                const int i = static_cast<int>(tid + u * act), d = 4 * i - tail_off(i, n);
+                float e[4] = {v[u].x, v[u].y, v[u].z, v[u].w};
+                if (d > 0) {  // component c is component c + d of what was loaded
+                    e[0] = d == 1 ? e[1] : d == 2 ? e[2] : e[3];
+                    e[1] = d == 1 ? e[2] : e[3];
+                    e[2] = e[3];
+                }
+#pragma unroll
+                for (int c = 0; c < 4; ++c)
+                    if (c + d < 4)
+                        acc[c] = Op::accum(acc[c], Op::kShift ? e[c] - kc[c] : e[c],
+                                           static_cast<int>(row + u * rps + rc[c]));
+            }
+        }
+        if constexpr (std::is_same_v<T, ArgPair>) {
+            if (chunk == 0) {
+#pragma unroll
+                for (int c = 0; c < 4; ++c)
+                    if (4 * tid + c < inner) first_nan_fix<Op>(acc[c], xo[4 * tid + c]);  // row 0
+            }
+        }
+#pragma unroll
+        for (int c = 0; c < 4; ++c) lds[4 * tid + c] = acc[c];
+    }
+    lds_fold_cols<Op>(lds, rps, inner, NT);
+    const size_t ob = static_cast<size_t>(o) * inner;
+    if (chunks == 1) {
+        for (unsigned j = tid; j < inner; j += NT) write_out<Op>(out, ob + j, lds[j]);
+        return;
+    }
+    T *po = part + static_cast<size_t>(o) * chunks * inner;
+    for (unsigned j = tid; j < inner; j += NT) st_dev(&po[static_cast<size_t>(chunk) * inner + j], lds[j]);
+    const bool last = chunks <= kTicketGroups ? last_block_ticket(ctr(counters, o), chunks, &flag)
+                                              : last_block_ticket2<kTicketGroups>(
+                                                    ctr(counters, static_cast<size_t>(o) * (kTicketGroups + 1)), chunks,
+                                                    chunk, &flag);
+    if (!last) return;
+    // q sets of chunks side by side, then folded like the columns above
+    const unsigned sets = inner < NT ? (NT / inner < chunks ? NT / inner : chunks) : 1u;
+    for (unsigned e = tid; e < sets * inner; e += NT) {
+        const unsigned q = e / inner;
+        lds[e] = combine_partials<Op>(po + e, (chunks - q + sets - 1) / sets, static_cast<size_t>(sets) * inner,
+                                      Op::identity());
+    }
+    lds_fold_cols<Op>(lds, sets, inner, NT);
+    for (unsigned j = tid; j < inner; j += NT) write_out<Op>(out, ob + j, lds[j]);
+}
+
+// Slices (or rows, as slices of one column) of fewer than four floats: one
+// thread per result.  Sum over the rows of [262144, 3]: 109 -> 3.5 us.
+template <class Op>
+__global__ __launch_bounds__(kBlock) void k_cols_few(const float *__restrict__ x, size_t outer, unsigned dim,
+                                                     unsigned inner, OutDesc out) {
+    const size_t q = static_cast<size_t>(blockIdx.x) * kBlock + threadIdx.x;
+    if (q >= outer * inner) return;
+    const size_t o = q / inner;
+    const float *xc = x + o * dim * inner + (q - o * inner);
+    typename Op::T a = Op::identity();
+    for (unsigned r = 0; r < dim; ++r)
+        a = Op::accum(a, Op::kShift ? xc[static_cast<size_t>(r) * inner] - xc[0] : xc[static_cast<size_t>(r) * inner],
+                      static_cast<int>(r));
+    first_nan_fix<Op>(a, xc[0]);
+    write_out<Op>(out, q, a);
+}
+
 __global__ void k_fill_f32(float *z, float v) { *z = v; }
 
 // ------------------------------------------------------------------ host
@@ -781,6 +1005,20 @@ void launch_rows(unsigned nb, hipStream_t hs, const float *x, size_t dim, unsign
                  typename Op::T *part, unsigned *counters, const TaggedSlots &tg, OutDesc out) {
     hipLaunchKernelGGL((k_rows<Op, UNR, MODE>), dim3(nb), dim3(kBlock), 0, hs, x, dim, segs, seg4, part, counters,
                        tg.slots, tg.epoch, tg.clear, exchange_wait_limit(), out);
+}
+
+// Whole aligned rows of one batch (k_rows_whole), many enough to fill the chip.
+template <class Op>
+bool use_whole(const float *x, size_t rows, size_t dim) {
+    const size_t nt = whole_block<Op>(), v4 = dim / 4;
+    return rows >= kTargetBlocks && aligned16(x) && dim % 4 == 0 && (v4 == 4 * nt || v4 == 8 * nt || v4 == 16 * nt);
+}
+// Rows of up to 4096 floats in registers; whole aligned rows keep their own
+// kernel ([4096, 4096] sum 10.5 us there, 11.5 here; [4096, 3000] 9.2 in the
+// workgroup-per-row form, 8.8 here).  A single row is the flat form's.
+template <class Op>
+bool use_short(const float *x, size_t rows, size_t dim) {
+    return rows > 1 && dim >= 4 && dim <= 4096 && rows <= 0x7fffffffu && !use_whole<Op>(x, rows, dim);
 }
 
 // Row plan: each row cut into `segs` segments of seg4 float4s (a multiple
@@ -796,8 +1034,36 @@ int run_rows(const float *x, size_t rows, size_t dim, OutDesc out, cxm_stream_t 
         return launch_status();
     }
     const size_t v4 = (dim + 3) / 4;  // float4s of the longest aligned body (rounded up; a row has at most this many)
+    if (dim < 4 && rows > 1) {  // a thread per row
+        const size_t blocks = (rows + kBlock - 1) / kBlock;
+        if (rows > 0x7fffffffu) return CXM_E_TOO_LARGE;
+        hipLaunchKernelGGL(k_cols_few<Op>, dim3(static_cast<unsigned>(blocks)), dim3(kBlock), 0, hs, x, rows,
+                           static_cast<unsigned>(dim), 1u, out);
+        return launch_status();
+    }
+    if (use_short<Op>(x, rows, dim)) {
+        const int d = static_cast<int>(dim);
+#define CXM_SHORT(G, NV)                                                                                            \
+    hipLaunchKernelGGL((k_rows_short<Op, G, NV>), dim3(static_cast<unsigned>((rows + kBlock / G - 1) / (kBlock / G))), \
+                       dim3(kBlock), 0, hs, x, rows, d, out)
+        if (v4 <= 4) CXM_SHORT(4, 1);
+        else if (v4 <= 8) CXM_SHORT(8, 1);
+        else if (v4 <= 16) CXM_SHORT(16, 1);
+        else if (v4 <= 32) CXM_SHORT(32, 1);
+        else if (v4 <= 64) CXM_SHORT(64, 1);
+        else if (v4 <= 128) CXM_SHORT(64, 2);
+        else if (v4 <= 256) CXM_SHORT(64, 4);
+        else if (v4 <= 512) CXM_SHORT(64, 8);
+        else CXM_SHORT(64, 16);
+#undef CXM_SHORT
+        return launch_status();
+    }
     size_t segs = 1;
-    if (rows < kTargetBlocks) {
+    // split rows only where there are too few of them: a workgroup per row ran
+    // [1500, 5000] in 6.4 us against 10.1 in two segments, [688, 10698] in 7.0
+    // against 8.2, [1000, 65536] in 38 against 44, but [300, 200000] in 45
+    // against 41
+    if (rows < 256 || (rows < 512 && dim > 32768)) {
         const size_t want = (kTargetBlocks + rows - 1) / rows;
         const size_t max_segs = (v4 + 255) / 256;
         segs = want < max_segs ? want : max_segs;
@@ -818,7 +1084,7 @@ int run_rows(const float *x, size_t rows, size_t dim, OutDesc out, cxm_stream_t 
     TaggedSlots tg{nullptr, 0, 0, 0};
     const int mode = segs == 1 ? 0 : (rows == 1 && sizeof(T) == 4 && segs <= kMaxFlatSegs ? 2 : 1);
     // whole aligned rows of one batch (every row starts 16-byte aligned)
-    if (mode == 0 && aligned16(x) && dim % 4 == 0) {
+    if (mode == 0 && use_whole<Op>(x, rows, dim)) {
         const unsigned nr = static_cast<unsigned>(rows);
         constexpr int nt = whole_block<Op>();
 #define CXM_WHOLE(U)                                                                                    \
@@ -858,20 +1124,21 @@ int run_rows(const float *x, size_t rows, size_t dim, OutDesc out, cxm_stream_t 
 }
 
 struct ColPlan {
-    int nw;          // waves per workgroup (4 or 16)
     size_t chunks;   // row chunks per column tile
 };
 
-// Default plan: 16-wave workgroups, about one per CU in total from 16
-// column tiles up and about 128 below (few chunks, so the last-workgroup
-// combine reads few partials).  Measured chunk sweeps (column sum, us):
-// [4096, 1024] 64 chunks 8.2, 32 chunks 7.0; [2048, 2048] 32: 7.2, 16: 6.5;
-// [8192, 512] 128: 11.0, 64: 8.1; [4096, 4096] 16: 13.1, 8: 14.8.
+// Default plan: 16-wave workgroups, at most one per CU (a few more would run
+// as a second round: [16384, 1280] 22.1 us with 260, 16.6 with 255).  More than 32 chunks
+// per tile meet in two levels; with all partials read by one workgroup, 128
+// workgroups in total had been the better plan for fewer than 16 tiles.
+// Measured then and now (column sum, us): [32450, 384] 16.1 -> 11.6,
+// [65536, 256] 20.8 -> 16.4, [16384, 256] 10.6 -> 6.9, [16000, 1001] 41.5 ->
+// 15.0, [8192, 512] 7.9 -> 7.0, [4096, 1024] 6.7 -> 6.6.
 ColPlan col_plan(size_t tiles, size_t dim) {
-    ColPlan p{16, 1};
-    const size_t target = tiles >= 16 ? 256 : 128;
+    ColPlan p{1};
+    const size_t target = 256;
     if (tiles < target) {
-        size_t want = (target + tiles - 1) / tiles;
+        size_t want = target / tiles;
         const size_t max_chunks = (dim + 63) / 64;  // >= 4 rows per wave
         p.chunks = want < max_chunks ? want : max_chunks;
         if (p.chunks == 0) p.chunks = 1;
@@ -879,7 +1146,79 @@ ColPlan col_plan(size_t tiles, size_t dim) {
     return p;
 }
 
-template <class Op, int UNRC = 8>
+constexpr size_t kColPartBytes = kFixedPartBytes;  // most partials a flat plan makes (the static region's share)
+
+// Flat plan (k_cols_flat) of [outer, dim, inner]: threads per workgroup, of
+// them at work, chunks per slice and their length.
+struct FlatPlan {
+    unsigned nt, act;
+    size_t chunks, chunk_floats;
+};
+constexpr int kFlatUnr = 8;
+size_t gcd4(size_t n) { return n % 4 == 0 ? 4 : n % 2 == 0 ? 2 : 1; }
+FlatPlan flat_plan(size_t outer, size_t dim, size_t inner, size_t elem) {
+    const size_t len = dim * inner, p = inner / gcd4(inner);  // p float4s: the fewest that are whole rows
+    FlatPlan f{};
+    f.nt = len <= 64 * 4 * kFlatUnr ? 64u : 256u;  // p <= kFlatInner
+    f.act = static_cast<unsigned>(f.nt / p * p);
+    const size_t step = 4 * static_cast<size_t>(f.act), steps = (len + step - 1) / step;
+    // about four 256-thread workgroups per CU, each with a batch of loads at
+    // least ([100000, 10] sum: 6.0 us with 512 workgroups in all, 5.7 with 1024)
+    size_t chunks = outer < 1024 ? 1024 / outer : 1;
+    const size_t most = (steps + kFlatUnr - 1) / kFlatUnr;
+    if (chunks > most) chunks = most;
+    while (chunks > 1 && outer * chunks * inner * elem > kColPartBytes) --chunks;
+    const size_t per = (steps + chunks - 1) / chunks;
+    f.chunk_floats = per * step;
+    f.chunks = (len + f.chunk_floats - 1) / f.chunk_floats;
+    return f;
+}
+
+template <class Op>
+int run_cols_flat(const float *x, size_t outer, size_t dim, size_t inner, OutDesc out, cxm_stream_t s, bool fixed) {
+    using T = typename Op::T;
+    hipStream_t hs = reinterpret_cast<hipStream_t>(s);
+    const size_t len = dim * inner;
+    FlatPlan f = flat_plan(outer, dim, inner, sizeof(T));
+    T *part = nullptr;
+    unsigned *counters = nullptr;
+    if (f.chunks > 1) {
+        Scratch sc;
+        const size_t nctr = f.chunks <= kTicketGroups ? outer : outer * (kTicketGroups + 1);
+        const int rc = acquire(fixed, s, nctr, outer * f.chunks * inner * sizeof(T), 0, &sc);
+        if (rc) {  // no scratch to be had (a capturing stream's first call): one workgroup per slice
+            (void)hipGetLastError();
+            f.chunks = 1;
+            f.chunk_floats = len;
+        } else {
+            part = static_cast<T *>(sc.part);
+            counters = sc.counters;
+        }
+    }
+    const size_t blocks = outer * f.chunks;
+    if (blocks * f.nt > 0xffffffffu) return CXM_E_TOO_LARGE;
+    const dim3 grid(static_cast<unsigned>(blocks)), block(f.nt);
+    const unsigned in = static_cast<unsigned>(inner), nc = static_cast<unsigned>(f.chunks);
+    if (f.nt == 64)
+        hipLaunchKernelGGL((k_cols_flat<Op, 64, kFlatUnr>), grid, block, 0, hs, x, in, f.act, len, nc, f.chunk_floats,
+                           part, counters, out);
+    else
+        hipLaunchKernelGGL((k_cols_flat<Op, 256, kFlatUnr>), grid, block, 0, hs, x, in, f.act, len, nc, f.chunk_floats,
+                           part, counters, out);
+    return launch_status();
+}
+
+// Flat for up to 64 columns, column tiles beyond.  Measured (sum, us, flat
+// against tiles): [4096, 10] 5.0 / 5.3, [100000, 10] 5.7 / 12.3, [30000, 33]
+// 6.0 / 7.6, [4096, 64] 4.6 / 5.2, but [4000, 100] 5.7 / 5.2, [40000, 100] 18.5
+// / 10.0, [7000, 130] 12.2 / 6.6: a tile's 256 columns are combined by as many
+// workgroups as there are tiles, a flat slice's by one.
+constexpr size_t kFlatInner = 64;
+
+constexpr size_t kColWaves = 16;  // waves per k_cols workgroup
+constexpr size_t kFewRows = 64;
+
+template <class Op>
 int run_cols_plan(const float *x, size_t outer, size_t dim, size_t inner, OutDesc out, ColPlan plan,
                   cxm_stream_t s, bool fixed = false) {
     using T = typename Op::T;
@@ -899,7 +1238,8 @@ int run_cols_plan(const float *x, size_t outer, size_t dim, size_t inner, OutDes
     unsigned *counters = nullptr;
     if (chunks > 1) {
         Scratch sc;
-        int rc = acquire(fixed, s, tiles, tiles * chunks * kColTile * sizeof(T), 0, &sc);
+        int rc = acquire(fixed, s, chunks <= kTicketGroups ? tiles : tiles * (kTicketGroups + 1),
+                         tiles * (chunks <= kTicketGroups ? chunks : chunks + kTicketGroups) * kColTile * sizeof(T), 0, &sc);
         if (rc) return rc;
         part = static_cast<T *>(sc.part);
         counters = sc.counters;
@@ -912,37 +1252,42 @@ int run_cols_plan(const float *x, size_t outer, size_t dim, size_t inner, OutDes
     const bool fast = vec && inner % kColTile == 0 &&
                       (rpc * inner + kColTile) * sizeof(float) < (size_t(1) << 31) && ntiles <= 65535 &&
                       outer <= 65535;
-    if (!fast && blocks * static_cast<size_t>(plan.nw) * kWave > 0xffffffffu) return CXM_E_TOO_LARGE;
+    if (!fast && blocks * kColWaves * kWave > 0xffffffffu) return CXM_E_TOO_LARGE;
     const dim3 grid = fast ? dim3(nc, nt, static_cast<unsigned>(outer)) : dim3(static_cast<unsigned>(blocks));
-#define CXM_COLS(VEC_, UNR_, NW_)                                                                              \
-    do {                                                                                                       \
-        if (VEC_ && fast)                                                                                      \
-            hipLaunchKernelGGL((k_cols<Op, VEC_, UNR_, NW_, true>), grid, dim3(NW_ * kWave), 0, hs, x, dim,      \
-                               inner, nt, nc, rpc, part, counters, out);                                       \
-        else                                                                                                   \
-            hipLaunchKernelGGL((k_cols<Op, VEC_, UNR_, NW_>), grid, dim3(NW_ * kWave), 0, hs, x, dim, inner,      \
-                               nt, nc, rpc, part, counters, out);                                              \
-    } while (0)
+    // tiles of equal width: with the last tile only a few columns wide, half
+    // the workgroups of an inner of 257 would stream next to nothing
+    const unsigned width = static_cast<unsigned>(((inner + 3) / 4 + ntiles - 1) / ntiles * 4);
+#define CXM_COLS(AL_, UNR_, FAST_, NW)                                                                              \
+    hipLaunchKernelGGL((k_cols<Op, AL_, UNR_, NW, FAST_>), grid, dim3(NW * kWave), 0, hs, x, dim, inner, nt, width, nc, \
+                       rpc, part, counters, out)
     if constexpr (sizeof(T) == 4) {  // the column argmax measured 14.3 -> 14.5 us in this form
-        if (fast && plan.nw == 16 && chunks > 1 && rpc == kWholeRows && dim == chunks * kWholeRows &&
+        if (fast && chunks > 1 && chunks <= kTicketGroups && rpc == kWholeRows && dim == chunks * kWholeRows &&
             inner <= 0xffffffffu) {
             hipLaunchKernelGGL(k_cols_whole<Op>, grid, dim3(16 * kWave), 0, hs, x, dim * inner,
                                static_cast<unsigned>(inner), nt, nc, part, counters, out);
             return launch_status();
         }
     }
-    if (plan.nw == 16) {
-        // With a multiple of 16 rows per wave, all 16 loads of a batch are in
-        // flight together (C2's column reductions: 13.4 against 13.8 us with
-        // batches of 8); other chunk sizes keep batches of UNRC, since rows
-        // past the last whole batch load one at a time.
-        if (vec && (rpc / 16) % 16 == 0) CXM_COLS(true, 16, 16);
-        else if (vec) CXM_COLS(true, UNRC, 16);
-        else CXM_COLS(false, 1, 16);
-    } else {
-        if (vec) CXM_COLS(true, UNRC, 4);
-        else CXM_COLS(false, 1, 4);
-    }
+    // With a multiple of 16 rows per wave, all 16 loads of a batch are in
+    // flight together (C2's column reductions: 13.4 against 13.8 us with
+    // batches of 8).  Other chunk sizes take batches of 8 or, for at most 4
+    // rows per wave, 4; so do tiles of more than 32 chunks ([65536, 256] sum
+    // 16.4 against 18.2 us, [16384, 1024] 16.4 against 17.2).
+    // Few rows and no chunks: four waves per tile with all of their rows in
+    // flight (sixteen would have a row or two each: [304, 22, 864] sum 7.7 us with 16 waves, 6.1 with 4).
+    const bool few = chunks == 1 && dim <= kFewRows;
+    const size_t rw = few ? (dim + 3) / 4 : rpc / kColWaves;  // rows per wave
+#define CXM_COLS_UNR(AL_, FAST_)                                                       \
+    if (few && rw <= 2) CXM_COLS(AL_, 2, FAST_, 4);                                    \
+    else if (few && rw <= 4) CXM_COLS(AL_, 4, FAST_, 4);                               \
+    else if (few) CXM_COLS(AL_, 8, FAST_, 4);                                          \
+    else if (rw % 16 == 0 && nc <= kTicketGroups) CXM_COLS(AL_, 16, FAST_, kColWaves); \
+    else if (rw <= 4) CXM_COLS(AL_, 4, FAST_, kColWaves);                              \
+    else CXM_COLS(AL_, 8, FAST_, kColWaves)
+    if (fast) { CXM_COLS_UNR(true, true); }
+    else if (vec) { CXM_COLS_UNR(true, false); }
+    else { CXM_COLS_UNR(false, false); }
+#undef CXM_COLS_UNR
 #undef CXM_COLS
     return launch_status();
 }
@@ -950,6 +1295,15 @@ int run_cols_plan(const float *x, size_t outer, size_t dim, size_t inner, OutDes
 template <class Op>
 int run_cols(const float *x, size_t outer, size_t dim, size_t inner, OutDesc out, cxm_stream_t s,
              bool fixed = false) {
+    if (dim * inner < 4) {
+        const size_t blocks = (outer * inner + kBlock - 1) / kBlock;
+        if (blocks > 0xffffffu) return CXM_E_TOO_LARGE;
+        hipLaunchKernelGGL(k_cols_few<Op>, dim3(static_cast<unsigned>(blocks)), dim3(kBlock), 0,
+                           reinterpret_cast<hipStream_t>(s), x, outer, static_cast<unsigned>(dim),
+                           static_cast<unsigned>(inner), out);
+        return launch_status();
+    }
+    if (inner <= kFlatInner) return run_cols_flat<Op>(x, outer, dim, inner, out, s, fixed);
     const size_t tiles = (inner + kColTile - 1) / kColTile * outer;
     return run_cols_plan<Op>(x, outer, dim, inner, out, col_plan(tiles, dim), s, fixed);
 }

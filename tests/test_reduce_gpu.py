@@ -15,6 +15,8 @@ from cortexmind_amd._lib import E_INVALID, call, lib
 from cortexmind_amd.data import SplitMix64, c2_reduce
 from cortexmind_amd.device import DeviceArray
 
+from gpu_util import bits_equal, dev, empty
+
 pytestmark = pytest.mark.gpu
 
 SUM_TOL = 1e-5
@@ -261,3 +263,81 @@ def test_unaligned_ragged_rows(hip, orc, off, sizes, op):
     x = SplitMix64(off * 7919 + sum(sizes)).normal(sizes if len(sizes) > 1 else sizes[0], 0.0, 2.0)
     check(op, x, sizes, orc, ptr_offset_floats=off)
 
+
+
+@pytest.mark.parametrize("sizes", [(1, 1, 2), (3, 1, 3), (2, 2, 2), (1, 2, 3), (1, 1, 4), (5, 3, 5), (160, 404, 3),
+                                   (1, 100003, 10), (1, 5000, 64), (2, 700, 63), (3, 1000, 257), (300, 9, 257),
+                                   (1, 4000, 255), (2, 65, 1021), (1, 3000, 1024), (1, 513, 1025), (2, 100, 1031),
+                                   (1, 1000, 4099), (1, 37, 4100)])
+@pytest.mark.parametrize("off", [0, 1])
+def test_columns_of_any_width(hip, orc, sizes, off):
+    """The flat column kernel at the edges of its plan (fewer floats than a
+    float4, one to three columns, thread counts that are not whole waves,
+    several chunks per slice with a ragged last one, both tickets) and the
+    column tiles it hands over to, each with rows that are no multiple of 4
+    and bases that are only 4-byte aligned."""
+    o, d, i = sizes
+    x = SplitMix64(0xC015 + 7 * o + 3 * d + i).uniform((o, d, i), -1.0, 1.0)
+    if d > 2:
+        x[0, :, 0] = x[0, 1, 0]  # ties: the first index wins
+        x[o - 1, 0, i - 1] = np.nan
+    dx = dev(x, off)
+    for op in ("sum", "mean", "max", "min", "argmax", "argmin", "norm1", "norm2", "var"):
+        z = empty((o, i), np.int32 if op.startswith("arg") else np.float32)
+        getattr(engine.reduce, op)(dx, z, o, d, i)
+        got = z.numpy()
+        x64 = x.astype(np.float64)
+        if op in ("max", "min"):
+            assert bits_equal(got, getattr(np, op)(x, axis=1))  # np.max / np.min give NaN for the NaN column
+        elif op.startswith("arg"):
+            # a NaN in the first row stays the answer (index 0), as does the first of equal values
+            assert np.array_equal(got, getattr(np, op)(x, axis=1))
+        else:
+            ref = {"sum": lambda: x64.sum(axis=1), "mean": lambda: x64.mean(axis=1),
+                   "norm1": lambda: np.abs(x64).sum(axis=1), "norm2": lambda: np.sqrt((x64 * x64).sum(axis=1)),
+                   "var": lambda: x64.var(axis=1)}[op]()
+            size = np.abs(x64).sum(axis=1) / (d if op == "mean" else 1)
+            if op in ("norm2", "var"):
+                size = ref + 1e-7
+            fin = np.isfinite(ref)
+            if op != "var":  # (a NaN among the deviations gives a variance of 0)
+                assert np.array_equal(fin, np.isfinite(got))
+            assert np.all(np.abs(got - ref)[fin] <= 1e-5 * size[fin])
+
+
+@pytest.mark.parametrize("dim", [1, 2, 3, 4, 5, 15, 16, 17, 31, 33, 63, 64, 65, 127, 129, 255, 257, 511, 513, 1003, 1025,
+                                 2047, 2049, 4095, 4097, 10698])
+@pytest.mark.parametrize("off", [0, 1])
+def test_rows_of_any_length(hip, dim, off):
+    """Short rows at the edges of their lanes-per-row and float4-per-lane
+    ranges, with a last workgroup partly empty, NaN and ties included."""
+    rows = 131
+    x = SplitMix64(0x50A7 + dim).uniform((rows, dim), -1.0, 1.0)
+    x[3, :] = -np.inf
+    x[4, :] = x[4, 0]
+    x[5, 0] = np.nan
+    dx = dev(x, off)
+    for op in ("sum", "mean", "max", "min", "argmax", "argmin", "norm1", "norm2", "var"):
+        z = empty((rows,), np.int32 if op.startswith("arg") else np.float32)
+        getattr(engine.reduce, op)(dx, z, rows, dim, 1)
+        got = z.numpy()
+        x64 = x.astype(np.float64)
+        if op in ("max", "min"):
+            ref = getattr(np, op)(x, axis=1)
+            if op == "max":
+                ref[3] = -np.finfo(np.float32).max  # the running maximum starts there
+            assert bits_equal(got, ref)
+        elif op.startswith("arg"):
+            assert np.array_equal(got, getattr(np, op)(x, axis=1))
+        else:
+            with np.errstate(invalid="ignore"):
+                ref = {"sum": lambda: x64.sum(axis=1), "mean": lambda: x64.mean(axis=1),
+                       "norm1": lambda: np.abs(x64).sum(axis=1), "norm2": lambda: np.sqrt((x64 * x64).sum(axis=1)),
+                       "var": lambda: x64.var(axis=1)}[op]()
+                size = np.abs(x64).sum(axis=1) / (dim if op == "mean" else 1)
+            if op in ("norm2", "var"):
+                size = ref + 1e-7
+            fin = np.isfinite(ref)
+            assert np.all(np.abs(got - ref)[fin] <= 1e-5 * size[fin])
+            if op != "var":
+                assert np.array_equal(np.isnan(ref), np.isnan(got))
