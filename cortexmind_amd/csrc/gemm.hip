@@ -22,7 +22,7 @@
 // C[8*(r/4) + 4*(l/32) + r%4][l%32].
 #include <atomic>
 
-#include "cxm_common.hpp"
+#include "gemm_epi.hpp"
 #include "mlp_side.hpp"
 
 // Per-workgroup timeline of the ring products, for the diagnostics build only
@@ -53,8 +53,6 @@ __device__ __forceinline__ void gemm_tl_mark(unsigned, unsigned) {}
 namespace cxm {
 namespace {
 
-typedef float floatx16 __attribute__((ext_vector_type(16)));
-
 constexpr int BM = 128, BN = 128, BK = 32, PAD = 4;
 constexpr int KQ = BK / 4;                      // 4-element groups along k in a tile row
 constexpr int kGemmThreads = 512;               // 8 waves: 2 (m) x 4 (n), each 64 x 32 of C
@@ -62,15 +60,6 @@ constexpr int WI = 2, WJ = 1;                   // 32x32 MFMA tiles per wave alo
 constexpr int SLOTS = BM * BK / 4 / kGemmThreads;  // float4 groups per thread per tile (A and B alike)
 constexpr int kColTileThin = 256;  // m columns per workgroup of the thin TN kernel
 
-
-// Workgroups are dispatched to the 8 XCDs round-robin (workgroup b runs on
-// XCD b % 8).  Renumbering b so that each XCD gets one contiguous eighth of
-// the row-major tile order makes the tiles sharing an XCD's L2 share A rows
-// (and B columns), instead of every XCD touching every row block.
-__device__ __forceinline__ unsigned xcd_remap(unsigned b, unsigned g) {
-    if (g % 8 != 0) return b;
-    return (b % 8) * (g / 8) + b / 8;
-}
 
 __device__ __forceinline__ void store_epi(const Epilogue &e, float *C, size_t row, size_t col, size_t N,
                                           float v) {
@@ -94,15 +83,6 @@ __device__ __forceinline__ void store_epi(const Epilogue &e, float *C, size_t ro
 // one straight block: loads, then arithmetic, then stores.  Element by
 // element, each store waited for its own load (a memory round trip per
 // element, 11 us of a 4096 x 1024 x 1024 product with a ReLU gate).
-__device__ __forceinline__ float epi_value(const Epilogue &e, float v, float bias, float pre) {
-    const float t = v * e.lr;  // SGD: matrix_t::sub(W, ScalarOp::mul(G, lr)): two roundings
-    const float sgd = pre - t;
-    float u = e.bias ? v + bias : v;
-    u = (e.act == CXM_ACT_RELU && 0.0f > u) ? 0.0f : u;
-    u = e.gate ? u * (pre > 0.0f ? 1.0f : 0.0f) : u;
-    return e.sgd ? sgd : u;
-}
-
 template <int WI_, int WJ_, class RowF, class ColF>
 __device__ __forceinline__ void store_tile_epi(const floatx16 (&acc)[WI_][WJ_], float *__restrict__ C, size_t M,
                                                size_t N, RowF row_of, ColF col_of, const Epilogue &e) {
@@ -1413,6 +1393,10 @@ int gemm_ex(const float *A, const float *B, float *C, size_t M, size_t K, size_t
     if (K == 0) return CXM_E_INVALID;
     {
         const int t = gemm_thin(A, B, C, M, K, N, ta, tb, epi, st);
+        if (t != 1) return t;
+    }
+    if (g_gemm_kc.load(std::memory_order_relaxed) < 0) {  // no kernel pinned
+        const int t = gemm_direct(A, B, C, M, K, N, ta, tb, epi, ring_shape_ok(A, B, M, K, N, ta, tb), st);
         if (t != 1) return t;
     }
     const size_t tiles_m = (M + BM - 1) / BM, tiles_n = (N + BN - 1) / BN;

@@ -1,0 +1,394 @@
+// fp32 products whose operands go straight from memory to the MFMA's
+// registers: small ones, and ragged ones of any size.
+//
+// The ring kernel of gemm.hip wants 16-byte aligned operands and 128x128
+// tiles; a product of a few hundred rows and columns leaves it on a handful
+// of CUs, where one tile of K = 784 takes 37 us of one CU's matrix cores.
+// Here a workgroup's NW waves all compute the same 32 WI x 32 WJ tile, each
+// over its own 8-k blocks (wave w takes blocks w, w + NW, ...: the four
+// blocks of a 128-byte line are read by waves of one CU at about the same
+// time), with no LDS and no barrier until the end, where the waves' sums
+// meet in LDS in wave order.  K is split over workgroups as well when there
+// are too few tiles for the chip.  Bound by MFMA issue with one or two waves
+// per SIMD (the loads' latency shows) and, for 32x32 tiles, by L1; 4096x300x4095
+// reaches 90 TFLOP/s, 40x784x256 4.9 us.
+//
+// Operands.  In MFMA e of an 8-k block, lanes 0-31 supply k = 4 lhi + e with
+// lhi = 0, lanes 32-63 with lhi = 1.  An operand whose k runs along its rows
+// (A [M, K], B [N, K]) gives a lane four k with one dword-aligned 128-bit load
+// per 32 rows; one stored [K, M] or [K, N] gives 32 W columns of one k with W
+// adjacent floats per lane (columns W l32 .. W l32 + W - 1: block i of the
+// accumulator holds columns W l + i).  Rows past the end re-read the last
+// one, columns past the end re-read the last W: their products land in
+// accumulators that are not stored.
+#include "gemm_epi.hpp"
+
+namespace cxm {
+namespace {
+
+typedef float f32x2u __attribute__((ext_vector_type(2), aligned(4)));
+
+// k-contiguous operand X[r][k] or not: X[k][r]; W blocks of 32 rows.
+template <bool KC, int W>
+struct Side {
+    const float *base;  // uniform: the tile's first row (KC) or column
+    size_t ld;
+    unsigned off[KC ? W : 1];  // bytes from base to this lane's data of k block 0
+    int shift;                 // !KC, W = 2: 1 where the lane's pair was moved back by one column
+
+    __device__ __forceinline__ void init(const float *X, size_t r0, size_t rows, size_t ldx, int l32, int lhi) {
+        ld = ldx;
+        shift = 0;
+        if constexpr (KC) {
+            base = X + r0 * ldx;
+#pragma unroll
+            for (int i = 0; i < W; ++i) {
+                const size_t r = r0 + 32 * i + l32;
+                off[i] = static_cast<unsigned>((((r < rows ? r : rows - 1) - r0) * ldx + 4 * lhi) * sizeof(float));
+            }
+        } else {
+            base = X + r0;
+            // the last whole W columns when this lane's run past the end
+            const size_t c = r0 + W * l32, last = rows - W;
+            const size_t cc = c < last ? c : last;
+            shift = c == cc + 1 ? 1 : 0;
+            // cc may lie before r0 (a tile of one column): base is moved back with it
+            const size_t back = r0 < last ? 0 : r0 - last;
+            base -= back;
+            off[0] = static_cast<unsigned>((cc - (r0 - back) + 4 * static_cast<size_t>(lhi) * ldx) * sizeof(float));
+        }
+    }
+    // This lane's operands of the 8-k block at k: f[i][e], block i, MFMA e.
+    __device__ __forceinline__ void load(size_t k, float (&f)[W][4]) const {
+        if constexpr (KC) {
+            const char *b = reinterpret_cast<const char *>(base + k);
+#pragma unroll
+            for (int i = 0; i < W; ++i) {
+                const f32x4u v = *reinterpret_cast<const f32x4u *>(b + off[i]);
+                f[i][0] = v.x; f[i][1] = v.y; f[i][2] = v.z; f[i][3] = v.w;
+            }
+        } else {
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+                const char *b = reinterpret_cast<const char *>(base + (k + e) * ld);
+                if constexpr (W == 2) {
+                    const f32x2u v = *reinterpret_cast<const f32x2u *>(b + off[0]);
+                    f[0][e] = v.x;
+                    f[1][e] = v.y;
+                } else {
+                    f[0][e] = *reinterpret_cast<const float *>(b + off[0]);
+                }
+            }
+        }
+    }
+    // What load left for the use: the moved pair's first column is its second float.
+    __device__ __forceinline__ void settle(float (&f)[W][4]) const {
+        if constexpr (!KC && W == 2) {
+#pragma unroll
+            for (int e = 0; e < 4; ++e) f[0][e] = shift ? f[1][e] : f[0][e];
+        }
+    }
+    // The last, partial block: n < 8 valid k; the others are zero on both sides.
+    __device__ __forceinline__ void load_tail(size_t k, int n, int lhi, float (&f)[W][4]) const {
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+            const int kk = 4 * lhi + e;
+            const bool in = kk < n;
+            const int kc = in ? kk : n - 1;
+#pragma unroll
+            for (int i = 0; i < W; ++i) {
+                // off holds 4 lhi: step from there to kc
+                const long d = KC ? static_cast<long>(kc) - 4 * lhi : (static_cast<long>(kc) - 4 * lhi) * static_cast<long>(ld);
+                const char *b = reinterpret_cast<const char *>(base + (KC ? k : k * ld)) + off[KC ? i : 0];
+                const float v = reinterpret_cast<const float *>(b)[d + (KC ? 0 : i)];
+                f[i][e] = in ? v : 0.0f;
+            }
+        }
+    }
+};
+
+constexpr int kDepth = 3;  // 8-k blocks in flight per wave
+
+// The sum of a float4's split partials (components `plane` floats apart) in
+// split order, four splits of loads in flight.
+__device__ __forceinline__ float4 sum_splits(const float *p, int plane, unsigned splits, size_t stride) {
+    float4 a = make_float4(0.f, 0.f, 0.f, 0.f);
+    for (unsigned s0 = 0; s0 < splits; s0 += 4) {
+        float4 t[4];
+#pragma unroll
+        for (unsigned u = 0; u < 4; ++u) {
+            const float *d = p + static_cast<size_t>(s0 + u < splits ? s0 + u : splits - 1) * stride;
+            t[u] = make_float4(ld_dev(d), ld_dev(d + plane), ld_dev(d + 2 * plane), ld_dev(d + 3 * plane));
+        }
+#pragma unroll
+        for (unsigned u = 0; u < 4; ++u)
+            if (s0 + u < splits) {
+                a.x += t[u].x; a.y += t[u].y; a.z += t[u].z; a.w += t[u].w;
+            }
+    }
+    return a;
+}
+
+template <int WI, int WJ, int NW, bool KCA, bool KCB>
+__global__ __launch_bounds__(NW * kWave) void k_gemm_direct(const float *__restrict__ A, const float *__restrict__ B,
+                                                            float *__restrict__ C, size_t M, size_t N, size_t K,
+                                                            unsigned tiles_n, unsigned splits, size_t kper,
+                                                            Epilogue epi, float *__restrict__ part,
+                                                            unsigned *__restrict__ counters) {
+    constexpr int TM = 32 * WI, TN = 32 * WJ, LP = TN + 4;
+    constexpr int NT = NW * kWave, Q = 32 * TN / 4;  // float4s of a 32-row block
+    __shared__ __attribute__((aligned(16))) float sums[NW][32 * LP];
+    __shared__ int flag;
+    const unsigned wg = xcd_remap(blockIdx.x, gridDim.x);
+    const unsigned tile = wg / splits, split = wg - tile * splits;
+    const size_t m0 = static_cast<size_t>(tile / tiles_n) * TM, n0 = static_cast<size_t>(tile % tiles_n) * TN;
+    const size_t kbeg = static_cast<size_t>(split) * kper;
+    const size_t kend = kbeg + kper < K ? kbeg + kper : K;
+    const int lane = threadIdx.x & (kWave - 1), l32 = lane & 31, lhi = lane >> 5;
+    const unsigned w = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
+
+    Side<KCA, WI> a;
+    Side<KCB, WJ> b;
+    a.init(A, m0, M, KCA ? K : M, l32, lhi);
+    b.init(B, n0, N, KCB ? K : N, l32, lhi);
+
+    floatx16 acc[WI][WJ];
+#pragma unroll
+    for (int i = 0; i < WI; ++i)
+#pragma unroll
+        for (int j = 0; j < WJ; ++j)
+#pragma unroll
+            for (int r = 0; r < 16; ++r) acc[i][j][r] = 0.0f;
+
+    // whole blocks of this wave: w, w + NW, ... < nb
+    const unsigned nb = static_cast<unsigned>((kend - kbeg) / 8);
+    const unsigned T = nb > w ? (nb - w + NW - 1) / NW : 0;
+    const size_t k0 = kbeg + 8 * static_cast<size_t>(w);
+    auto at = [&](unsigned t) { return k0 + static_cast<size_t>(t < T ? t : T - 1) * (8 * NW); };
+    float fa[kDepth][WI][4], fb[kDepth][WJ][4];
+    auto mul = [&](float (&x)[WI][4], float (&y)[WJ][4]) {
+        a.settle(x);
+        b.settle(y);
+#pragma unroll
+        for (int e = 0; e < 4; ++e)
+#pragma unroll
+            for (int i = 0; i < WI; ++i)
+#pragma unroll
+                for (int j = 0; j < WJ; ++j)
+                    acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x2f32(x[i][e], y[j][e], acc[i][j], 0, 0, 0);
+    };
+    if (T > 0) {
+#pragma unroll
+        for (int d = 0; d < kDepth; ++d) {
+            a.load(at(d), fa[d]);
+            b.load(at(d), fb[d]);
+        }
+        __builtin_amdgcn_sched_barrier(0);
+        unsigned t = 0;
+        for (; t + kDepth <= T; t += kDepth) {
+#pragma unroll
+            for (int d = 0; d < kDepth; ++d) {
+                mul(fa[d], fb[d]);
+                a.load(at(t + d + kDepth), fa[d]);
+                b.load(at(t + d + kDepth), fb[d]);
+                __builtin_amdgcn_sched_barrier(0);
+            }
+        }
+#pragma unroll
+        for (int d = 0; d < kDepth; ++d)
+            if (t + d < T) mul(fa[d], fb[d]);
+    }
+    const int rest = static_cast<int>((kend - kbeg) % 8);
+    if (rest != 0 && w == nb % NW) {
+        float x[WI][4], y[WJ][4];
+        a.load_tail(kbeg + 8 * static_cast<size_t>(nb), rest, lhi, x);
+        b.load_tail(kbeg + 8 * static_cast<size_t>(nb), rest, lhi, y);
+        mul(x, y);
+    }
+
+    // the waves' sums meet in LDS, one 32-row block i of the accumulators at a
+    // time (a quarter or half of the LDS, so that more workgroups fit a CU)
+    constexpr int PT = (Q + NT - 1) / NT;  // float4s per thread and block
+    constexpr bool kAll = Q % NT == 0;     // every thread has PT of them
+    float4 v[WI][PT];
+#pragma unroll
+    for (int i = 0; i < WI; ++i) {
+        if (i > 0) __syncthreads();
+#pragma unroll
+        for (int j = 0; j < WJ; ++j)
+#pragma unroll
+            for (int r = 0; r < 16; ++r)
+                sums[w][(8 * (r / 4) + 4 * lhi + (r % 4)) * LP + (KCB ? 32 * j + l32 : WJ * l32 + j)] = acc[i][j][r];
+        __syncthreads();
+#pragma unroll
+        for (int p = 0; p < PT; ++p) {
+            const int q = threadIdx.x + p * NT;
+            if (!kAll && q >= Q) break;
+            const int o = (q / (TN / 4)) * LP + (q % (TN / 4)) * 4;
+            v[i][p] = *reinterpret_cast<const float4 *>(&sums[0][o]);
+#pragma unroll
+            for (int s = 1; s < NW; ++s) {
+                const float4 u = *reinterpret_cast<const float4 *>(&sums[s][o]);
+                v[i][p].x += u.x; v[i][p].y += u.y; v[i][p].z += u.z; v[i][p].w += u.w;
+            }
+        }
+    }
+    if (splits > 1) {
+        // four planes, one per component, so that a wave's dword stores are contiguous
+        constexpr int PL = TM * TN / 4;
+        float *my = part + (static_cast<size_t>(tile) * splits + split) * (TM * TN);
+#pragma unroll
+        for (int i = 0; i < WI; ++i)
+#pragma unroll
+            for (int p = 0; p < PT; ++p) {
+                const int q = threadIdx.x + p * NT;
+                if (!kAll && q >= Q) break;
+                float *d = my + i * Q + q;
+                st_dev(d, v[i][p].x); st_dev(d + PL, v[i][p].y); st_dev(d + 2 * PL, v[i][p].z); st_dev(d + 3 * PL, v[i][p].w);
+            }
+        if (!last_block_ticket(ctr(counters, tile), splits, &flag)) return;
+        const float *tp = part + static_cast<size_t>(tile) * splits * (TM * TN);
+#pragma unroll
+        for (int i = 0; i < WI; ++i)
+#pragma unroll
+            for (int p = 0; p < PT; ++p) {
+                const int q = threadIdx.x + p * NT;
+                if (!kAll && q >= Q) break;
+                v[i][p] = sum_splits(tp + i * Q + q, PL, splits, TM * TN);
+            }
+    }
+    // epilogue: a float4 of one row per thread, element by element at the edge
+    const float *pre_src = epi.sgd ? C : epi.gate;
+#pragma unroll
+    for (int i = 0; i < WI; ++i)
+#pragma unroll
+        for (int p = 0; p < PT; ++p) {
+            const int q = threadIdx.x + p * NT;
+            if (!kAll && q >= Q) break;
+            const int ml = q / (TN / 4);
+            const size_t row = m0 + (KCA ? 32 * i + ml : WI * ml + i), col = n0 + (q % (TN / 4)) * 4;
+            if (row >= M || col >= N) continue;
+            const size_t o = row * N + col;
+            const float u[4] = {v[i][p].x, v[i][p].y, v[i][p].z, v[i][p].w};
+            if (col + 4 <= N) {
+                float4 pre = make_float4(0.f, 0.f, 0.f, 0.f), bias = make_float4(0.f, 0.f, 0.f, 0.f);
+                if (pre_src) pre = ld4_any<false>(pre_src + o);
+                if (epi.bias) bias = ld4_any<false>(epi.bias + col);
+                *reinterpret_cast<f32x4u *>(C + o) =
+                    f32x4u{epi_value(epi, u[0], bias.x, pre.x), epi_value(epi, u[1], bias.y, pre.y),
+                           epi_value(epi, u[2], bias.z, pre.z), epi_value(epi, u[3], bias.w, pre.w)};
+            } else {
+#pragma unroll
+                for (int c = 0; c < 4; ++c)
+                    if (col + c < N)
+                        C[o + c] =
+                            epi_value(epi, u[c], epi.bias ? epi.bias[col + c] : 0.0f, pre_src ? pre_src[o + c] : 0.0f);
+            }
+        }
+}
+
+// Tiles and K splits of one product.
+struct DirectPlan {
+    size_t tiles, tiles_n, splits, kper;
+};
+DirectPlan direct_plan(size_t M, size_t N, size_t K, size_t tm, size_t tn, size_t nw, size_t target) {
+    DirectPlan p{};
+    p.tiles_n = (N + tn - 1) / tn;
+    p.tiles = (M + tm - 1) / tm * p.tiles_n;
+    const size_t step = 8 * nw;  // k of one block per wave
+    p.splits = 1;
+    if (p.tiles < target) {
+        p.splits = target / p.tiles;
+        const size_t most = K / (kDepth * step);  // at least a wave's pipeline depth each
+        if (p.splits > most) p.splits = most;
+        if (p.splits < 1) p.splits = 1;
+    }
+    p.kper = ((K + p.splits - 1) / p.splits + step - 1) / step * step;
+    p.splits = (K + p.kper - 1) / p.kper;
+    return p;
+}
+
+template <int WI, int WJ, int NW>
+int launch_direct(const float *A, const float *B, float *C, size_t M, size_t K, size_t N, int ta, int tb,
+                  const Epilogue &epi, size_t target, cxm_stream_t st) {
+    DirectPlan p = direct_plan(M, N, K, 32 * WI, 32 * WJ, NW, target);
+    float *part = nullptr;
+    unsigned *counters = nullptr;
+    if (p.splits > 1) {
+        Workspace ws;
+        if (get_workspace(st, p.tiles, p.tiles * p.splits * (32 * WI * 32 * WJ) * sizeof(float), &ws)) {
+            (void)hipGetLastError();  // no scratch to be had (a capturing stream's first call): K unsplit
+            p.splits = 1;
+            p.kper = K;
+        } else {
+            part = static_cast<float *>(ws.scratch);
+            counters = ws.counters;
+        }
+    }
+    const size_t wgs = p.tiles * p.splits;
+    if (wgs > 0x7fffffu) return 1;
+    const dim3 grid(static_cast<unsigned>(wgs)), block(NW * kWave);
+    const unsigned tn = static_cast<unsigned>(p.tiles_n), sp = static_cast<unsigned>(p.splits);
+    hipStream_t s = reinterpret_cast<hipStream_t>(st);
+    if (!ta && !tb)
+        hipLaunchKernelGGL((k_gemm_direct<WI, WJ, NW, true, false>), grid, block, 0, s, A, B, C, M, N, K, tn, sp, p.kper, epi,
+                           part, counters);
+    else if (!ta)
+        hipLaunchKernelGGL((k_gemm_direct<WI, WJ, NW, true, true>), grid, block, 0, s, A, B, C, M, N, K, tn, sp, p.kper, epi,
+                           part, counters);
+    else
+        hipLaunchKernelGGL((k_gemm_direct<WI, WJ, NW, false, false>), grid, block, 0, s, A, B, C, M, N, K, tn, sp, p.kper, epi,
+                           part, counters);
+    return launch_status();
+}
+
+// Whether the ring of gemm.hip, which takes this product, is the faster: its
+// 128x128 tiles times its K splits fill nine tenths of the chip's rounds and
+// are long enough for its fill and epilogue, or a long K is split over three
+// quarters of it.
+bool ring_fits(size_t M, size_t N, size_t K) {
+    const size_t tiles = ((M + 127) / 128) * ((N + 127) / 128), cus = device_cus();
+    size_t splits = 1;
+    if (tiles < cus * 3 / 4 && K >= 512) {  // gemm_ex's split
+        splits = cus / tiles < K / 256 ? cus / tiles : K / 256;
+        if (splits < 1) splits = 1;
+    }
+    const size_t kper = ((K + splits - 1) / splits + 127) / 128 * 128;
+    splits = (K + kper - 1) / kper;
+    const size_t rounds = (tiles * splits + cus - 1) / cus;
+    const double used = static_cast<double>(M) * N * K /
+                        (static_cast<double>(rounds * cus) * 128 * 128 * (splits > 1 ? kper : K));
+    return (used >= 0.9 && kper >= 512) || (used >= 0.76 && splits > 1 && K >= 2048);
+}
+
+}  // namespace
+
+// The tile by the product's size.  Measured (us; 32x32 / 32x64 / 64x64 tiles
+// with this K split / ring or, ragged, the register-staged kernels):
+//   40x784x256        4.9 /  7.2 /  12   /  35.8
+//   512x512x512       5.3 /  7.8 /  11   /  25.3
+//   333x2000x517     13.4 / 15.7 /  23   /  35.8
+//   640x1024x1024    20.3 / 22.5 /  24   /  28.6
+//   1000x1000x1000   26.0 / 22.6 /  24.6 /  42.7
+//   1536x1024x1024   39.4 / 32.9 /  40.2 /  42.2
+//   3000x700x1500    91.8 / 67.3 /  66.5 / 112.7
+//   4100x300x4095   150   / 122  / 111   / 173
+//   300x4100x4095 TN 131  / 129  / 122   / 175
+//   3072x1024x1024   75.7 / 62.1 /  57.4 /  68.2
+//   4096x1024x1024   98.6 / 81.2 /  74.9 /  70.1
+//   784x4096x1024 TN 102  / 82.5 /  82.9 /  73.9
+// Small grids want many small tiles; a 64x64 tile reads half as much per
+// flop, which counts once every CU has two; beyond K = 2048 its splits pay.
+int gemm_direct(const float *A, const float *B, float *C, size_t M, size_t K, size_t N, int ta, int tb,
+                const Epilogue &epi, bool ring, cxm_stream_t st) {
+    // 32-bit byte offsets within a tile; pairs of columns of a [K, M] / [K, N] operand
+    constexpr size_t kMaxLd = size_t(1) << 23;
+    if ((ta && tb) || M >= kMaxLd || N >= kMaxLd || K >= kMaxLd || (ta && M < 2) || (!tb && N < 2)) return 1;
+    if (ring && ring_fits(M, N, K)) return 1;
+    const size_t t64 = ((M + 63) / 64) * ((N + 63) / 64);
+    if (t64 < 200) return launch_direct<1, 1, 4>(A, B, C, M, K, N, ta, tb, epi, 256, st);
+    if (t64 < 600 && K < 2048) return launch_direct<1, 2, 4>(A, B, C, M, K, N, ta, tb, epi, 256, st);
+    return launch_direct<2, 2, 4>(A, B, C, M, K, N, ta, tb, epi, K < 2048 ? 1 : 768, st);
+}
+
+}  // namespace cxm

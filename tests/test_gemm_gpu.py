@@ -185,3 +185,40 @@ def test_thin_products(hip, orc, m, k, n, ta, tb):
         got_g = run(a, b, ta, tb, gate=gate)
         assert np.all(np.abs(got_g - ref * (gate > 0)) <= bound(a, b))
         assert np.all(got_g[gate <= 0] == 0)
+
+
+@pytest.mark.parametrize("m,k,n", [(1, 1, 2), (2, 1, 2), (2, 3, 3), (31, 7, 33), (32, 8, 32), (33, 9, 65), (65, 31, 31),
+                                   (64, 97, 64), (63, 200, 129), (17, 1003, 66), (3, 4099, 37), (517, 333, 1030),
+                                   (1021, 65, 1023), (1601, 131, 1543), (901, 2051, 1025)], ids=lambda v: str(v))
+@pytest.mark.parametrize("ta,tb", [(0, 0), (1, 0), (0, 1)])
+@pytest.mark.parametrize("off", [0, 1])
+def test_direct_products(hip, m, k, n, ta, tb, off):
+    """Products that no wide load fits: each tile of the direct kernels at its
+    edges, K below, at and past whole 8-k blocks and its splits, bases that
+    are only 4-byte aligned, and the epilogue's bias, ReLU and gate, against
+    float64.  A NaN in one row of A and one column of B stays in them."""
+    g = SplitMix64(0xD17 + 131 * m + 17 * k + n + 1000 * ta + 2000 * tb)
+    a, b, bias, gate = g.normal((m, k)), g.normal((k, n)), g.normal((n,)), g.normal((m, n))
+    da, db = dev(stored(a, ta), off), dev(stored(b, tb), off)
+    ref = a.astype(np.float64) @ b.astype(np.float64)
+    lim = bound(a, b) + 2e-7 * np.abs(bias)
+    guard = np.full(m * n + 9, 7.0, np.float32)
+    for kind in ("plain", "bias_relu", "gate"):
+        c = dev(guard, 4)
+        c.ptr += 4 * off
+        engine.gemm(da, db, c, m, k, n, ta, tb, bias=dev(bias) if kind == "bias_relu" else None,
+                    act=ACT_RELU if kind == "bias_relu" else ACT_NONE, gate=dev(gate, off) if kind == "gate" else None)
+        full = c.base.numpy()
+        got = full[4 + off:4 + off + m * n].reshape(m, n)
+        assert np.all(full[4:4 + off] == 7.0) and np.all(full[4 + off + m * n:] == 7.0)
+        want = np.maximum(ref + bias, 0.0) if kind == "bias_relu" else np.where(gate > 0, ref, 0.0) if kind == "gate" else ref
+        assert np.all(np.abs(got - want) <= lim)
+    a[m // 2, k - 1] = np.nan
+    b[0, n - 1] = np.inf
+    da, db, c = dev(stored(a, ta), off), dev(stored(b, tb), off), empty((m, n))
+    engine.gemm(da, db, c, m, k, n, ta, tb)
+    bad = ~np.isfinite(c.numpy())
+    want = np.zeros((m, n), bool)
+    want[m // 2, :] = True
+    want[:, n - 1] = True
+    assert np.array_equal(bad, want)
