@@ -42,7 +42,7 @@
 #include <atomic>
 
 #include "cxm_common.hpp"
-#include "half.hpp"
+#include "gemm16.hpp"
 
 namespace cxm {
 namespace {
@@ -50,21 +50,6 @@ namespace {
 constexpr int kH_BM = 128, kH_BN = 128, kH_BK = 64;
 constexpr int kH_KP = kH_BK + 8;  // LDS row stride in 16-bit elements
 constexpr int kHThreads = 256;
-
-typedef float f32x16 __attribute__((ext_vector_type(16)));
-typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
-typedef _Float16 f16x8 __attribute__((ext_vector_type(8)));
-typedef unsigned u32x2 __attribute__((ext_vector_type(2)));
-
-template <int DT>
-__device__ __forceinline__ f32x16 mfma16(u32x4 a, u32x4 b, f32x16 c) {
-    if constexpr (DT == CXM_DT_BF16)
-        return __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8, a), __builtin_bit_cast(bf16x8, b), c,
-                                                       0, 0, 0);
-    else
-        return __builtin_amdgcn_mfma_f32_32x32x16_f16(__builtin_bit_cast(f16x8, a), __builtin_bit_cast(f16x8, b), c, 0,
-                                                      0, 0);
-}
 
 __device__ __forceinline__ unsigned xcd_remap16(unsigned b, unsigned g) {
     if (g % 8 != 0) return b;
@@ -895,7 +880,7 @@ int dispatch16(const uint16_t *A, const uint16_t *B, uint16_t *C, size_t M, size
                                   static_cast<unsigned>(tn), s);
 }
 
-// Kernel choice, where the ring's conditions hold (M, N multiples of the
+// Kernel choice after gemm16_direct has had its pick; where the ring's conditions hold (M, N multiples of the
 // tile, K of 128, 16-byte aligned bases; A stored [K,M] is first transposed
 // into the stream's workspace, B is read as stored):
 //  * at least 128 tiles of 256x256: the 256 ring, else the 256x256
@@ -953,6 +938,10 @@ int gemm16(const uint16_t *A, const uint16_t *B, uint16_t *C, size_t M, size_t K
         kernel = pinned;
         if (kernel == 2 && !ring256) kernel = 1;
         if (kernel == 3 && !ring128) kernel = 0;
+    }
+    if (pinned < 0) {
+        const int t = gemm16_direct(A, B, C, M, K, N, ta, tb, DT, ring256 || ring128, va && vb, st);
+        if (t != 1) return t;
     }
     if (kernel == 2) return launch_ring<DT, 256>(A, B, C, M, N, K, ta, tb, st);
     if (kernel == 3) return launch_ring<DT, 128>(A, B, C, M, N, K, ta, tb, st);

@@ -109,26 +109,6 @@ struct Side {
 
 constexpr int kDepth = 3;  // 8-k blocks in flight per wave
 
-// The sum of a float4's split partials (components `plane` floats apart) in
-// split order, four splits of loads in flight.
-__device__ __forceinline__ float4 sum_splits(const float *p, int plane, unsigned splits, size_t stride) {
-    float4 a = make_float4(0.f, 0.f, 0.f, 0.f);
-    for (unsigned s0 = 0; s0 < splits; s0 += 4) {
-        float4 t[4];
-#pragma unroll
-        for (unsigned u = 0; u < 4; ++u) {
-            const float *d = p + static_cast<size_t>(s0 + u < splits ? s0 + u : splits - 1) * stride;
-            t[u] = make_float4(ld_dev(d), ld_dev(d + plane), ld_dev(d + 2 * plane), ld_dev(d + 3 * plane));
-        }
-#pragma unroll
-        for (unsigned u = 0; u < 4; ++u)
-            if (s0 + u < splits) {
-                a.x += t[u].x; a.y += t[u].y; a.z += t[u].z; a.w += t[u].w;
-            }
-    }
-    return a;
-}
-
 template <int WI, int WJ, int NW, bool KCA, bool KCB>
 __global__ __launch_bounds__(NW * kWave) void k_gemm_direct(const float *__restrict__ A, const float *__restrict__ B,
                                                             float *__restrict__ C, size_t M, size_t N, size_t K,
@@ -287,31 +267,10 @@ __global__ __launch_bounds__(NW * kWave) void k_gemm_direct(const float *__restr
         }
 }
 
-// Tiles and K splits of one product.
-struct DirectPlan {
-    size_t tiles, tiles_n, splits, kper;
-};
-DirectPlan direct_plan(size_t M, size_t N, size_t K, size_t tm, size_t tn, size_t nw, size_t target) {
-    DirectPlan p{};
-    p.tiles_n = (N + tn - 1) / tn;
-    p.tiles = (M + tm - 1) / tm * p.tiles_n;
-    const size_t step = 8 * nw;  // k of one block per wave
-    p.splits = 1;
-    if (p.tiles < target) {
-        p.splits = target / p.tiles;
-        const size_t most = K / (kDepth * step);  // at least a wave's pipeline depth each
-        if (p.splits > most) p.splits = most;
-        if (p.splits < 1) p.splits = 1;
-    }
-    p.kper = ((K + p.splits - 1) / p.splits + step - 1) / step * step;
-    p.splits = (K + p.kper - 1) / p.kper;
-    return p;
-}
-
 template <int WI, int WJ, int NW>
 int launch_direct(const float *A, const float *B, float *C, size_t M, size_t K, size_t N, int ta, int tb,
                   const Epilogue &epi, size_t target, cxm_stream_t st) {
-    DirectPlan p = direct_plan(M, N, K, 32 * WI, 32 * WJ, NW, target);
+    DirectPlan p = direct_plan(M, N, K, 32 * WI, 32 * WJ, 8 * NW, kDepth, target);
     float *part = nullptr;
     unsigned *counters = nullptr;
     if (p.splits > 1) {

@@ -188,3 +188,34 @@ def test_kernel_choice_argument(hip):
     assert lib().cxm_gemm16_kernel(4) == E_INVALID
     assert lib().cxm_gemm16_kernel(-2) == E_INVALID
     assert lib().cxm_gemm16_kernel(-1) == 0
+
+
+@pytest.mark.parametrize("shape", [(1, 1, 2), (2, 5, 3), (31, 15, 33), (33, 17, 65), (64, 16, 31), (63, 161, 130),
+                                   (3, 2077, 37), (515, 333, 1030), (250, 1033, 699), (1025, 70, 1023), (901, 2051, 517)],
+                         ids=lambda s: "x".join(map(str, s)))
+@pytest.mark.parametrize("ta,tb", [(0, 0), (0, 1), (1, 0)])
+@pytest.mark.parametrize("dt", [DT_BF16, DT_F16])
+def test_direct_products(hip, orc, shape, ta, tb, dt):
+    """Ragged and small products on the direct kernels: tiles at their edges,
+    K below, at and past whole 16-k blocks and its splits, 2-byte aligned
+    bases, outputs within their buffer; a NaN of A stays in its row."""
+    m, k, n = shape
+    g = SplitMix64(0xD16 + 131 * m + 17 * k + n + 1000 * ta + 2000 * tb + dt)
+    a, a64 = rand16(g, (m, k), dt, orc)
+    b, b64 = rand16(g, (k, n), dt, orc)
+
+    def product(a, off):
+        da, db = dev(np.ascontiguousarray(a.T) if ta else a, off), dev(np.ascontiguousarray(b.T) if tb else b, off)
+        c = dev(np.full(m * n + 9, 0x1234, np.uint16), 4 + off)
+        call("cxm_gemm_t", da.ptr, db.ptr, c.ptr, m, k, n, ta, tb, dt, None)
+        full = c.base.numpy()
+        s = 4 + off
+        assert np.all(full[s + m * n:] == 0x1234)
+        return full[s:s + m * n].reshape(m, n)
+
+    for off in (0, 1):
+        check(product(a, off), a64, b64, dt, orc)
+    a = a.copy()
+    a[m // 2, k - 1] = 0x7fff  # NaN in either type
+    got = orc.convert(product(a, 0).ravel(), dt, DT_F32).reshape(m, n)
+    assert np.all(np.isnan(got[m // 2])) and not np.any(np.isnan(np.delete(got, m // 2, axis=0)))
