@@ -15,6 +15,8 @@
 // library is built with -ffp-contract=off, so x*s+b is a rounded product
 // followed by a rounded sum, never an fma.  ReLU is an explicit select
 // (0 > t ? 0 : t), matching _mm256_max_ps(0, t) for -0.0 and NaN.
+#include <type_traits>
+
 #include "cxm_common.hpp"
 #include "ops.hpp"
 
@@ -106,11 +108,97 @@ template <int ACT>
 struct ActF {
     __device__ float operator()(float t) const { return act<ACT>(t); }
 };
+// ---------------------------------------------------- flat row maps
+//
+// Row-structured maps over rows that are no multiple of four floats, or too
+// short for k_rowmap4's 256-column tiles: the matrix is read as one run of
+// aligned float4s, and a float4's row and column come from its index by a
+// multiplication with the row length's precomputed reciprocal.  A float4 that
+// runs past its row's end takes the next row's operands for the rest (rows
+// are at least four floats long, so there is one such end at most).
+// Measured: row broadcast over [3001, 1003] 6.9 -> 5.6 us (a 64-bit division and
+// dword accesses per element before), [2396, 55] 4.2 -> 3.9 us (a launch).
+
+// Division of 32-bit numbers by an invariant d >= 1: Granlund and Montgomery,
+// "Division by invariant integers using multiplication" (1994), figure 4.1.
+struct FastDiv {
+    unsigned mul, sh1, sh2;
+    __device__ unsigned operator()(unsigned e) const {
+        const unsigned t = __umulhi(mul, e);
+        return (t + ((e - t) >> sh1)) >> sh2;
+    }
+};
+inline FastDiv fast_div(unsigned d) {
+    unsigned l = 0;
+    while (l < 32 && (1ull << l) < d) ++l;
+    const unsigned long long m = ((1ull << 32) * ((1ull << l) - d)) / d + 1;
+    return FastDiv{static_cast<unsigned>(m), l < 1 ? l : 1u, l < 1 ? 0u : l - 1};
+}
+
+// y[c .. c+3] of an n-float row, wrapping to y[0 ..] past its end (c < n, n >= 4).
+__device__ __forceinline__ float4 wrap4(const float *__restrict__ y, unsigned c, unsigned n) {
+    const unsigned off = c < n - 4 ? c : n - 4, d = c - off;
+    const float4 v = ld4_any<false>(y + off), h = ld4_any<false>(y);
+    float4 o;
+    o.x = d == 0 ? v.x : d == 1 ? v.y : d == 2 ? v.z : v.w;
+    o.y = d == 0 ? v.y : d == 1 ? v.z : d == 2 ? v.w : h.x;
+    o.z = d == 0 ? v.z : d == 1 ? v.w : d == 2 ? h.x : h.y;
+    o.w = d == 0 ? v.w : d == 1 ? h.x : d == 2 ? h.y : h.z;
+    return o;
+}
+
+// f.flat(v, r, c, m, n): the output float4 for the elements at (r, c ..),
+// f.one(v, r, c): one element.
+template <class F, bool AL>
+__global__ __launch_bounds__(kBlock) void k_flatmap4(F f, const float *x, float *z, unsigned total, unsigned m,
+                                                     unsigned n, FastDiv by_n) {
+    const size_t i = stream_vec();
+    const unsigned n4 = total / 4;
+    if (i < n4) {
+        const unsigned e = 4 * static_cast<unsigned>(i), r = by_n(e);
+        st4_any_stream<AL>(z + e, f.flat(ld4_any_stream<AL>(x + e), r, e - r * n, m, n));
+    } else if (i == n4) {
+        for (unsigned j = 4 * n4; j < total; ++j) {
+            const unsigned r = by_n(j);
+            z[j] = f.one(x[j], r, j - r * n);
+        }
+    }
+}
+
+// Whether the flat map takes an [m, n] row map: 32-bit element numbers, and
+// rows that k_rowmap4 does not take (`rows4`: n a multiple of 4, everything
+// 16-byte aligned) or leaves more than a fifth of its lanes idle on.
+// Measured at [m, n], flat / row tiles (us): affine forward [60000, 32] 4.7 /
+// 14.2, [3000, 520] 4.3 / 5.2, [4096, 320] 4.1 / 4.3, [7000, 480] 6.7 / 6.6,
+// [8192, 8192] 87.5 / 82.5 (its operands cross from L2 once per wave).
+inline bool use_flatmap(size_t m, size_t n, bool rows4) {
+    if (n < 4 || m > 0xfffffc00u / n) return false;
+    const size_t n4 = n / 4, lanes = (n4 + kWave - 1) / kWave * kWave;
+    return !rows4 || n4 * 5 < lanes * 4;
+}
+
+template <class F>
+int run_flatmap(const F &f, const float *x, float *z, size_t m, size_t n, hipStream_t s) {
+    const unsigned total = static_cast<unsigned>(m * n), g = map4_grid(total);
+    const FastDiv d = fast_div(static_cast<unsigned>(n));
+    if (aligned16(x) && aligned16(z))
+        hipLaunchKernelGGL((k_flatmap4<F, true>), dim3(g), dim3(kBlock), 0, s, f, x, z, total, static_cast<unsigned>(m),
+                           static_cast<unsigned>(n), d);
+    else
+        hipLaunchKernelGGL((k_flatmap4<F, false>), dim3(g), dim3(kBlock), 0, s, f, x, z, total, static_cast<unsigned>(m),
+                           static_cast<unsigned>(n), d);
+    return launch_status();
+}
+
 // z[i,j] = x[i,j] op y[j]
 template <int OP>
 struct RowBcastF {
     const float *y;
     __device__ float4 operator()(float4 v, unsigned, size_t j4) const { return bin4<OP>(v, ld4(y + 4 * j4)); }
+    __device__ float4 flat(float4 v, unsigned, unsigned c, unsigned, unsigned n) const {
+        return bin4<OP>(v, wrap4(y, c, n));
+    }
+    __device__ float one(float v, unsigned, unsigned c) const { return bin_t<OP>(v, y[c]); }
 };
 // z[i,j] = x[i,j] op y[i]
 template <int OP>
@@ -120,13 +208,28 @@ struct ColBcastF {
         const float c = y[row];
         return bin4<OP>(v, make_float4(c, c, c, c));
     }
+    __device__ float4 flat(float4 v, unsigned r, unsigned c, unsigned m, unsigned n) const {
+        const float a = y[r], b = y[r + 1 < m ? r + 1 : r];
+        return bin4<OP>(v, make_float4(a, c + 1 < n ? a : b, c + 2 < n ? a : b, c + 3 < n ? a : b));
+    }
+    __device__ float one(float v, unsigned r, unsigned) const { return bin_t<OP>(v, y[r]); }
 };
 // y = act(x*scale[j] + bias[j]): product and sum rounded separately
 template <int ACT>
 struct AffineF {
     const float *scale, *bias;
     __device__ float4 operator()(float4 v, unsigned, size_t j4) const {
-        const float4 sc = ld4(scale + 4 * j4), b = ld4(bias + 4 * j4);
+        return apply(v, ld4(scale + 4 * j4), ld4(bias + 4 * j4));
+    }
+    __device__ float4 flat(float4 v, unsigned, unsigned c, unsigned, unsigned n) const {
+        return apply(v, wrap4(scale, c, n), wrap4(bias, c, n));
+    }
+    __device__ float one(float v, unsigned, unsigned c) const {
+        float t = v * scale[c];
+        t = t + bias[c];
+        return act<ACT>(t);
+    }
+    __device__ static float4 apply(float4 v, float4 sc, float4 b) {
         float4 t;
         t.x = v.x * sc.x; t.y = v.y * sc.y; t.z = v.z * sc.z; t.w = v.w * sc.w;
         t.x = t.x + b.x; t.y = t.y + b.y; t.z = t.z + b.z; t.w = t.w + b.w;
@@ -165,145 +268,194 @@ __global__ __launch_bounds__(kBlock) void k_affine_fwd_scalar(const float *x, co
 
 // ----------------------------------------------------- affine backward
 
-// dz = dy*act'(y); dx = dz*scale[j]; dscale[j] = sum_i dz*x; dbias[j] = sum_i dz.
-// Workgroup = 256 columns (64 lanes x float4) x a chunk of rows; its NW
-// waves take interleaved rows and meet in LDS; chunks are combined in
-// chunk order by the last workgroup of the column tile.  With tile_major
-// the chunks of a tile are adjacent in launch order, so early tiles'
-// combines overlap later tiles' streaming.
-constexpr int kAffTile = 256;
+constexpr unsigned kAffGroups = 32;  // groups of chunks of one tile (512 chunks at most)
 
-template <int ACT, bool VEC, int UNR, int NW>
-__global__ __launch_bounds__(NW * kWave) void k_affine_bwd(const float *__restrict__ x,
-                                                           const float *__restrict__ scale,
-                                                           const float *__restrict__ y,
-                                                           const float *__restrict__ dy,
-                                                           float *__restrict__ dx,
-                                                           float *__restrict__ dscale,
-                                                           float *__restrict__ dbias, size_t m, size_t n,
-                                                           unsigned ntiles, unsigned chunks,
-                                                           size_t rows_per_chunk, int tile_major,
-                                                           float *__restrict__ part,
-                                                           unsigned *__restrict__ counters) {
-    constexpr int NSLOT = VEC ? NW : NW / 4;
-    __shared__ float lds_s[NSLOT][kAffTile];
-    __shared__ float lds_b[NSLOT][kAffTile];
+// dz = dy*act'(y); dx = dz*scale[j]; dscale[j] = sum_i dz*x; dbias[j] = sum_i dz.
+// A 256-thread workgroup takes a tile of 4 G columns (G lanes x float4) and a
+// chunk of rows; its 256 / G lane groups take interleaved rows, UNR of them
+// in flight, and meet in LDS.  The chunks of a tile are adjacent in launch
+// order, so early tiles' combines overlap later tiles' streaming; the last
+// workgroup of a tile combines them in chunk order, beyond 32 chunks in two
+// levels (groups of kPartGroup).  AL: 16-byte aligned rows (G = 64 only);
+// otherwise dword-aligned accesses, the last lane of a row reading its last
+// four columns and keeping its own (n >= 4).  [6848, 83] backward 43 -> 7.9 us
+// (dword accesses, and one workgroup summing 428 partials, before);
+// [8192, 256] 50 -> 13.5 us.
+constexpr int kAffTile = 256;  // stride of a tile's partials
+
+template <int ACT, bool AL, int G, int UNR>
+__global__ __launch_bounds__(kBlock) void k_affine_bwd(const float *__restrict__ x, const float *__restrict__ scale,
+                                                       const float *__restrict__ y, const float *__restrict__ dy,
+                                                       float *__restrict__ dx, float *__restrict__ dscale,
+                                                       float *__restrict__ dbias, size_t m, size_t n, unsigned chunks,
+                                                       size_t rows_per_chunk, float *__restrict__ part,
+                                                       float *__restrict__ tops, unsigned *__restrict__ counters) {
+    constexpr int NS = kBlock / G, TW = 4 * G;
+    __shared__ float lds_s[NS][TW];
+    __shared__ float lds_b[NS][TW];
     __shared__ int flag;
-    unsigned tile, chunk;
-    if (tile_major) {
-        chunk = blockIdx.x % chunks;
-        tile = blockIdx.x / chunks;
-    } else {
-        tile = blockIdx.x % ntiles;
-        chunk = blockIdx.x / ntiles;
-    }
-    const int tid = threadIdx.x;
+    const unsigned tile = blockIdx.x / chunks, chunk = blockIdx.x - tile * chunks;
+    const int tid = threadIdx.x, lane = tid % G, g = tid / G;
     const size_t r0 = static_cast<size_t>(chunk) * rows_per_chunk;
     const size_t r1 = r0 + rows_per_chunk < m ? r0 + rows_per_chunk : m;
-
-    if constexpr (VEC) {
-        const int lane = tid & (kWave - 1);
-        const int w = tid / kWave;
-        const size_t col = static_cast<size_t>(tile) * kAffTile + lane * 4;
-        float as[4] = {0, 0, 0, 0}, ab[4] = {0, 0, 0, 0};
-        if (col < n) {
-            const float4 sc = ld4(scale + col);
-            size_t r = r0 + w;
-            auto body = [&](size_t rr, float4 xv, float4 yv, float4 gv) {
-                float4 dz;
-                dz.x = gv.x * dact<ACT>(yv.x); dz.y = gv.y * dact<ACT>(yv.y);
-                dz.z = gv.z * dact<ACT>(yv.z); dz.w = gv.w * dact<ACT>(yv.w);
-                float4 d;
-                d.x = dz.x * sc.x; d.y = dz.y * sc.y; d.z = dz.z * sc.z; d.w = dz.w * sc.w;
-                st4_stream(dx + rr * n + col, d);
-                const float p0 = dz.x * xv.x, p1 = dz.y * xv.y, p2 = dz.z * xv.z, p3 = dz.w * xv.w;
-                as[0] = as[0] + p0; as[1] = as[1] + p1; as[2] = as[2] + p2; as[3] = as[3] + p3;
-                ab[0] = ab[0] + dz.x; ab[1] = ab[1] + dz.y; ab[2] = ab[2] + dz.z; ab[3] = ab[3] + dz.w;
-            };
-            for (; r + (UNR - 1) * NW < r1; r += UNR * NW) {
-                float4 xv[UNR], yv[UNR], gv[UNR];
-#pragma unroll
-                for (int u = 0; u < UNR; ++u) {
-                    const size_t o = (r + u * NW) * n + col;
-                    xv[u] = ld4_stream(x + o);
-                    yv[u] = ld4_stream(y + o);
-                    gv[u] = ld4_stream(dy + o);
-                }
-#pragma unroll
-                for (int u = 0; u < UNR; ++u) body(r + u * NW, xv[u], yv[u], gv[u]);
+    const size_t col = static_cast<size_t>(tile) * TW + lane * 4;
+    const size_t pos = AL || col + 4 <= n ? col : n - 4;
+    const int d = col < n ? static_cast<int>(col - pos) : 4;  // columns pos .. pos + d - 1 are another lane's
+    float as[4] = {0, 0, 0, 0}, ab[4] = {0, 0, 0, 0};
+    if (d < 4) {
+        const float4 sc = ld4_any<AL>(scale + pos);
+        size_t r = r0 + g;
+        auto body = [&](size_t rr, float4 xv, float4 yv, float4 gv) {
+            float4 dz;
+            dz.x = gv.x * dact<ACT>(yv.x); dz.y = gv.y * dact<ACT>(yv.y);
+            dz.z = gv.z * dact<ACT>(yv.z); dz.w = gv.w * dact<ACT>(yv.w);
+            float4 o;
+            o.x = dz.x * sc.x; o.y = dz.y * sc.y; o.z = dz.z * sc.z; o.w = dz.w * sc.w;
+            float *p = dx + rr * n + pos;
+            if (AL || d == 0) {
+                st4_any_stream<AL>(p, o);
+            } else {
+                if (d <= 1) p[1] = o.y;
+                if (d <= 2) p[2] = o.z;
+                p[3] = o.w;
             }
-            for (; r < r1; r += NW) {
-                const size_t o = r * n + col;
-                body(r, ld4_stream(x + o), ld4_stream(y + o), ld4_stream(dy + o));
-            }
-        }
+            const float p0 = dz.x * xv.x, p1 = dz.y * xv.y, p2 = dz.z * xv.z, p3 = dz.w * xv.w;
+            as[0] = as[0] + p0; as[1] = as[1] + p1; as[2] = as[2] + p2; as[3] = as[3] + p3;
+            ab[0] = ab[0] + dz.x; ab[1] = ab[1] + dz.y; ab[2] = ab[2] + dz.z; ab[3] = ab[3] + dz.w;
+        };
+        for (; r < r1; r += UNR * NS) {
+            float4 xv[UNR], yv[UNR], gv[UNR];
 #pragma unroll
-        for (int c = 0; c < 4; ++c) {
-            lds_s[w][lane * 4 + c] = as[c];
-            lds_b[w][lane * 4 + c] = ab[c];
-        }
-    } else {
-        const int c = tid % kAffTile, ph = tid / kAffTile;
-        const size_t col = static_cast<size_t>(tile) * kAffTile + c;
-        float ms = 0.0f, mb = 0.0f;
-        if (col < n) {
-            const float sc = scale[col];
-            for (size_t r = r0 + ph; r < r1; r += NSLOT) {
-                const size_t o = r * n + col;
-                const float dz = dy[o] * dact<ACT>(y[o]);
-                dx[o] = dz * sc;
-                const float p = dz * x[o];
-                ms = ms + p;
-                mb = mb + dz;
+            for (int u = 0; u < UNR; ++u) {  // rows past the chunk's end re-read its last one
+                const size_t o = (UNR == 1 || r + u * NS < r1 ? r + u * NS : r1 - 1) * n + pos;
+                xv[u] = ld4_any_stream<AL>(x + o);
+                yv[u] = ld4_any_stream<AL>(y + o);
+                gv[u] = ld4_any_stream<AL>(dy + o);
             }
+            if constexpr (UNR > 1) __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+            for (int u = 0; u < UNR; ++u)
+                if (UNR == 1 || r + u * NS < r1) body(r + u * NS, xv[u], yv[u], gv[u]);
         }
-        lds_s[ph][c] = ms;
-        lds_b[ph][c] = mb;
+    }
+#pragma unroll
+    for (int c = 0; c < 4; ++c) {
+        if (d < 4 && c >= d) {
+            lds_s[g][lane * 4 + c - d] = as[c];
+            lds_b[g][lane * 4 + c - d] = ab[c];
+        }
     }
     __syncthreads();
-    const bool owner = tid < kAffTile;  // threads 0..255 own one column each from here
+    const size_t oc = static_cast<size_t>(tile) * TW + tid;
+    const bool put = tid < TW && oc < n;  // these threads own one column each from here
     float ms = 0.0f, mb = 0.0f;
-    if (owner) {
+    if (put) {
 #pragma unroll
-        for (int k = 0; k < NSLOT; ++k) {  // slots in order
+        for (int k = 0; k < NS; ++k) {  // groups in order
             ms = ms + lds_s[k][tid];
             mb = mb + lds_b[k][tid];
         }
     }
-    const size_t col = static_cast<size_t>(tile) * kAffTile + tid;
     if (chunks == 1) {
-        if (owner && col < n) {
-            dscale[col] = ms;
-            dbias[col] = mb;
+        if (put) {
+            dscale[oc] = ms;
+            dbias[oc] = mb;
         }
         return;
     }
-    const size_t slot = static_cast<size_t>(tile) * chunks;
-    if (owner) {
-        st_dev(&part[((slot + chunk) * 2 + 0) * kAffTile + tid], ms);
-        st_dev(&part[((slot + chunk) * 2 + 1) * kAffTile + tid], mb);
-    }
-    if (!last_block_ticket(ctr(counters, tile), chunks, &flag)) return;
-    if (owner) {
-        // both sums' loads go out together, 8 chunks at a time
-        float a = 0.0f, bsum = 0.0f;
-        for (unsigned c0 = 0; c0 < chunks; c0 += 8) {
+    // the sum of `count` pairs of partials, eight at a time in flight
+    auto sum = [&](const float *p, unsigned count) {
+        ms = 0.0f;
+        mb = 0.0f;
+        for (unsigned c0 = 0; c0 < count; c0 += 8) {
             float va[8], vb[8];
 #pragma unroll
             for (unsigned u = 0; u < 8; ++u) {
-                const bool in = c0 + u < chunks;
-                va[u] = in ? ld_dev(&part[((slot + c0 + u) * 2 + 0) * kAffTile + tid]) : 0.0f;
-                vb[u] = in ? ld_dev(&part[((slot + c0 + u) * 2 + 1) * kAffTile + tid]) : 0.0f;
+                const bool in = c0 + u < count;
+                va[u] = in ? ld_dev(&p[((c0 + u) * 2 + 0) * kAffTile + tid]) : 0.0f;
+                vb[u] = in ? ld_dev(&p[((c0 + u) * 2 + 1) * kAffTile + tid]) : 0.0f;
             }
 #pragma unroll
             for (unsigned u = 0; u < 8; ++u) {
-                a = a + va[u];
-                bsum = bsum + vb[u];
+                ms = ms + va[u];
+                mb = mb + vb[u];
             }
         }
-        if (col < n) {
-            dscale[col] = a;
-            dbias[col] = bsum;
+    };
+    float *pt = part + static_cast<size_t>(tile) * chunks * 2 * kAffTile;
+    if (put) {
+        st_dev(&pt[(static_cast<size_t>(chunk) * 2 + 0) * kAffTile + tid], ms);
+        st_dev(&pt[(static_cast<size_t>(chunk) * 2 + 1) * kAffTile + tid], mb);
+    }
+    if (chunks <= 2 * kPartGroup) {
+        if (!last_block_ticket(ctr(counters, tile), chunks, &flag)) return;
+        if (put) sum(pt, chunks);
+    } else {
+        const unsigned groups = (chunks + kPartGroup - 1) / kPartGroup, q = chunk / kPartGroup;
+        const unsigned size = (q + 1) * kPartGroup <= chunks ? kPartGroup : chunks - q * kPartGroup;
+        unsigned *cg = ctr(counters, static_cast<size_t>(tile) * (kAffGroups + 1));
+        float *tp = tops + static_cast<size_t>(tile) * kAffGroups * 2 * kAffTile;
+        if (!last_block_ticket(ctr(cg, q), size, &flag)) return;
+        if (put) {
+            sum(pt + static_cast<size_t>(q) * kPartGroup * 2 * kAffTile, size);
+            st_dev(&tp[(q * 2 + 0) * kAffTile + tid], ms);
+            st_dev(&tp[(q * 2 + 1) * kAffTile + tid], mb);
+        }
+        if (!last_block_ticket(ctr(cg, kAffGroups), groups, &flag)) return;
+        if (put) sum(tp, groups);
+    }
+    if (put) {
+        dscale[oc] = ms;
+        dbias[oc] = mb;
+    }
+}
+
+// Rows of fewer than four floats: thread t of a chunk's workgroup takes
+// column t % n of every 256 / n-th row; the last workgroup adds the at most
+// 256 chunks' partials, a chunk per thread.
+template <int ACT>
+__global__ __launch_bounds__(kBlock) void k_affine_bwd_few(const float *__restrict__ x, const float *__restrict__ scale,
+                                                           const float *__restrict__ y, const float *__restrict__ dy,
+                                                           float *__restrict__ dx, float *__restrict__ dscale,
+                                                           float *__restrict__ dbias, size_t m, unsigned n,
+                                                           unsigned chunks, size_t rows_per_chunk,
+                                                           float *__restrict__ part, unsigned *__restrict__ counters) {
+    __shared__ float lds[kWavesPerBlock];
+    __shared__ int flag;
+    const unsigned rows = kBlock / n, c = threadIdx.x % n, g = threadIdx.x / n;
+    const size_t r0 = blockIdx.x * rows_per_chunk, r1 = r0 + rows_per_chunk < m ? r0 + rows_per_chunk : m;
+    float ms = 0.0f, mb = 0.0f;
+    if (g < rows) {
+        const float sc = scale[c];
+        for (size_t r = r0 + g; r < r1; r += rows) {
+            const size_t o = r * n + c;
+            const float dz = dy[o] * dact<ACT>(y[o]);
+            const float p = dz * x[o];
+            dx[o] = dz * sc;
+            ms = ms + p;
+            mb = mb + dz;
+        }
+    }
+    for (unsigned j = 0; j < n; ++j) {
+        const float s = block_reduce<SumOp, kBlock>(c == j && g < rows ? ms : 0.0f, lds);
+        const float b = block_reduce<SumOp, kBlock>(c == j && g < rows ? mb : 0.0f, lds);
+        if (threadIdx.x != 0) continue;
+        if (chunks == 1) {
+            dscale[j] = s;
+            dbias[j] = b;
+        } else {
+            st_dev(&part[(j * 2 + 0) * kBlock + blockIdx.x], s);
+            st_dev(&part[(j * 2 + 1) * kBlock + blockIdx.x], b);
+        }
+    }
+    if (chunks == 1 || !last_block_ticket2<kAffGroups>(counters, chunks, blockIdx.x, &flag)) return;
+    for (unsigned j = 0; j < n; ++j) {
+        const bool in = threadIdx.x < chunks;
+        const float s = block_reduce<SumOp, kBlock>(in ? ld_dev(&part[(j * 2 + 0) * kBlock + threadIdx.x]) : 0.0f, lds);
+        const float b = block_reduce<SumOp, kBlock>(in ? ld_dev(&part[(j * 2 + 1) * kBlock + threadIdx.x]) : 0.0f, lds);
+        if (threadIdx.x == 0) {
+            dscale[j] = s;
+            dbias[j] = b;
         }
     }
 }
@@ -384,12 +536,21 @@ struct BcastL {
     }
 };
 
+template <int OP>
+struct BcastFlatL {
+    static int run(const float *x, const float *y, float *z, size_t m, size_t n, int row_mode, hipStream_t s) {
+        if (row_mode) return run_flatmap(RowBcastF<OP>{y}, x, z, m, n, s);
+        return run_flatmap(ColBcastF<OP>{y}, x, z, m, n, s);
+    }
+};
+
 int bcast(const float *x, const float *y, float *z, size_t m, size_t n, int op, int row_mode,
           cxm_stream_t s) {
     if (!x || !y || !z || op < CXM_OP_ADD || op > CXM_OP_DIV) return CXM_E_INVALID;
     if (m == 0 || n == 0) return CXM_OK;
-    if (n % 4 == 0 && aligned16(x) && aligned16(z) && (!row_mode || aligned16(y)))
-        return dispatch_op<BcastL>(op, x, y, z, m, n, row_mode, hs(s));
+    const bool rows4 = n % 4 == 0 && aligned16(x) && aligned16(z) && (!row_mode || aligned16(y));
+    if (use_flatmap(m, n, rows4)) return dispatch_op<BcastFlatL>(op, x, y, z, m, n, row_mode, hs(s));
+    if (rows4) return dispatch_op<BcastL>(op, x, y, z, m, n, row_mode, hs(s));
     hipLaunchKernelGGL(k_bcast_scalar, dim3(stream_grid((m * n + 3) / 4)), dim3(kBlock), 0, hs(s), x,
                        y, z, m, n, op, row_mode);
     return launch_status();
@@ -411,8 +572,9 @@ template <int ACT>
 int affine_fwd_t(const float *x, const float *scale, const float *bias, float *y, size_t m,
                  size_t n, hipStream_t s) {
     unsigned grid, tpr;
-    if (n % 4 == 0 && aligned16(x) && aligned16(scale) && aligned16(bias) && aligned16(y) &&
-        rowmap4_grid(m, n / 4, &grid, &tpr)) {
+    const bool rows4 = n % 4 == 0 && aligned16(x) && aligned16(scale) && aligned16(bias) && aligned16(y);
+    if (use_flatmap(m, n, rows4)) return run_flatmap(AffineF<ACT>{scale, bias}, x, y, m, n, s);
+    if (rows4 && rowmap4_grid(m, n / 4, &grid, &tpr)) {
         hipLaunchKernelGGL(k_rowmap4<AffineF<ACT>>, dim3(grid), dim3(kBlock), 0, s, AffineF<ACT>{scale, bias},
                            x, y, m, n / 4, tpr);
     } else {
@@ -430,51 +592,75 @@ int affine_fwd_t(const float *x, const float *scale, const float *bias, float *y
 // rows of loads per wave, with or without a scheduling barrier that keeps
 // them together), 2048 shorter workgroups, 384 workgroups (CUs unevenly
 // loaded) and 16-wave workgroups were all slower, by 5-25%.
-struct AffBwdPlan {
-    size_t chunks;   // 0: enough for about 512 workgroups
-    int tile_major;  // chunks of one tile adjacent in launch order
-};
+// Few rows per lane group (at most kAffFew) have several rows of loads in
+// flight where rows are narrow (four: [20000, 16] 8.7 -> 7.7 us, [8000, 96] 9.3
+// -> 7.9) or ragged (two: [3001, 1003] 16.0 -> 15.0): there the serial round
+// trips count.  Wide aligned rows keep one ([4000, 1000] 16.9 us with one,
+// 18.3 with four).
+constexpr size_t kAffFew = 16;
 
-template <int ACT>
-int affine_bwd_plan(const float *x, const float *scale, const float *y, const float *dy, float *dx,
-                    float *dscale, float *dbias, size_t m, size_t n, AffBwdPlan plan, cxm_stream_t st) {
-    const bool vec = n % 4 == 0 && aligned16(x) && aligned16(scale) && aligned16(y) &&
-                     aligned16(dy) && aligned16(dx);
-    const size_t ntiles = (n + kAffTile - 1) / kAffTile;
-    size_t chunks = plan.chunks;
-    if (chunks == 0) chunks = (512 + ntiles - 1) / ntiles;
-    const size_t max_chunks = (m + 15) / 16;
+template <int ACT, bool AL, int G>
+int affine_bwd_launch(const float *x, const float *scale, const float *y, const float *dy, float *dx, float *dscale,
+                      float *dbias, size_t m, size_t n, cxm_stream_t st) {
+    constexpr size_t NS = kBlock / G, TW = 4 * G;
+    const size_t ntiles = (n + TW - 1) / TW;
+    size_t chunks = 512 / ntiles;  // one more workgroup than 512 would be a round of its own
+    const size_t max_chunks = (m + 4 * NS - 1) / (4 * NS);  // at least four rows per lane group
     if (chunks > max_chunks) chunks = max_chunks;
     if (chunks < 1) chunks = 1;
     size_t rpc = (m + chunks - 1) / chunks;
-    rpc = (rpc + 15) / 16 * 16;
+    rpc = (rpc + NS - 1) / NS * NS;
     chunks = (m + rpc - 1) / rpc;
-    if (chunks < 1) chunks = 1;
     if (ntiles * chunks > 0x7fffffffu) return CXM_E_TOO_LARGE;
-    float *part = nullptr;
+    float *part = nullptr, *tops = nullptr;
     unsigned *counters = nullptr;
     if (chunks > 1) {
         Workspace ws;
-        int rc = get_workspace(st, ntiles, ntiles * chunks * 2 * kAffTile * sizeof(float), &ws);
+        const bool two = chunks > 2 * kPartGroup;
+        int rc = get_workspace(st, two ? ntiles * (kAffGroups + 1) : ntiles,
+                               ntiles * (chunks + (two ? kAffGroups : 0)) * 2 * kAffTile * sizeof(float), &ws);
         if (rc) return rc;
         part = static_cast<float *>(ws.scratch);
+        tops = part + ntiles * chunks * 2 * kAffTile;
         counters = ws.counters;
     }
     const dim3 grid(static_cast<unsigned>(ntiles * chunks));
-    const unsigned nt = static_cast<unsigned>(ntiles), nc = static_cast<unsigned>(chunks);
-#define CXM_AFFB(VEC_)                                                                                  \
-    hipLaunchKernelGGL((k_affine_bwd<ACT, VEC_, 1, 4>), grid, dim3(4 * kWave), 0, hs(st), x, scale, y, dy, dx,    \
-                       dscale, dbias, m, n, nt, nc, rpc, plan.tile_major, part, counters)
-    if (vec) CXM_AFFB(true);
-    else CXM_AFFB(false);
-#undef CXM_AFFB
+    const unsigned nc = static_cast<unsigned>(chunks);
+    constexpr int kUnr = G < kWave ? 4 : AL ? 1 : 2;
+    if (kUnr > 1 && rpc <= kAffFew * NS)
+        hipLaunchKernelGGL((k_affine_bwd<ACT, AL, G, kUnr>), grid, dim3(kBlock), 0, hs(st), x, scale, y, dy, dx, dscale,
+                           dbias, m, n, nc, rpc, part, tops, counters);
+    else
+        hipLaunchKernelGGL((k_affine_bwd<ACT, AL, G, 1>), grid, dim3(kBlock), 0, hs(st), x, scale, y, dy, dx, dscale,
+                           dbias, m, n, nc, rpc, part, tops, counters);
     return launch_status();
 }
 
 template <int ACT>
 int affine_bwd_t(const float *x, const float *scale, const float *y, const float *dy, float *dx,
                  float *dscale, float *dbias, size_t m, size_t n, cxm_stream_t st) {
-    return affine_bwd_plan<ACT>(x, scale, y, dy, dx, dscale, dbias, m, n, AffBwdPlan{0, 1}, st);
+    if (n < 4) {
+        size_t chunks = (m + 1023) / 1024 < kBlock ? (m + 1023) / 1024 : kBlock;
+        const size_t rpc = (m + chunks - 1) / chunks;
+        chunks = (m + rpc - 1) / rpc;
+        Workspace ws{};
+        if (chunks > 1) {
+            const int rc = get_workspace(st, kAffGroups + 1, 6 * kBlock * sizeof(float), &ws);
+            if (rc) return rc;
+        }
+        hipLaunchKernelGGL(k_affine_bwd_few<ACT>, dim3(static_cast<unsigned>(chunks)), dim3(kBlock), 0, hs(st), x, scale,
+                           y, dy, dx, dscale, dbias, m, static_cast<unsigned>(n), static_cast<unsigned>(chunks), rpc,
+                           static_cast<float *>(ws.scratch), ws.counters);
+        return launch_status();
+    }
+    // the fewest lanes whose float4s cover a row, up to a wave
+    const size_t v4 = (n + 3) / 4;
+    if (v4 <= 8) return affine_bwd_launch<ACT, false, 8>(x, scale, y, dy, dx, dscale, dbias, m, n, st);
+    if (v4 <= 16) return affine_bwd_launch<ACT, false, 16>(x, scale, y, dy, dx, dscale, dbias, m, n, st);
+    if (v4 <= 32) return affine_bwd_launch<ACT, false, 32>(x, scale, y, dy, dx, dscale, dbias, m, n, st);
+    if (n % 4 == 0 && aligned16(x) && aligned16(scale) && aligned16(y) && aligned16(dy) && aligned16(dx))
+        return affine_bwd_launch<ACT, true, 64>(x, scale, y, dy, dx, dscale, dbias, m, n, st);
+    return affine_bwd_launch<ACT, false, 64>(x, scale, y, dy, dx, dscale, dbias, m, n, st);
 }
 
 // ------------------------------------------------- sum / mean backward

@@ -112,14 +112,14 @@ constexpr int kDepth = 3;  // 8-k blocks in flight per wave
 template <int WI, int WJ, int NW, bool KCA, bool KCB>
 __global__ __launch_bounds__(NW * kWave) void k_gemm_direct(const float *__restrict__ A, const float *__restrict__ B,
                                                             float *__restrict__ C, size_t M, size_t N, size_t K,
-                                                            unsigned tiles_n, unsigned splits, size_t kper,
+                                                            unsigned wgs, unsigned tiles_n, unsigned splits, size_t kper,
                                                             Epilogue epi, float *__restrict__ part,
                                                             unsigned *__restrict__ counters) {
     constexpr int TM = 32 * WI, TN = 32 * WJ, LP = TN + 4;
     constexpr int NT = NW * kWave, Q = 32 * TN / 4;  // float4s of a 32-row block
     __shared__ __attribute__((aligned(16))) float sums[NW][32 * LP];
     __shared__ int flag;
-    const unsigned wg = xcd_remap(blockIdx.x, gridDim.x);
+    const unsigned wg = xcd_remap(blockIdx.x, wgs);
     const unsigned tile = wg / splits, split = wg - tile * splits;
     const size_t m0 = static_cast<size_t>(tile / tiles_n) * TM, n0 = static_cast<size_t>(tile % tiles_n) * TN;
     const size_t kbeg = static_cast<size_t>(split) * kper;
@@ -287,16 +287,16 @@ int launch_direct(const float *A, const float *B, float *C, size_t M, size_t K, 
     const size_t wgs = p.tiles * p.splits;
     if (wgs > 0x7fffffu) return 1;
     const dim3 grid(static_cast<unsigned>(wgs)), block(NW * kWave);
-    const unsigned tn = static_cast<unsigned>(p.tiles_n), sp = static_cast<unsigned>(p.splits);
+    const unsigned nw = static_cast<unsigned>(wgs), tn = static_cast<unsigned>(p.tiles_n), sp = static_cast<unsigned>(p.splits);
     hipStream_t s = reinterpret_cast<hipStream_t>(st);
     if (!ta && !tb)
-        hipLaunchKernelGGL((k_gemm_direct<WI, WJ, NW, true, false>), grid, block, 0, s, A, B, C, M, N, K, tn, sp, p.kper, epi,
+        hipLaunchKernelGGL((k_gemm_direct<WI, WJ, NW, true, false>), grid, block, 0, s, A, B, C, M, N, K, nw, tn, sp, p.kper, epi,
                            part, counters);
     else if (!ta)
-        hipLaunchKernelGGL((k_gemm_direct<WI, WJ, NW, true, true>), grid, block, 0, s, A, B, C, M, N, K, tn, sp, p.kper, epi,
+        hipLaunchKernelGGL((k_gemm_direct<WI, WJ, NW, true, true>), grid, block, 0, s, A, B, C, M, N, K, nw, tn, sp, p.kper, epi,
                            part, counters);
     else
-        hipLaunchKernelGGL((k_gemm_direct<WI, WJ, NW, false, false>), grid, block, 0, s, A, B, C, M, N, K, tn, sp, p.kper, epi,
+        hipLaunchKernelGGL((k_gemm_direct<WI, WJ, NW, false, false>), grid, block, 0, s, A, B, C, M, N, K, nw, tn, sp, p.kper, epi,
                            part, counters);
     return launch_status();
 }

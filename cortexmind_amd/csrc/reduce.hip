@@ -618,7 +618,8 @@ constexpr int kColTile = 256;  // columns per workgroup
 // ones that are theirs.  The per-wave results meet in LDS and threads 0..255
 // combine them in wave order.  Workgroup b -> (chunk, tile, outer slice),
 // chunk fastest: the chunks of one tile are adjacent in launch order, so its
-// combine runs while later tiles still stream.  Rows past the last whole
+// combine runs while later tiles still stream.  (No gridDim: the implicit
+// kernel arguments it brings cost 0.2-0.3 us of host time per launch.)  Rows past the last whole
 // batch of UNR go out as one batch too, its loads clamped to the chunk's last
 // row and only its own rows folded (one at a time, each waited a memory
 // round trip for the last).
@@ -626,6 +627,7 @@ template <class Op, bool AL, int UNR, int NW, bool FAST = false>
 __global__ __launch_bounds__(NW * kWave) void k_cols(const float *__restrict__ x, size_t dim,
                                                      size_t inner, unsigned ntiles, unsigned width, unsigned chunks,
                                                      size_t rows_per_chunk, typename Op::T *__restrict__ part,
+                                                     typename Op::T *__restrict__ tops,
                                                      unsigned *__restrict__ counters, OutDesc out) {
     using T = typename Op::T;
     __shared__ T lds[NW][kColTile];
@@ -784,7 +786,7 @@ __global__ __launch_bounds__(NW * kWave) void k_cols(const float *__restrict__ x
         const unsigned groups = (chunks + kPartGroup - 1) / kPartGroup, g = chunk / kPartGroup;
         const unsigned size = (g + 1) * kPartGroup <= chunks ? kPartGroup : chunks - g * kPartGroup;
         unsigned *cg = ctr(counters, t * (kTicketGroups + 1));
-        T *top = part + static_cast<size_t>(gridDim.x) * gridDim.y * gridDim.z * kColTile + t * kTicketGroups * kColTile;
+        T *top = tops + t * kTicketGroups * kColTile;
         if (!last_block_ticket(ctr(cg, g), size, &flag)) return;
         if (owner)
             st_dev(&top[g * kColTile + tid],
@@ -1257,9 +1259,10 @@ int run_cols_plan(const float *x, size_t outer, size_t dim, size_t inner, OutDes
     // tiles of equal width: with the last tile only a few columns wide, half
     // the workgroups of an inner of 257 would stream next to nothing
     const unsigned width = static_cast<unsigned>(((inner + 3) / 4 + ntiles - 1) / ntiles * 4);
+    T *tops = part ? part + blocks * kColTile : nullptr;  // the group partials of more than 32 chunks
 #define CXM_COLS(AL_, UNR_, FAST_, NW)                                                                              \
     hipLaunchKernelGGL((k_cols<Op, AL_, UNR_, NW, FAST_>), grid, dim3(NW * kWave), 0, hs, x, dim, inner, nt, width, nc, \
-                       rpc, part, counters, out)
+                       rpc, part, tops, counters, out)
     if constexpr (sizeof(T) == 4) {  // the column argmax measured 14.3 -> 14.5 us in this form
         if (fast && chunks > 1 && chunks <= kTicketGroups && rpc == kWholeRows && dim == chunks * kWholeRows &&
             inner <= 0xffffffffu) {

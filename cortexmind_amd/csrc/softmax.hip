@@ -773,16 +773,16 @@ __global__ __launch_bounds__(kBlock) void k_sm_bwd_any(const float *__restrict__
 // adds them in order and writes the mean.
 constexpr unsigned kXentGroups = 32;
 
-__device__ __forceinline__ void xent_loss(float nll, float *loss, size_t b, float *part, unsigned *counters,
+__device__ __forceinline__ void xent_loss(float nll, float *loss, size_t b, unsigned blocks, float *part, unsigned *counters,
                                           float *lds, int *flag) {
     nll = block_reduce<SumOp, kBlock>(nll, lds);
-    if (gridDim.x == 1) {
+    if (blocks == 1) {
         if (threadIdx.x == 0) loss[0] = nll / static_cast<float>(b);
         return;
     }
     if (threadIdx.x == 0) st_dev(&part[blockIdx.x], nll);
-    if (!last_block_ticket2<kXentGroups>(counters, gridDim.x, blockIdx.x, flag)) return;
-    const unsigned mine = threadIdx.x < gridDim.x ? (gridDim.x - threadIdx.x + kBlock - 1) / kBlock : 0;
+    if (!last_block_ticket2<kXentGroups>(counters, blocks, blockIdx.x, flag)) return;
+    const unsigned mine = threadIdx.x < blocks ? (blocks - threadIdx.x + kBlock - 1) / kBlock : 0;
     float t = combine_partials<SumOp>(part + threadIdx.x, mine, kBlock, 0.0f);
     t = block_reduce<SumOp, kBlock>(t, lds);
     if (threadIdx.x == 0) loss[0] = t / static_cast<float>(b);
@@ -791,7 +791,7 @@ __device__ __forceinline__ void xent_loss(float nll, float *loss, size_t b, floa
 // c < 4: one thread per row.
 __global__ __launch_bounds__(kBlock) void k_xent_few(const float *__restrict__ logits,
                                                      const int32_t *__restrict__ labels, float *__restrict__ loss,
-                                                     float *__restrict__ dl, size_t b, size_t c, float inv_b,
+                                                     float *__restrict__ dl, size_t b, size_t c, float inv_b, unsigned blocks,
                                                      float *__restrict__ part, unsigned *__restrict__ counters) {
     __shared__ float lds[kWavesPerBlock];
     __shared__ int flag;
@@ -818,7 +818,7 @@ __global__ __launch_bounds__(kBlock) void k_xent_few(const float *__restrict__ l
             dr[j] = p * inv_b;
         }
     }
-    xent_loss(nll, loss, b, part, counters, lds, &flag);
+    xent_loss(nll, loss, b, blocks, part, counters, lds, &flag);
 }
 
 // 4 <= c <= 256 NV (G = 64) or 4 G: G lanes per row, NV float4 per lane at
@@ -829,7 +829,7 @@ __global__ __launch_bounds__(kBlock) void k_xent_few(const float *__restrict__ l
 template <int G, int NV>
 __global__ __launch_bounds__(kBlock) void k_xent_rows(const float *__restrict__ logits,
                                                       const int32_t *__restrict__ labels, float *__restrict__ loss,
-                                                      float *__restrict__ dl, size_t b, int c, float inv_b,
+                                                      float *__restrict__ dl, size_t b, int c, float inv_b, unsigned blocks,
                                                       float *__restrict__ part, unsigned *__restrict__ counters) {
     __shared__ float lds[kWavesPerBlock];
     __shared__ int flag;
@@ -879,14 +879,14 @@ __global__ __launch_bounds__(kBlock) void k_xent_rows(const float *__restrict__ 
     }
     float nll = 0.0f;
     if (live && l == 0) nll = ok ? -((xl - m) - logf(s)) : NAN;
-    xent_loss(nll, loss, b, part, counters, lds, &flag);
+    xent_loss(nll, loss, b, blocks, part, counters, lds, &flag);
 }
 
 // Wider rows: one workgroup per row, three sweeps (the second and third
 // mostly hit L2), four loads in flight per thread.
 __global__ __launch_bounds__(kBlock) void k_xent_wide(const float *__restrict__ logits,
                                                       const int32_t *__restrict__ labels, float *__restrict__ loss,
-                                                      float *__restrict__ dl, size_t b, int c, float inv_b,
+                                                      float *__restrict__ dl, size_t b, int c, float inv_b, unsigned blocks,
                                                       float *__restrict__ part, unsigned *__restrict__ counters) {
     __shared__ float lds[kWavesPerBlock];
     __shared__ int flag;
@@ -932,7 +932,7 @@ __global__ __launch_bounds__(kBlock) void k_xent_wide(const float *__restrict__ 
     });
     float nll = 0.0f;
     if (threadIdx.x == 0) nll = ok ? -((xl - m) - logf(s)) : NAN;
-    xent_loss(nll, loss, b, part, counters, lds, &flag);
+    xent_loss(nll, loss, b, blocks, part, counters, lds, &flag);
 }
 
 // ------------------------------------------------------------------ host
@@ -1222,14 +1222,15 @@ int cxm_softmax_xent_f32(const float *logits, const int32_t *labels, float *loss
     if (rc) return rc;
     hipStream_t s = hs(st);
     const float inv_b = 1.0f / static_cast<float>(b);
-    const dim3 grid(static_cast<unsigned>(blocks));
+    const unsigned nb = static_cast<unsigned>(blocks);
+    const dim3 grid(nb);
     float *part = static_cast<float *>(ws.scratch);
     const int ci = static_cast<int>(c);
 #define CXM_XENT(G, NV)                                                                                              \
-    hipLaunchKernelGGL((k_xent_rows<G, NV>), grid, dim3(kBlock), 0, s, logits, labels, loss, dlogits, b, ci, inv_b,  \
+    hipLaunchKernelGGL((k_xent_rows<G, NV>), grid, dim3(kBlock), 0, s, logits, labels, loss, dlogits, b, ci, inv_b, nb,  \
                        part, ws.counters)
     if (c < 4)
-        hipLaunchKernelGGL(k_xent_few, grid, dim3(kBlock), 0, s, logits, labels, loss, dlogits, b, c, inv_b, part,
+        hipLaunchKernelGGL(k_xent_few, grid, dim3(kBlock), 0, s, logits, labels, loss, dlogits, b, c, inv_b, nb, part,
                            ws.counters);
     else if (v4 <= 4) CXM_XENT(4, 1);
     else if (v4 <= 8) CXM_XENT(8, 1);
@@ -1241,7 +1242,7 @@ int cxm_softmax_xent_f32(const float *logits, const int32_t *labels, float *loss
     else if (v4 <= 512) CXM_XENT(64, 8);
     else if (c <= kWaveRowMax) CXM_XENT(64, 16);
     else
-        hipLaunchKernelGGL(k_xent_wide, grid, dim3(kBlock), 0, s, logits, labels, loss, dlogits, b, ci, inv_b, part,
+        hipLaunchKernelGGL(k_xent_wide, grid, dim3(kBlock), 0, s, logits, labels, loss, dlogits, b, ci, inv_b, nb, part,
                            ws.counters);
 #undef CXM_XENT
     return launch_status();

@@ -229,3 +229,51 @@ def test_tanh_ranges(hip):
     assert got[0] == 0.0 and not np.signbit(got[0]) and got[1] == 0.0 and np.signbit(got[1])
     assert got[2] == 1.0 and got[3] == -1.0 and np.isnan(got[4])
     assert list(got[5:]) == [1.0, -1.0, 1.0, -1.0]
+
+
+@pytest.mark.parametrize("m,n", [(1, 4), (3, 5), (7, 7), (300, 1), (5000, 2), (3000, 3), (65, 16), (129, 33), (1000, 61),
+                                 (517, 65), (300, 129), (90, 255), (700, 257), (33, 1003), (2, 4097), (9000, 35),
+                                 (4096, 130)])
+@pytest.mark.parametrize("off", [0, 1])
+def test_row_maps_of_any_width(hip, orc, m, n, off):
+    """The flat row maps and the affine backward's lane groups at the edges of
+    their ranges, rows of no multiple of four floats and bases that are only
+    4-byte aligned, in buffers whose surroundings must stay: broadcasts and
+    the ReLU affine forward and dX bit for bit, the column sums against
+    float64."""
+    g = SplitMix64(0xF1A7 + 31 * m + n)
+    x, dy = g.normal((m, n)), g.normal((m, n))
+    row, col, bias = g.uniform((n,), 0.5, 1.5), g.uniform((m,), 0.5, 1.5), g.normal((n,), 0.0, 0.1)
+    dx_, drow, dcol, dbias, ddy = dev(x, off), dev(row, off), dev(col, off), dev(bias, off), dev(dy, off)
+
+    def guarded(shape):
+        size = int(np.prod(shape))
+        v = dev(np.full(size + 9, 7.0, np.float32), 4 + off)
+
+        def read():
+            full = v.base.numpy()
+            s = 4 + off
+            assert np.all(full[:s] == 0.0) and np.all(full[s + size:] == 7.0)
+            return full[s:s + size].reshape(shape)
+        return v, read
+
+    for op in range(4):
+        f = (np.add, np.subtract, np.multiply, np.divide)[op]
+        for fn, operand, want in (("cxm_bcast_row_f32", drow, f(x, row)), ("cxm_bcast_col_f32", dcol, f(x, col[:, None]))):
+            z, read = guarded((m, n))
+            call(fn, dx_.ptr, operand.ptr, z.ptr, m, n, op, None)
+            assert bits_equal(read(), want)
+    z, read = guarded((m, n))
+    call("cxm_affine_act_fwd_f32", dx_.ptr, drow.ptr, dbias.ptr, z.ptr, m, n, 1, None)
+    y = np.where(0.0 > x * row + bias, np.float32(0.0), x * row + bias)
+    assert bits_equal(read(), y)
+    d, read = guarded((m, n))
+    ds, read_s = guarded((n,))
+    db, read_b = guarded((n,))
+    dyv = dev(y, off)
+    call("cxm_affine_act_bwd_f32", dx_.ptr, drow.ptr, dyv.ptr, ddy.ptr, d.ptr, ds.ptr, db.ptr, m, n, 1, None)
+    dz = dy * np.where(y > 0, np.float32(1.0), np.float32(0.0))
+    assert bits_equal(read(), dz * row)
+    dz64, x64 = dz.astype(np.float64), x.astype(np.float64)
+    assert np.all(np.abs(read_s() - (dz64 * x64).sum(0)) <= 1e-5 * np.abs(dz64 * x64).sum(0) + 1e-30)
+    assert np.all(np.abs(read_b() - dz64.sum(0)) <= 1e-5 * np.abs(dz64).sum(0) + 1e-30)
