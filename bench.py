@@ -516,7 +516,7 @@ def wl_c1(E, D):
     nbuf = 128  # 2 MiB each: 256 MiB of inputs and 256 MiB of outputs rotate
     xs = [D.from_numpy(x) for _ in range(nbuf)]
     ys = [D((r, c)) for _ in range(nbuf)]
-    ops = [Op("softmax_fwd", "k_sm_fwd_wave<4,false,2>",
+    ops = [Op("softmax_fwd", "k_sm_fwd_rows<64,4,false,true>",
               lambda k: E.softmax.forward(xs[k % nbuf], ys[k % nbuf], r, c), 2 * 4 * x.size)]
     desc = {"workload": "C1 row softmax fp32 [512,1024] N(0,1)*4", "shape": [r, c],
             "rotating_input_buffers": nbuf,
@@ -542,7 +542,7 @@ def wl_c3(E, D):
         ops.append(Op(f"fwd_{nm}", f"k_rowmap4<AffineF<{act}>>",
                       lambda k, act=act: A.affine_fwd(dx_, ds_, db_, y_, m, n, act), 2 * big + 2 * 4 * n))
     for act, nm in [(E.ACT_RELU, "relu"), (E.ACT_SIGMOID, "sigmoid"), (E.ACT_TANH, "tanh")]:
-        ops.append(Op(f"bwd_{nm}", f"k_affine_bwd<{act},true,1,4>",
+        ops.append(Op(f"bwd_{nm}", f"k_affine_bwd<{act},true,64,1>",
                       lambda k, act=act: A.affine_bwd(dx_, ds_, y_, dy_, dX, dS, dB, m, n, act),
                       4 * big + 3 * 4 * n))
     desc = {"workload": "C3 Y=act(X*scale+bias) fp32 [8192,8192], fwd+bwd, act in relu/sigmoid/tanh",
