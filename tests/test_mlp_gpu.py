@@ -160,3 +160,18 @@ def test_mlp_pair_without_free_cus_vs_oracle(hip, orc):
         w = "w" + k[1]
         scale = max(np.abs(params[w]).max(), np.abs(ref[w]).max())
         assert np.max(np.abs(final[k] - ref[k])) <= 1e-4 * scale, k
+
+
+@pytest.mark.parametrize("d2", [252, 256, 260, 508, 512, 516])
+def test_mlp_head_widths_vs_oracle(hip, orc, d2):
+    """The fused output layer takes 4, 8 or 16 waves by d2 (64 columns each):
+    widths at and on either side of the two lines, a partial last 16-row
+    tile, one step, same bars as above."""
+    x, labels, params = c5_mlp(batch=37, dims=(24, 40, d2, 10))
+    losses, final = gpu_steps(x, labels, params, 0.05, 1)
+    ref = {k: v.copy() for k, v in params.items()}
+    want = orc.mlp_step(x, labels, ref, 0.05)
+    assert abs(losses[0] - want) <= 1e-5 * max(abs(want), 1e-3), (losses, want)
+    for k in ref:
+        scale = np.abs(ref["w" + k[1]]).max()
+        assert np.max(np.abs(final[k] - ref[k])) <= 1e-4 * scale, k
