@@ -107,9 +107,14 @@ struct Side {
     }
 };
 
-constexpr int kDepth = 3;  // 8-k blocks in flight per wave
+constexpr int kDepth = 3;      // 8-k blocks in flight per wave
+// Blocks per run of sums (264 k), a multiple of kDepth.  In one chain of all
+// its K / (NW splits) terms a wave's rounding error grows with the square
+// root of the chain: 333x8191x517, 2048 terms, 8.1e-7 of the result against
+// 64 bits, 3.0e-7 in runs.
+constexpr unsigned kRun = 33;
 
-template <int WI, int WJ, int NW, bool KCA, bool KCB>
+template <int WI, int WJ, int NW, bool KCA, bool KCB, bool RUNS>
 __global__ __launch_bounds__(NW * kWave) void k_gemm_direct(const float *__restrict__ A, const float *__restrict__ B,
                                                             float *__restrict__ C, size_t M, size_t N, size_t K,
                                                             unsigned wgs, unsigned tiles_n, unsigned splits, size_t kper,
@@ -140,6 +145,29 @@ __global__ __launch_bounds__(NW * kWave) void k_gemm_direct(const float *__restr
 #pragma unroll
             for (int r = 0; r < 16; ++r) acc[i][j][r] = 0.0f;
 
+    // RUNS: every kRun blocks the sums so far are added to `total` and begin
+    // again from zero (see kRun).
+    floatx16 total[WI][WJ];
+    if constexpr (RUNS) {
+#pragma unroll
+        for (int i = 0; i < WI; ++i)
+#pragma unroll
+            for (int j = 0; j < WJ; ++j) total[i][j] = acc[i][j];
+    }
+    auto close_run = [&] {
+        if constexpr (RUNS) {
+#pragma unroll
+            for (int i = 0; i < WI; ++i)
+#pragma unroll
+                for (int j = 0; j < WJ; ++j)
+#pragma unroll
+                    for (int r = 0; r < 16; ++r) {
+                        total[i][j][r] = total[i][j][r] + acc[i][j][r];
+                        acc[i][j][r] = 0.0f;
+                    }
+        }
+    };
+
     // whole blocks of this wave: w, w + NW, ... < nb
     const unsigned nb = static_cast<unsigned>((kend - kbeg) / 8);
     const unsigned T = nb > w ? (nb - w + NW - 1) / NW : 0;
@@ -165,14 +193,19 @@ __global__ __launch_bounds__(NW * kWave) void k_gemm_direct(const float *__restr
         }
         __builtin_amdgcn_sched_barrier(0);
         unsigned t = 0;
-        for (; t + kDepth <= T; t += kDepth) {
+        for (;;) {
+            const unsigned stop = RUNS && T - t > kRun ? t + kRun : T;
+            for (; t + kDepth <= stop; t += kDepth) {
 #pragma unroll
-            for (int d = 0; d < kDepth; ++d) {
-                mul(fa[d], fb[d]);
-                a.load(at(t + d + kDepth), fa[d]);
-                b.load(at(t + d + kDepth), fb[d]);
-                __builtin_amdgcn_sched_barrier(0);
+                for (int d = 0; d < kDepth; ++d) {
+                    mul(fa[d], fb[d]);
+                    a.load(at(t + d + kDepth), fa[d]);
+                    b.load(at(t + d + kDepth), fb[d]);
+                    __builtin_amdgcn_sched_barrier(0);
+                }
             }
+            if (stop == T) break;
+            close_run();
         }
 #pragma unroll
         for (int d = 0; d < kDepth; ++d)
@@ -184,6 +217,13 @@ __global__ __launch_bounds__(NW * kWave) void k_gemm_direct(const float *__restr
         a.load_tail(kbeg + 8 * static_cast<size_t>(nb), rest, lhi, x);
         b.load_tail(kbeg + 8 * static_cast<size_t>(nb), rest, lhi, y);
         mul(x, y);
+    }
+    if constexpr (RUNS) {
+        close_run();
+#pragma unroll
+        for (int i = 0; i < WI; ++i)
+#pragma unroll
+            for (int j = 0; j < WJ; ++j) acc[i][j] = total[i][j];
     }
 
     // the waves' sums meet in LDS, one 32-row block i of the accumulators at a
@@ -289,15 +329,20 @@ int launch_direct(const float *A, const float *B, float *C, size_t M, size_t K, 
     const dim3 grid(static_cast<unsigned>(wgs)), block(NW * kWave);
     const unsigned nw = static_cast<unsigned>(wgs), tn = static_cast<unsigned>(p.tiles_n), sp = static_cast<unsigned>(p.splits);
     hipStream_t s = reinterpret_cast<hipStream_t>(st);
-    if (!ta && !tb)
-        hipLaunchKernelGGL((k_gemm_direct<WI, WJ, NW, true, false>), grid, block, 0, s, A, B, C, M, N, K, nw, tn, sp, p.kper, epi,
-                           part, counters);
-    else if (!ta)
-        hipLaunchKernelGGL((k_gemm_direct<WI, WJ, NW, true, true>), grid, block, 0, s, A, B, C, M, N, K, nw, tn, sp, p.kper, epi,
-                           part, counters);
-    else
-        hipLaunchKernelGGL((k_gemm_direct<WI, WJ, NW, false, false>), grid, block, 0, s, A, B, C, M, N, K, nw, tn, sp, p.kper, epi,
-                           part, counters);
+#define CXM_DIRECT(KCA, KCB, RUNS)                                                                                    \
+    hipLaunchKernelGGL((k_gemm_direct<WI, WJ, NW, KCA, KCB, RUNS>), grid, block, 0, s, A, B, C, M, N, K, nw, tn, sp, \
+                       p.kper, epi, part, counters)
+    constexpr bool kRuns = NW == 4 && WI * WJ <= 2;
+    if (kRuns && p.kper > 8 * NW * kRun) {
+        if (!ta && !tb) CXM_DIRECT(true, false, kRuns);
+        else if (!ta) CXM_DIRECT(true, true, kRuns);
+        else CXM_DIRECT(false, false, kRuns);
+    } else {
+        if (!ta && !tb) CXM_DIRECT(true, false, false);
+        else if (!ta) CXM_DIRECT(true, true, false);
+        else CXM_DIRECT(false, false, false);
+    }
+#undef CXM_DIRECT
     return launch_status();
 }
 
@@ -338,6 +383,10 @@ bool ring_fits(size_t M, size_t N, size_t K) {
 //   784x4096x1024 TN 102  / 82.5 /  82.9 /  73.9
 // Small grids want many small tiles; a 64x64 tile reads half as much per
 // flop, which counts once every CU has two; beyond K = 2048 its splits pay.
+// 32x64 tiles of more than 1056 k keep their waves' chains within kRun blocks
+// by eight waves instead of four (1203x2000x1500 A B 79 us with four, 81 with
+// eight, 93 with runs), for A B^T, whose loads eight waves slow down, by runs
+// (106 / 115 / 98).
 int gemm_direct(const float *A, const float *B, float *C, size_t M, size_t K, size_t N, int ta, int tb,
                 const Epilogue &epi, bool ring, cxm_stream_t st) {
     // 32-bit byte offsets within a tile; pairs of columns of a [K, M] / [K, N] operand
@@ -346,7 +395,10 @@ int gemm_direct(const float *A, const float *B, float *C, size_t M, size_t K, si
     if (ring && ring_fits(M, N, K)) return 1;
     const size_t t64 = ((M + 63) / 64) * ((N + 63) / 64);
     if (t64 < 200) return launch_direct<1, 1, 4>(A, B, C, M, K, N, ta, tb, epi, 256, st);
-    if (t64 < 600 && K < 2048) return launch_direct<1, 2, 4>(A, B, C, M, K, N, ta, tb, epi, 256, st);
+    if (t64 < 600 && K < 2048) {
+        if (K > 4 * 8 * kRun && !tb) return launch_direct<1, 2, 8>(A, B, C, M, K, N, ta, tb, epi, 256, st);
+        return launch_direct<1, 2, 4>(A, B, C, M, K, N, ta, tb, epi, 256, st);
+    }
     return launch_direct<2, 2, 4>(A, B, C, M, K, N, ta, tb, epi, K < 2048 ? 1 : 768, st);
 }
 

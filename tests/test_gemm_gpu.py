@@ -222,3 +222,24 @@ def test_direct_products(hip, m, k, n, ta, tb, off):
     want[m // 2, :] = True
     want[:, n - 1] = True
     assert np.array_equal(bad, want)
+
+
+@pytest.mark.parametrize("m,k,n", [(250, 8191, 700), (333, 4100, 517), (500, 3001, 500), (48, 4100, 2192),
+                                   (512, 4096, 511)], ids=lambda v: str(v))
+@pytest.mark.parametrize("ta,tb", [(0, 0), (1, 0), (0, 1)])
+def test_long_k_error(hip, m, k, n, ta, tb):
+    """Few tiles and a long K: the root mean square error stays that of sums
+    in runs, not of one chain per wave.  A chain of L products of unit
+    normals rounds partial sums of size sqrt(1) .. sqrt(L) by 2^-23 / sqrt(24)
+    of their size each (rms over a mantissa): 2^-23 / sqrt(48) * sqrt(L) of
+    the result, whatever the number of chains.  L: the K split of 128x128
+    tiles over 256 CUs, at least 256, or the direct tiles' 264 and their runs'
+    own sum; a quarter on top for the partial sums' sums."""
+    g = SplitMix64(0x10C + m + 3 * k + 7 * n + 11 * ta + 13 * tb)
+    a, b = g.normal((m, k)), g.normal((k, n))
+    got = run(a, b, ta, tb).astype(np.float64)
+    ref = a.astype(np.float64) @ b.astype(np.float64)
+    tiles = -(-m // 128) * -(-n // 128)
+    length = max(k / min(256 // tiles, k // 256), 264 + k / (4 * 264))
+    err = np.linalg.norm(got - ref) / np.linalg.norm(ref)
+    assert err <= 1.25 * 2.0**-23 / np.sqrt(48.0) * np.sqrt(length), err
