@@ -1274,18 +1274,20 @@ __global__ __launch_bounds__(kThinNT) void k_gemm_thin_k(const float *__restrict
 // (where its shape conditions hold, else 1).
 std::atomic<int> g_gemm_kc{-1};
 
-// Measured on gfx950 (TFLOP/s, best variant vs the others):
+// The choice among these kernels, for what gemm_direct (which has its pick of
+// A B, A^T B and A B^T first, see there) leaves to them.  Measured on gfx950
+// (TFLOP/s, best variant vs the others):
 //  * grids of >= 1024 workgroups (8192^3, 4096^3): four waves of 64x64, BK 32
 //    (125 / 115 against <= 116 / 113);
 //  * A^T B (the MLP's weight gradients, split K): k-major tiles with the XCD
 //    renumbering (97.5 and 77 against 87-89 and 70-75);
 //  * A B and A B^T at 256-tile grids: k-contiguous tiles, BK 32, with the
 //    renumbering (93 and 104 against 90 and 94 for the k-major kernel).
-//  * the ring (M, N, K multiples of 128, 16-byte aligned bases) for A B,
-//    A B^T and A^T B: 99-100 against 92-95 at 4096x1024x1024, 133 against
-//    113 at 4096^3, 135 against 125 at 8192^3; A^T B with K split four ways
-//    (1024x4096x1024) 3-8% faster than the k-major kernel in interleaved
-//    runs.
+//  * the ring (K a multiple of 8, 16-byte aligned bases, see ring_shape_ok)
+//    for A B, A B^T and A^T B: 99-100 against 92-95 at 4096x1024x1024, 133
+//    against 113 at 4096^3, 135 against 125 at 8192^3; A^T B with K split
+//    four ways (1024x4096x1024) 3-8% faster than the k-major kernel in
+//    interleaved runs.
 inline int gemm_variant(bool ta, bool tb, unsigned wgs, bool ring_ok) {
     const int pinned = g_gemm_kc.load(std::memory_order_relaxed);
     if (pinned == 7) return ring_ok ? 7 : 1;
@@ -1395,30 +1397,22 @@ int gemm_ex(const float *A, const float *B, float *C, size_t M, size_t K, size_t
         const int t = gemm_thin(A, B, C, M, K, N, ta, tb, epi, st);
         if (t != 1) return t;
     }
-    if (g_gemm_kc.load(std::memory_order_relaxed) < 0) {  // no kernel pinned
-        const int t = gemm_direct(A, B, C, M, K, N, ta, tb, epi, ring_shape_ok(A, B, M, K, N, ta, tb), st);
-        if (t != 1) return t;
-    }
-    const size_t tiles_m = (M + BM - 1) / BM, tiles_n = (N + BN - 1) / BN;
-    const size_t tiles = tiles_m * tiles_n;
-    // Split K when the tile grid alone cannot fill the chip's CUs (256 here);
-    // each split keeps at least 256 of K.
-    size_t splits = 1;
-    // (at most one workgroup per CU: one 8-wave workgroup fills a CU, and
-    // one more would run as a second round)
-    const size_t cus = device_cus();
-    if (tiles < cus * 3 / 4 && K >= 512) {
-        splits = cus / tiles;
-        const size_t max_splits = K / 256;
-        if (splits > max_splits) splits = max_splits;
-        if (splits < 1) splits = 1;
-    }
-    // a split's k range is a whole number of the kernel's k steps (the
-    // ring's: four stages of 32)
     // the ring: whole 8-k blocks; a partial last M or N tile is clamped,
     // which needs the [K, M] / [K, N] storage's row length a multiple of 4;
     // its lanes address a stage with 32-bit byte offsets (ring_offsets)
     const bool ring_ok = ring_shape_ok(A, B, M, K, N, ta, tb);
+    // 128-bit global loads need the stored row length to be a multiple of 4.
+    const bool va = aligned16(A) && (ta ? M % 4 == 0 : K % 4 == 0);
+    const bool vb = aligned16(B) && (tb ? K % 4 == 0 : N % 4 == 0);
+    if (g_gemm_kc.load(std::memory_order_relaxed) < 0) {  // no kernel pinned
+        const int t = gemm_direct(A, B, C, M, K, N, ta, tb, epi, ring_ok, (va ? 1 : 0) + (vb ? 1 : 0), st);
+        if (t != 1) return t;
+    }
+    const size_t tiles_m = (M + BM - 1) / BM, tiles_n = (N + BN - 1) / BN;
+    const size_t tiles = tiles_m * tiles_n;
+    size_t splits = gemm_splits(tiles, K, device_cus());
+    // a split's k range is a whole number of the kernel's k steps (the
+    // ring's: four stages of 32)
     const int variant = gemm_variant(ta, tb, static_cast<unsigned>(tiles * splits), ring_ok);
     const size_t kstep = variant == 7 ? 4 * kRBK : (variant == 2 || variant == 4) ? 64 : BK;
     size_t kper = (K + splits - 1) / splits;
@@ -1434,9 +1428,6 @@ int gemm_ex(const float *A, const float *B, float *C, size_t M, size_t K, size_t
         part = static_cast<float *>(ws.scratch);
         counters = ws.counters;
     }
-    // 128-bit global loads need the stored row length to be a multiple of 4.
-    const bool va = aligned16(A) && (ta ? M % 4 == 0 : K % 4 == 0);
-    const bool vb = aligned16(B) && (tb ? K % 4 == 0 : N % 4 == 0);
     const dim3 grid(static_cast<unsigned>(tiles * splits));
     hipStream_t s = reinterpret_cast<hipStream_t>(st);
     const unsigned tn = static_cast<unsigned>(tiles_n), sp = static_cast<unsigned>(splits);
@@ -1457,14 +1448,7 @@ bool ring_plan(const float *A, const float *B, size_t M, size_t K, size_t N, int
     if (N <= kThin || K <= kThin) return false;  // thin kernels
     const bool ring_ok = ring_shape_ok(A, B, M, K, N, ta, tb);
     const size_t tm = (M + BM - 1) / BM, tn = (N + BN - 1) / BN, t = tm * tn;
-    size_t sp = 1;
-    const size_t cus = device_cus();
-    if (t < cus * 3 / 4 && K >= 512) {
-        sp = cus / t;
-        const size_t max_splits = K / 256;
-        if (sp > max_splits) sp = max_splits;
-        if (sp < 1) sp = 1;
-    }
+    size_t sp = gemm_splits(t, K, device_cus());
     if (gemm_variant(ta, tb, static_cast<unsigned>(t * sp), ring_ok) != 7) return false;
     size_t kp = (K + sp - 1) / sp;
     kp = (kp + 4 * kRBK - 1) / (4 * kRBK) * (4 * kRBK);

@@ -346,23 +346,39 @@ int launch_direct(const float *A, const float *B, float *C, size_t M, size_t K, 
     return launch_status();
 }
 
-// Whether the ring of gemm.hip, which takes this product, is the faster: its
-// 128x128 tiles times its K splits fill nine tenths of the chip's rounds and
-// are long enough for its fill and epilogue, or a long K is split over three
-// quarters of it.
-bool ring_fits(size_t M, size_t N, size_t K) {
+// Estimated times, in us, of a product on the kernels of gemm.hip and on the
+// direct tiles: rounds of workgroups over the chip, each its own cost plus its
+// k range times the cost per k.  gemm_direct takes the smaller one.
+
+// 128x128 tiles, one workgroup per CU and round: 60 ns per k in the ring, 70
+// in the register-staged kernels (78 in the four-wave ones of large grids), 80
+// with element loads of one operand, 85 (A B^T 95) of both.
+double staged_us(size_t M, size_t N, size_t K, int tb, bool ring, int vecs) {
     const size_t tiles = ((M + 127) / 128) * ((N + 127) / 128), cus = device_cus();
-    size_t splits = 1;
-    if (tiles < cus * 3 / 4 && K >= 512) {  // gemm_ex's split
-        splits = cus / tiles < K / 256 ? cus / tiles : K / 256;
-        if (splits < 1) splits = 1;
-    }
-    const size_t kper = ((K + splits - 1) / splits + 127) / 128 * 128;
+    size_t splits = gemm_splits(tiles, K, cus);
+    const size_t step = ring ? 128 : 32, kper = ((K + splits - 1) / splits + step - 1) / step * step;
     splits = (K + kper - 1) / kper;
     const size_t rounds = (tiles * splits + cus - 1) / cus;
-    const double used = static_cast<double>(M) * N * K /
-                        (static_cast<double>(rounds * cus) * 128 * 128 * (splits > 1 ? kper : K));
-    return (used >= 0.9 && kper >= 512) || (used >= 0.76 && splits > 1 && K >= 2048);
+    const double per_k = ring ? 0.060 : vecs == 0 ? (tb ? 0.095 : 0.085) : vecs == 1 ? 0.080 : tiles * splits >= 1024 ? 0.078 : 0.070;
+    return 3.0 + (splits > 1 ? 4.0 + 0.7 * splits : 0.0) + 7.5 * rounds - 1.5 + rounds * per_k * (splits > 1 ? kper : K);
+}
+
+// Direct tiles of 32 wi x 32 wj: kPerK per k of one 32x32 block, by tile and
+// form (A B, A^T B, A B^T); more where an odd K puts the rows of a k-contiguous
+// operand at odd alignments, for A B^T of long K, and for the splits of A^T B
+// (short ones above all).  Of the smallest tiles, a second round only partly there
+// costs less than a whole one.
+double direct_us(size_t M, size_t N, size_t K, int ta, int tb, size_t wi, size_t wj, size_t nw, size_t target) {
+    constexpr double kPerK[3][3] = {{0.0066, 0.0062, 0.0070}, {0.0050, 0.0055, 0.0062}, {0.0043, 0.0045, 0.0047}};
+    const size_t blocks = wi * wj;
+    const DirectPlan p = direct_plan(M, N, K, 32 * wi, 32 * wj, 8 * nw, kDepth, target);
+    const double x = static_cast<double>(p.tiles * p.splits) / device_cus(), k = p.splits > 1 ? p.kper : K;
+    double e = kPerK[blocks == 4 ? 2 : blocks - 1][tb ? 2 : ta ? 1 : 0], rounds = ceil(x);
+    if (!ta && K % 4 != 0 && (tb || blocks == 1)) e *= blocks == 4 && k >= 4096 ? 1.4 : 1.12;
+    else if (blocks == 4 && tb && K >= 2048) e *= p.splits > 1 ? 1.2 : 1.15;
+    else if (blocks == 4 && ta && p.splits > 1) e *= k < 1200 ? 1.4 : 1.2;
+    if (blocks == 1 && !tb && x > 1.0 && x < 2.0) rounds = 1.4 * x - 0.6 < 2.0 ? 1.4 * x - 0.6 : 2.0;
+    return 4.0 + rounds * blocks * ((blocks == 4 ? 0.42 : 0.3) + e * k);
 }
 
 }  // namespace
@@ -388,18 +404,24 @@ bool ring_fits(size_t M, size_t N, size_t K) {
 // eight, 93 with runs), for A B^T, whose loads eight waves slow down, by runs
 // (106 / 115 / 98).
 int gemm_direct(const float *A, const float *B, float *C, size_t M, size_t K, size_t N, int ta, int tb,
-                const Epilogue &epi, bool ring, cxm_stream_t st) {
+                const Epilogue &epi, bool ring, int vecs, cxm_stream_t st) {
     // 32-bit byte offsets within a tile; pairs of columns of a [K, M] / [K, N] operand
     constexpr size_t kMaxLd = size_t(1) << 23;
     if ((ta && tb) || M >= kMaxLd || N >= kMaxLd || K >= kMaxLd || (ta && M < 2) || (!tb && N < 2)) return 1;
-    if (ring && ring_fits(M, N, K)) return 1;
     const size_t t64 = ((M + 63) / 64) * ((N + 63) / 64);
-    if (t64 < 200) return launch_direct<1, 1, 4>(A, B, C, M, K, N, ta, tb, epi, 256, st);
+    const double staged = staged_us(M, N, K, tb, ring, vecs);
+    if (t64 < 200) {
+        if (direct_us(M, N, K, ta, tb, 1, 1, 4, 256) > staged) return 1;
+        return launch_direct<1, 1, 4>(A, B, C, M, K, N, ta, tb, epi, 256, st);
+    }
     if (t64 < 600 && K < 2048) {
+        if (direct_us(M, N, K, ta, tb, 1, 2, 4, 256) > staged) return 1;
         if (K > 4 * 8 * kRun && !tb) return launch_direct<1, 2, 8>(A, B, C, M, K, N, ta, tb, epi, 256, st);
         return launch_direct<1, 2, 4>(A, B, C, M, K, N, ta, tb, epi, 256, st);
     }
-    return launch_direct<2, 2, 4>(A, B, C, M, K, N, ta, tb, epi, K < 2048 ? 1 : 768, st);
+    const size_t target = K < 2048 ? 1 : 768;
+    if (direct_us(M, N, K, ta, tb, 2, 2, 4, target) > staged) return 1;
+    return launch_direct<2, 2, 4>(A, B, C, M, K, N, ta, tb, epi, target, st);
 }
 
 }  // namespace cxm

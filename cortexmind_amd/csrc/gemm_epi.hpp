@@ -49,6 +49,15 @@ __device__ __forceinline__ float4 sum_splits(const float *p, int plane, unsigned
     return a;
 }
 
+// K splits of a product of 128x128 tiles: where the tiles alone cannot fill
+// the chip, at most one workgroup per CU (one fills a CU, and one more would
+// run as a second round), each split at least 256 of K.
+inline size_t gemm_splits(size_t tiles, size_t K, size_t cus) {
+    if (tiles >= cus * 3 / 4 || K < 512) return 1;
+    const size_t splits = cus / tiles < K / 256 ? cus / tiles : K / 256;
+    return splits < 1 ? 1 : splits;
+}
+
 // Tiles and K splits of one product of the direct kernels: about `target`
 // workgroups, each split at least `depth` steps of `step` k (a block per wave).
 struct DirectPlan {
@@ -75,6 +84,6 @@ inline DirectPlan direct_plan(size_t M, size_t N, size_t K, size_t tm, size_t tn
 // A B^T and A^T B.  `ring`: the ring kernel would take the product.  Returns
 // 1 when it is better left to the kernels of gemm.hip.
 int gemm_direct(const float *A, const float *B, float *C, size_t M, size_t K, size_t N, int ta, int tb,
-                const Epilogue &epi, bool ring, cxm_stream_t st);
+                const Epilogue &epi, bool ring, int vecs, cxm_stream_t st);
 
 }  // namespace cxm

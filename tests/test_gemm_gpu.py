@@ -243,3 +243,27 @@ def test_long_k_error(hip, m, k, n, ta, tb):
     length = max(k / min(256 // tiles, k // 256), 264 + k / (4 * 264))
     err = np.linalg.norm(got - ref) / np.linalg.norm(ref)
     assert err <= 1.25 * 2.0**-23 / np.sqrt(48.0) * np.sqrt(length), err
+
+
+@pytest.mark.parametrize("m,k,n,ta,tb,variant", [(1203, 2000, 1500, 0, 1, 7), (1024, 3000, 1024, 1, 0, 7),
+                                                 (1500, 4100, 700, 1, 0, 6), (800, 4100, 801, 0, 0, 1),
+                                                 (1800, 4100, 1800, 0, 1, 1), (4092, 4092, 4096, 0, 1, 3),
+                                                 (1400, 2000, 1409, 0, 0, None), (700, 1000, 700, 0, 1, None),
+                                                 (3000, 252, 3000, 1, 0, None)], ids=lambda v: str(v))
+def test_direct_or_staged(hip, m, k, n, ta, tb, variant):
+    """A product whose 128x128 tiles fill the chip's rounds over a long K is
+    left to the ring or the register-staged kernels (up to a third faster
+    there), the others run on the direct tiles: told apart by the bits, since
+    the direct tiles sum k in another order than the kernels a variant pins."""
+    g = SplitMix64(0xD5 + m + 3 * k + 7 * n)
+    a, b = g.normal((m, k)), g.normal((k, n))
+    got = run(a, b, ta, tb)
+    same = {}
+    try:
+        for v in (1, 3, 6, 7):
+            _pin(v)
+            same[v] = np.array_equal(run(a, b, ta, tb).view(np.uint32), got.view(np.uint32))
+    finally:
+        _pin(-1)
+    assert any(same.values()) == (variant is not None)
+    assert variant is None or same[variant]
