@@ -1406,7 +1406,7 @@ int gemm_ex(const float *A, const float *B, float *C, size_t M, size_t K, size_t
     const bool vb = aligned16(B) && (tb ? K % 4 == 0 : N % 4 == 0);
     if (g_gemm_kc.load(std::memory_order_relaxed) < 0) {  // no kernel pinned
         const int t = gemm_direct(A, B, C, M, K, N, ta, tb, epi, ring_ok, (va ? 1 : 0) + (vb ? 1 : 0), st);
-        if (t != 1) return t;
+        if (t != kDeclined) return t;
     }
     const size_t tiles_m = (M + BM - 1) / BM, tiles_n = (N + BN - 1) / BN;
     const size_t tiles = tiles_m * tiles_n;

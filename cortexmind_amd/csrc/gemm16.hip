@@ -43,6 +43,7 @@
 
 #include "cxm_common.hpp"
 #include "gemm16.hpp"
+#include "gemm_epi.hpp"
 
 namespace cxm {
 namespace {
@@ -941,7 +942,7 @@ int gemm16(const uint16_t *A, const uint16_t *B, uint16_t *C, size_t M, size_t K
     }
     if (pinned < 0) {
         const int t = gemm16_direct(A, B, C, M, K, N, ta, tb, DT, ring256 || ring128, va && vb, st);
-        if (t != 1) return t;
+        if (t != kDeclined) return t;
     }
     if (kernel == 2) return launch_ring<DT, 256>(A, B, C, M, N, K, ta, tb, st);
     if (kernel == 3) return launch_ring<DT, 128>(A, B, C, M, N, K, ta, tb, st);

@@ -27,7 +27,7 @@ __device__ __forceinline__ f32x16 mfma16(u32x4 a, u32x4 b, f32x16 c) {
 // The direct 16-bit kernels (gemm16_direct.hip): any shape, 2-byte alignment,
 // A B, A B^T and A^T B.  `ring`: a ring kernel would take the product; `vec`:
 // both operands' stored rows allow the staged kernels' 128-bit loads.
-// Returns 1 when it is better left to the kernels of gemm16.hip.
+// kDeclined (gemm_epi.hpp): left to the kernels of gemm16.hip.
 int gemm16_direct(const uint16_t *A, const uint16_t *B, uint16_t *C, size_t M, size_t K, size_t N, bool ta, bool tb,
                   int dtype, bool ring, bool vec, cxm_stream_t st);
 

@@ -263,22 +263,21 @@ __global__ __launch_bounds__(NW * kWave) void k_gemm16_direct(const uint16_t *__
 template <int DT, int WI, int WJ, int NW>
 int launch_direct16(const uint16_t *A, const uint16_t *B, uint16_t *C, size_t M, size_t K, size_t N, bool ta, bool tb,
                     size_t target, cxm_stream_t st) {
-    DirectPlan p = direct_plan(M, N, K, 32 * WI, 32 * WJ, 16 * NW, kDepth, target);
+    const DirectPlan p = direct_plan(M, N, K, 32 * WI, 32 * WJ, 16 * NW, kDepth, target);
     float *part = nullptr;
     unsigned *counters = nullptr;
     if (p.splits > 1) {
         Workspace ws;
-        if (get_workspace(st, p.tiles, p.tiles * p.splits * (32 * WI * 32 * WJ) * sizeof(float), &ws)) {
-            (void)hipGetLastError();  // no scratch to be had (a capturing stream's first call): K unsplit
-            p.splits = 1;
-            p.kper = K;
-        } else {
-            part = static_cast<float *>(ws.scratch);
-            counters = ws.counters;
-        }
+        const int rc = get_workspace(st, p.tiles, p.tiles * p.splits * (32 * WI * 32 * WJ) * sizeof(float), &ws);
+        // a capturing stream without scratch: the kernels of gemm16.hip run the
+        // shapes that need none of them and refuse the others
+        if (rc == CXM_E_CAPTURE) return kDeclined;
+        if (rc) return rc;
+        part = static_cast<float *>(ws.scratch);
+        counters = ws.counters;
     }
     const size_t wgs = p.tiles * p.splits;
-    if (wgs > 0x7fffffu) return 1;
+    if (wgs > 0x7fffffu) return kDeclined;
     const dim3 grid(static_cast<unsigned>(wgs)), block(NW * kWave);
     const unsigned nw = static_cast<unsigned>(wgs), tn = static_cast<unsigned>(p.tiles_n), sp = static_cast<unsigned>(p.splits);
     hipStream_t s = reinterpret_cast<hipStream_t>(st);
@@ -332,8 +331,8 @@ int gemm16_direct(const uint16_t *A, const uint16_t *B, uint16_t *C, size_t M, s
                   int dtype, bool ring, bool vec, cxm_stream_t st) {
     // 32-bit byte offsets within a tile; pairs of columns of a [K, M] / [K, N] operand
     constexpr size_t kMaxLd = size_t(1) << 23;
-    if ((ta && tb) || M >= kMaxLd || N >= kMaxLd || K >= kMaxLd || (ta && M < 2) || (!tb && N < 2)) return 1;
-    if (staged_faster(M, K, N, ta, tb, ring, vec)) return 1;
+    if ((ta && tb) || M >= kMaxLd || N >= kMaxLd || K >= kMaxLd || (ta && M < 2) || (!tb && N < 2)) return kDeclined;
+    if (staged_faster(M, K, N, ta, tb, ring, vec)) return kDeclined;
     if (dtype == CXM_DT_BF16) return run_direct16<CXM_DT_BF16>(A, B, C, M, K, N, ta, tb, st);
     return run_direct16<CXM_DT_F16>(A, B, C, M, K, N, ta, tb, st);
 }

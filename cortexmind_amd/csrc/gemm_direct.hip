@@ -310,22 +310,21 @@ __global__ __launch_bounds__(NW * kWave) void k_gemm_direct(const float *__restr
 template <int WI, int WJ, int NW>
 int launch_direct(const float *A, const float *B, float *C, size_t M, size_t K, size_t N, int ta, int tb,
                   const Epilogue &epi, size_t target, cxm_stream_t st) {
-    DirectPlan p = direct_plan(M, N, K, 32 * WI, 32 * WJ, 8 * NW, kDepth, target);
+    const DirectPlan p = direct_plan(M, N, K, 32 * WI, 32 * WJ, 8 * NW, kDepth, target);
     float *part = nullptr;
     unsigned *counters = nullptr;
     if (p.splits > 1) {
         Workspace ws;
-        if (get_workspace(st, p.tiles, p.tiles * p.splits * (32 * WI * 32 * WJ) * sizeof(float), &ws)) {
-            (void)hipGetLastError();  // no scratch to be had (a capturing stream's first call): K unsplit
-            p.splits = 1;
-            p.kper = K;
-        } else {
-            part = static_cast<float *>(ws.scratch);
-            counters = ws.counters;
-        }
+        const int rc = get_workspace(st, p.tiles, p.tiles * p.splits * (32 * WI * 32 * WJ) * sizeof(float), &ws);
+        // a capturing stream without scratch: the kernels of gemm.hip run the
+        // shapes that need none of them and refuse the others
+        if (rc == CXM_E_CAPTURE) return kDeclined;
+        if (rc) return rc;
+        part = static_cast<float *>(ws.scratch);
+        counters = ws.counters;
     }
     const size_t wgs = p.tiles * p.splits;
-    if (wgs > 0x7fffffu) return 1;
+    if (wgs > 0x7fffffu) return kDeclined;
     const dim3 grid(static_cast<unsigned>(wgs)), block(NW * kWave);
     const unsigned nw = static_cast<unsigned>(wgs), tn = static_cast<unsigned>(p.tiles_n), sp = static_cast<unsigned>(p.splits);
     hipStream_t s = reinterpret_cast<hipStream_t>(st);
@@ -407,20 +406,20 @@ int gemm_direct(const float *A, const float *B, float *C, size_t M, size_t K, si
                 const Epilogue &epi, bool ring, int vecs, cxm_stream_t st) {
     // 32-bit byte offsets within a tile; pairs of columns of a [K, M] / [K, N] operand
     constexpr size_t kMaxLd = size_t(1) << 23;
-    if ((ta && tb) || M >= kMaxLd || N >= kMaxLd || K >= kMaxLd || (ta && M < 2) || (!tb && N < 2)) return 1;
+    if ((ta && tb) || M >= kMaxLd || N >= kMaxLd || K >= kMaxLd || (ta && M < 2) || (!tb && N < 2)) return kDeclined;
     const size_t t64 = ((M + 63) / 64) * ((N + 63) / 64);
     const double staged = staged_us(M, N, K, tb, ring, vecs);
     if (t64 < 200) {
-        if (direct_us(M, N, K, ta, tb, 1, 1, 4, 256) > staged) return 1;
+        if (direct_us(M, N, K, ta, tb, 1, 1, 4, 256) > staged) return kDeclined;
         return launch_direct<1, 1, 4>(A, B, C, M, K, N, ta, tb, epi, 256, st);
     }
     if (t64 < 600 && K < 2048) {
-        if (direct_us(M, N, K, ta, tb, 1, 2, 4, 256) > staged) return 1;
+        if (direct_us(M, N, K, ta, tb, 1, 2, 4, 256) > staged) return kDeclined;
         if (K > 4 * 8 * kRun && !tb) return launch_direct<1, 2, 8>(A, B, C, M, K, N, ta, tb, epi, 256, st);
         return launch_direct<1, 2, 4>(A, B, C, M, K, N, ta, tb, epi, 256, st);
     }
     const size_t target = K < 2048 ? 1 : 768;
-    if (direct_us(M, N, K, ta, tb, 2, 2, 4, target) > staged) return 1;
+    if (direct_us(M, N, K, ta, tb, 2, 2, 4, target) > staged) return kDeclined;
     return launch_direct<2, 2, 4>(A, B, C, M, K, N, ta, tb, epi, target, st);
 }
 

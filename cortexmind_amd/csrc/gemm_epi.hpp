@@ -49,6 +49,10 @@ __device__ __forceinline__ float4 sum_splits(const float *p, int plane, unsigned
     return a;
 }
 
+// What the direct kernels return for a product that they leave to the others
+// (no status code).
+constexpr int kDeclined = -1000;
+
 // K splits of a product of 128x128 tiles: where the tiles alone cannot fill
 // the chip, at most one workgroup per CU (one fills a CU, and one more would
 // run as a second round), each split at least 256 of K.

@@ -93,7 +93,10 @@ int grow(WsEntry &w, Region &r, size_t size, size_t bytes, bool cap, cxm_stream_
     }
     void *p = nullptr;
     hipError_t e = hipMalloc(&p, bytes);
-    if (e != hipSuccess) return st(e);
+    if (e != hipSuccess) {
+        (void)hipGetLastError();  // returned here, not again by the next launch's check
+        return st(e);
+    }
     e = hipMemsetAsync(p, 0, bytes, hs);
     if (e != hipSuccess) {
         (void)hipFree(p);

@@ -41,7 +41,13 @@ typedef struct ihipEvent_t *cxm_event_t;   /* a hipEvent_t */
  * stream's workspace, exchange region or tagged slots) that the stream does
  * not have yet, or not large enough: nothing was allocated, filled, waited
  * for or launched.  Make one eager call of the same shapes on the stream
- * before capture. */
+ * before capture.  Three calls use scratch only to be faster and, captured
+ * without, record a form that needs none instead: a product of short K or
+ * with many tiles (and any 16-bit one outside the rings), a reduction over
+ * columns of at least 256 slices of up to 64 columns each, and a softmax of
+ * long rows that are no multiple of 4 floats or not 16-byte aligned.  That
+ * form is slower, stays so in the graph's replays, and sums in another order
+ * than the eager call, which the eager call before capture avoids too. */
 #define CXM_E_CAPTURE (-4)
 
 /* Binary operator codes (Engine/AVX2/broadcast.hpp:29-56, Engine/AVX2/matrix.hpp:38-94). */

@@ -339,3 +339,86 @@ def test_tags_differ_across_streams(hip):
             assert zs[i].numpy(streams[i]).tobytes() == ref.numpy().tobytes(), (rep, i)
         for st in streams:
             st.close()
+
+
+def _gemm32(m, k, n, ta, tb):
+    return lambda L, a, b, c, s: L.cxm_gemm_f32(a, b, c, m, k, n, ta, tb, None, 0, None, s)
+
+
+def _gemm16(m, k, n, ta, tb):
+    return lambda L, a, b, c, s: L.cxm_gemm_t(a, b, c, m, k, n, ta, tb, 1, s)  # bf16
+
+
+# calls whose eager form needs scratch: refused on a capturing stream without,
+# or run there by a kernel that needs none
+NO_SCRATCH = [
+    ("fp32 product, split either way", _gemm32(300, 3001, 200, 0, 0), "refused"),
+    ("fp32 product, split either way", _gemm32(256, 2048, 300, 1, 0), "refused"),
+    ("fp32 product of short K", _gemm32(40, 300, 256, 0, 0), "accepted"),
+    ("fp32 product of short K", _gemm32(65, 500, 67, 1, 0), "accepted"),
+    ("fp32 product of short K", _gemm32(65, 500, 67, 0, 1), "accepted"),
+    ("16-bit product", _gemm16(333, 2000, 517, 0, 0), "accepted"),
+    ("16-bit product", _gemm16(40, 1000, 67, 0, 1), "accepted"),
+    ("16-bit A^T B in the ring", _gemm16(256, 2048, 256, 1, 0), "refused"),
+]
+
+
+@pytest.mark.parametrize("what,fn,state", NO_SCRATCH, ids=[f"{i}-{w}" for i, (w, _, _) in enumerate(NO_SCRATCH)])
+def test_capture_on_a_stream_without_scratch(hip, what, fn, state):
+    """Either CXM_E_CAPTURE with nothing recorded or allocated, or a recorded
+    form that needs no scratch: its replays on new data, with eager calls
+    between them on another stream, agree with the eager form to the rounding
+    of the sums (whose order differs).  Outputs of both forms lie within 1e-5
+    (bf16: two ulps) of the terms' magnitude, here at most 1 each."""
+    from cortexmind_amd._lib import E_CAPTURE, lib
+
+    h, L, s, s2 = hip_rt(), lib(), Stream(), Stream()
+    n = 1 << 22  # floats of each buffer
+    bf16 = what.startswith("16-bit")
+    a, b, c, c2 = (DeviceArray((n,), np.float32) for _ in range(4))
+    g = SplitMix64(0x5C2A)
+
+    def fill(buf, shape=(n,)):
+        x = g.uniform(shape, -1.0, 1.0)
+        if bf16:  # two bf16 values of magnitude below 1 in every word
+            x = (x.view(np.uint32) >> 16 | (g.uniform(shape, -1.0, 1.0).view(np.uint32) & 0xFFFF0000)).view(np.float32)
+        buf.upload(x)
+
+    fill(a), fill(b)
+    try:
+        assert h.hipStreamBeginCapture(s.handle, CAPTURE_RELAXED) == 0
+        st = fn(L, a.ptr, b.ptr, c.ptr, s.handle)
+        graph = ctypes.c_void_p()
+        assert h.hipStreamEndCapture(s.handle, ctypes.byref(graph)) == 0
+        nodes = ctypes.c_size_t(99)
+        h.hipGraphGetNodes.argtypes = [ctypes.c_void_p, ctypes.c_void_p, ctypes.POINTER(ctypes.c_size_t)]
+        h.hipGraphGetNodes.restype = ctypes.c_int
+        assert h.hipGraphGetNodes(graph, None, ctypes.byref(nodes)) == 0
+        assert all(_query(s, which)[0] is None for which in (0, 1, 2))
+        if state == "refused":
+            assert st == E_CAPTURE and nodes.value == 0
+            h.hipGraphDestroy(graph)
+            return
+        assert st == 0 and nodes.value >= 1
+        exe = ctypes.c_void_p()
+        assert h.hipGraphInstantiate(ctypes.byref(exe), graph, None, None, 0) == 0
+        for _ in range(3):
+            fill(a), fill(b)
+            for out in (c, c2):
+                out.fill_bytes(0)
+            assert fn(L, a.ptr, b.ptr, c2.ptr, s2.handle) == 0
+            want = c2.numpy(s2)
+            s.sync()
+            assert h.hipGraphLaunch(exe, s.handle) == 0
+            got = c.numpy(s)
+            if bf16:
+                got, want = ((x.view(np.uint16).astype(np.uint32) << 16).view(np.float32) for x in (got, want))
+                assert np.all(np.abs(got - want) <= 2.0**-7 * np.abs(want) + 1e-2)
+            else:
+                assert np.all(np.abs(got - want) <= 1e-5 * 500)
+            assert np.any(want != 0.0)
+        h.hipGraphExecDestroy(exe)
+        h.hipGraphDestroy(graph)
+    finally:
+        s.close()
+        s2.close()
