@@ -1188,10 +1188,13 @@ int run_cols_flat(const float *x, size_t outer, size_t dim, size_t inner, OutDes
         Scratch sc;
         const size_t nctr = f.chunks <= kTicketGroups ? outer : outer * (kTicketGroups + 1);
         const int rc = acquire(fixed, s, nctr, outer * f.chunks * inner * sizeof(T), 0, &sc);
-        if (rc) {  // no scratch to be had (a capturing stream's first call): one workgroup per slice
-            (void)hipGetLastError();
+        if (rc == CXM_E_CAPTURE && (outer >= 256 || dim <= 64)) {
+            // a capturing stream without scratch, and slices that are many or
+            // short enough: one workgroup per slice
             f.chunks = 1;
             f.chunk_floats = len;
+        } else if (rc) {
+            return rc;
         } else {
             part = static_cast<T *>(sc.part);
             counters = sc.counters;

@@ -44,9 +44,9 @@ typedef struct ihipEvent_t *cxm_event_t;   /* a hipEvent_t */
  * before capture.  Three calls use scratch only to be faster and, captured
  * without, record a form that needs none instead: a product of short K or
  * with many tiles (and any 16-bit one outside the rings), a reduction over
- * columns of at least 256 slices of up to 64 columns each, and a softmax of
- * long rows that are no multiple of 4 floats or not 16-byte aligned.  That
- * form is slower, stays so in the graph's replays, and sums in another order
+ * up to 64 columns of each of 256 or more slices, or of 64 or fewer rows, and
+ * a softmax of long rows that are no multiple of 4 floats or not 16-byte
+ * aligned.  That form is slower, stays so in the graph's replays, and sums in another order
  * than the eager call, which the eager call before capture avoids too. */
 #define CXM_E_CAPTURE (-4)
 

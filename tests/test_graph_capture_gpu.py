@@ -349,6 +349,14 @@ def _gemm16(m, k, n, ta, tb):
     return lambda L, a, b, c, s: L.cxm_gemm_t(a, b, c, m, k, n, ta, tb, 1, s)  # bf16
 
 
+def _cols(outer, dim, inner):
+    return lambda L, a, b, c, s: L.cxm_reduce_sum_f32(a, c, outer, dim, inner, s)
+
+
+def _softmax(rows, cols):
+    return lambda L, a, b, c, s: L.cxm_softmax_fwd_f32(a, c, rows, cols, 1, s)
+
+
 # calls whose eager form needs scratch: refused on a capturing stream without,
 # or run there by a kernel that needs none
 NO_SCRATCH = [
@@ -360,6 +368,13 @@ NO_SCRATCH = [
     ("16-bit product", _gemm16(333, 2000, 517, 0, 0), "accepted"),
     ("16-bit product", _gemm16(40, 1000, 67, 0, 1), "accepted"),
     ("16-bit A^T B in the ring", _gemm16(256, 2048, 256, 1, 0), "refused"),
+    ("narrow columns, few slices", _cols(1, 100000, 10), "refused"),
+    ("narrow columns, few slices", _cols(100, 4000, 4), "refused"),
+    ("narrow columns, many slices", _cols(300, 1200, 10), "accepted"),
+    ("narrow columns, short slices", _cols(7, 62, 33), "accepted"),
+    ("ragged long rows", _softmax(5, 40001), "accepted"),
+    ("ragged long rows, two passes", _softmax(3, 600001), "accepted"),
+    ("aligned long rows", _softmax(5, 40000), "refused"),
 ]
 
 
@@ -368,8 +383,8 @@ def test_capture_on_a_stream_without_scratch(hip, what, fn, state):
     """Either CXM_E_CAPTURE with nothing recorded or allocated, or a recorded
     form that needs no scratch: its replays on new data, with eager calls
     between them on another stream, agree with the eager form to the rounding
-    of the sums (whose order differs).  Outputs of both forms lie within 1e-5
-    (bf16: two ulps) of the terms' magnitude, here at most 1 each."""
+    of the sums (whose order differs): 1e-5 of at most 1200 terms of magnitude
+    below 1 whose sums stay below 500 (bf16: two ulps)."""
     from cortexmind_amd._lib import E_CAPTURE, lib
 
     h, L, s, s2 = hip_rt(), lib(), Stream(), Stream()
