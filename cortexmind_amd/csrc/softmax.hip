@@ -983,6 +983,12 @@ int sm_bwd_rows(const float *y, const float *dy, float *dx, size_t rows, size_t 
 
 // Long rows: split when a row exceeds the wave kernel's register capacity.
 bool use_split(size_t cols) { return cols > kWaveRowMax; }
+// Ragged long rows whose segments make a grid of less than 2^32 threads (a
+// wave per row serves the rest).
+bool split_grid_ok(size_t rows, size_t cols) {
+    constexpr size_t L = kBlock * 4 * kSegNV;
+    return use_split(cols) && rows * ((cols + L - 1) / L) <= 0xffffffu;
+}
 
 // Single pass when the row has at most kXMaxSegs segments and the exchange
 // region stays small (rows * 1.25 KiB).
@@ -1126,11 +1132,10 @@ int softmax_fwd(const float *x, float *y, size_t rows, size_t cols, int log_mode
         if (use_x(rows, cols) && x != y) return sm_fwd_x<true>(x, y, rows, cols, log_mode, st);
         return sm_fwd_split<kSegNV, true>(x, y, rows, cols, log_mode, st);
     }
-    if (cols >= 4) {
+    if (split_grid_ok(rows, cols)) {
         const int rc = use_x(rows, cols) && x != y ? sm_fwd_x<false>(x, y, rows, cols, log_mode, st)
                                                    : sm_fwd_split<kSegNV, false>(x, y, rows, cols, log_mode, st);
-        if (rc == CXM_OK) return rc;
-        (void)hipGetLastError();  // no scratch to be had (a capturing stream's first call): the form without
+        if (rc != CXM_E_CAPTURE) return rc;  // a capturing stream without scratch: the form that needs none
     }
     const dim3 grid(ceil_div(rows, kWavesPerBlock));
     if (log_mode) hipLaunchKernelGGL(k_sm_fwd_any<true>, grid, dim3(kBlock), 0, s, x, y, rows, cols);
@@ -1159,11 +1164,10 @@ int softmax_bwd(const float *y, const float *dy, float *dx, size_t rows, size_t 
         if (use_x(rows, cols) && apart) return sm_bwd_x<true>(y, dy, dx, rows, cols, log_mode, st);
         return sm_bwd_split<kSegNV, true>(y, dy, dx, rows, cols, log_mode, st);
     }
-    if (cols >= 4) {
+    if (split_grid_ok(rows, cols)) {
         const int rc = use_x(rows, cols) && apart ? sm_bwd_x<false>(y, dy, dx, rows, cols, log_mode, st)
                                                   : sm_bwd_split<kSegNV, false>(y, dy, dx, rows, cols, log_mode, st);
-        if (rc == CXM_OK) return rc;
-        (void)hipGetLastError();  // as in the forward
+        if (rc != CXM_E_CAPTURE) return rc;  // as in the forward
     }
     const dim3 grid(ceil_div(rows, kWavesPerBlock));
     if (log_mode) hipLaunchKernelGGL(k_sm_bwd_any<true>, grid, dim3(kBlock), 0, s, y, dy, dx, rows, cols);
