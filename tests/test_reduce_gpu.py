@@ -341,3 +341,29 @@ def test_rows_of_any_length(hip, dim, off):
             assert np.all(np.abs(got - ref)[fin] <= 1e-5 * size[fin])
             if op != "var":
                 assert np.array_equal(np.isnan(ref), np.isnan(got))
+
+
+@pytest.mark.parametrize("dim", [33, 34, 65, 67, 129, 130])
+def test_short_rows_error(hip, dim):
+    """Rows a little longer than a power of two of floats: their last lane's
+    few floats are added to one lane's sum, not to the whole row's, so the
+    error against 64 bits stays below that of sums of four floats met
+    pairwise from the first on, the rest last (fp32, the same inputs)."""
+    rows = 40000
+    x = SplitMix64(0x5047 + dim).normal((rows, dim), 0.5, 1.0)
+    z = DeviceArray((rows,), np.float32)
+    engine.reduce.sum(DeviceArray.from_numpy(x), z, rows, dim, 1)
+    ref = x.astype(np.float64).sum(axis=1)
+    quads = np.zeros((rows, -(-dim // 4) * 4), np.float32)
+    quads[:, :dim] = x
+    quads = quads.reshape(rows, -1, 4)
+    t = (quads[..., 0] + quads[..., 1]) + (quads[..., 2] + quads[..., 3])
+    while t.shape[1] > 1:
+        n = t.shape[1] // 2 * 2
+        t = np.concatenate([t[:, 0:n:2] + t[:, 1:n:2], t[:, n:]], axis=1)
+
+    def error(a):
+        return np.sqrt(np.mean((a - ref) ** 2))
+
+    t = t[:, 0]
+    assert error(z.numpy()) <= 0.96 * error(t), (error(z.numpy()), error(t))
