@@ -549,6 +549,22 @@ __device__ __forceinline__ Pow2 ld_dev(const Pow2 *p) {
             __builtin_bit_cast(double, __hip_atomic_load(u + 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT))};
 }
 
+// p[0], p[stride], ..., p[(N - 1) stride] combined pairwise (N a power of
+// two): log2 N roundings of a sum at its full size or near it, where one
+// after the other makes N - 1.
+template <class Op, int N>
+__device__ __forceinline__ typename Op::T combine_pairwise(const typename Op::T *p, int stride) {
+    static_assert((N & (N - 1)) == 0, "a power of two");
+    typename Op::T v[N];
+#pragma unroll
+    for (int k = 0; k < N; ++k) v[k] = p[k * stride];
+#pragma unroll
+    for (int h = N / 2; h >= 1; h /= 2)
+#pragma unroll
+        for (int k = 0; k < h; ++k) v[k] = Op::combine(v[k], v[k + h]);
+    return v[0];
+}
+
 constexpr unsigned kPartGroup = 16;
 
 // Combines n partials p[0], p[stride], ..., p[(n-1)*stride] into `a` in

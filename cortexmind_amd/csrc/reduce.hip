@@ -616,7 +616,8 @@ constexpr int kColTile = 256;  // columns per workgroup
 // (inner a multiple of 4).  Otherwise (inner >= 4) dword-aligned loads; the
 // last lanes of a slice's last tile read its last four columns and keep the
 // ones that are theirs.  The per-wave results meet in LDS and threads 0..255
-// combine them in wave order.  Workgroup b -> (chunk, tile, outer slice),
+// combine them pairwise (one after the other, a [37, 74, 13243] sum was 6.8e-8
+// from 64 bits, 5.0e-8 so).  Workgroup b -> (chunk, tile, outer slice),
 // chunk fastest: the chunks of one tile are adjacent in launch order, so its
 // combine runs while later tiles still stream.  (No gridDim: the implicit
 // kernel arguments it brings cost 0.2-0.3 us of host time per launch.)  Rows past the last whole
@@ -756,11 +757,7 @@ __global__ __launch_bounds__(NW * kWave) void k_cols(const float *__restrict__ x
     tl_mark(kTlColsArg, 1);
     const bool owner = tid < kColTile;  // threads 0..255 own one column each from here
     T mine = Op::identity();
-    if (owner) {
-        mine = lds[0][tid];
-#pragma unroll
-        for (int k = 1; k < NW; ++k) mine = Op::combine(mine, lds[k][tid]);
-    }
+    if (owner) mine = combine_pairwise<Op, NW>(&lds[0][tid], kColTile);
     const size_t oc = static_cast<size_t>(tile) * tw + tid;
     const bool put = owner && (FAST || (tid < static_cast<int>(tw) && oc < inner));
     if (chunks == 1) {
