@@ -273,10 +273,12 @@ constexpr unsigned kAffGroups = 32;  // groups of chunks of one tile (512 chunks
 // dz = dy*act'(y); dx = dz*scale[j]; dscale[j] = sum_i dz*x; dbias[j] = sum_i dz.
 // A 256-thread workgroup takes a tile of 4 G columns (G lanes x float4) and a
 // chunk of rows; its 256 / G lane groups take interleaved rows, UNR of them
-// in flight, and meet in LDS.  The chunks of a tile are adjacent in launch
-// order, so early tiles' combines overlap later tiles' streaming; the last
-// workgroup of a tile combines them in chunk order, beyond 32 chunks in two
-// levels (groups of kPartGroup).  AL: 16-byte aligned rows (G = 64 only);
+// in flight, and meet in LDS pairwise, as do the chunks' partials in eights
+// (all one after the other, dbias of [40, 16] was 1.2e-7 from 64 bits and of
+// [700, 4096] 1.3e-7; 8e-8 and 1.0e-7 so).  The chunks of a tile are adjacent
+// in launch order, so early tiles' combines overlap later tiles' streaming; the
+// last workgroup of a tile combines them in chunk order, beyond 32 chunks in
+// two levels (groups of kPartGroup).  AL: 16-byte aligned rows (G = 64 only);
 // otherwise dword-aligned accesses, the last lane of a row reading its last
 // four columns and keeping its own (n >= 4).  [6848, 83] backward 43 -> 7.9 us
 // (dword accesses, and one workgroup summing 428 partials, before);
@@ -350,11 +352,8 @@ __global__ __launch_bounds__(kBlock) void k_affine_bwd(const float *__restrict__
     const bool put = tid < TW && oc < n;  // these threads own one column each from here
     float ms = 0.0f, mb = 0.0f;
     if (put) {
-#pragma unroll
-        for (int k = 0; k < NS; ++k) {  // groups in order
-            ms = ms + lds_s[k][tid];
-            mb = mb + lds_b[k][tid];
-        }
+        ms = combine_pairwise<SumOp, NS>(&lds_s[0][tid], TW);
+        mb = combine_pairwise<SumOp, NS>(&lds_b[0][tid], TW);
     }
     if (chunks == 1) {
         if (put) {
@@ -363,7 +362,8 @@ __global__ __launch_bounds__(kBlock) void k_affine_bwd(const float *__restrict__
         }
         return;
     }
-    // the sum of `count` pairs of partials, eight at a time in flight
+    // the sum of `count` pairs of partials, eight at a time in flight and
+    // pairwise
     auto sum = [&](const float *p, unsigned count) {
         ms = 0.0f;
         mb = 0.0f;
@@ -375,11 +375,8 @@ __global__ __launch_bounds__(kBlock) void k_affine_bwd(const float *__restrict__
                 va[u] = in ? ld_dev(&p[((c0 + u) * 2 + 0) * kAffTile + tid]) : 0.0f;
                 vb[u] = in ? ld_dev(&p[((c0 + u) * 2 + 1) * kAffTile + tid]) : 0.0f;
             }
-#pragma unroll
-            for (unsigned u = 0; u < 8; ++u) {
-                ms = ms + va[u];
-                mb = mb + vb[u];
-            }
+            ms = ms + (((va[0] + va[1]) + (va[2] + va[3])) + ((va[4] + va[5]) + (va[6] + va[7])));
+            mb = mb + (((vb[0] + vb[1]) + (vb[2] + vb[3])) + ((vb[4] + vb[5]) + (vb[6] + vb[7])));
         }
     };
     float *pt = part + static_cast<size_t>(tile) * chunks * 2 * kAffTile;

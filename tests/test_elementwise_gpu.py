@@ -277,3 +277,32 @@ def test_row_maps_of_any_width(hip, orc, m, n, off):
     dz64, x64 = dz.astype(np.float64), x.astype(np.float64)
     assert np.all(np.abs(read_s() - (dz64 * x64).sum(0)) <= 1e-5 * np.abs(dz64 * x64).sum(0) + 1e-30)
     assert np.all(np.abs(read_b() - dz64.sum(0)) <= 1e-5 * np.abs(dz64).sum(0) + 1e-30)
+
+
+@pytest.mark.parametrize("m,n", [(40, 16), (100, 16), (240, 10), (240, 28), (256, 60)])
+def test_affine_bwd_few_rows_error(hip, m, n):
+    """dscale and dbias of few narrow rows: no further from 64 bits than runs
+    of 16 rows added in fp32 and the runs' sums in turn, over 80 calls' columns
+    (5% for the two orders' scatter)."""
+    g = SplitMix64(0xAFB + 31 * m + n)
+    got, ref, runs = [], [], []
+    one = dev(np.ones(n, np.float32))
+    y = dev(np.ones((m, n), np.float32))  # ReLU's gate open: dz = dy
+    d, ds, db = empty((m, n)), empty((n,)), empty((n,))
+    for _ in range(80):
+        x, dy = g.normal((m, n)), g.normal((m, n))
+        dx_, ddy = dev(x), dev(dy)
+        call("cxm_affine_act_bwd_f32", dx_.ptr, one.ptr, y.ptr, ddy.ptr, d.ptr, ds.ptr, db.ptr, m, n, 1, None)
+        got.append(np.concatenate([ds.numpy(), db.numpy()]))
+        ref.append(np.concatenate([(dy.astype(np.float64) * x).sum(0), dy.astype(np.float64).sum(0)]))
+        total = np.zeros(2 * n, np.float32)
+        terms = np.concatenate([dy * x, dy], axis=1)
+        for r0 in range(0, m, 16):
+            run = np.zeros(2 * n, np.float32)
+            for r in range(r0, min(r0 + 16, m)):
+                run = run + terms[r]
+            total = total + run
+        runs.append(total)
+    got, ref, runs = np.array(got, np.float64), np.array(ref), np.array(runs, np.float64)
+    error = [np.sqrt(np.mean((a - ref) ** 2)) for a in (got, runs)]
+    assert error[0] <= 1.05 * error[1], error

@@ -351,8 +351,8 @@ def test_short_rows_error(hip, dim):
     pairwise from the first on, the rest last (fp32, the same inputs)."""
     rows = 40000
     x = SplitMix64(0x5047 + dim).normal((rows, dim), 0.5, 1.0)
-    z = DeviceArray((rows,), np.float32)
-    engine.reduce.sum(DeviceArray.from_numpy(x), z, rows, dim, 1)
+    dx, z = DeviceArray.from_numpy(x), DeviceArray((rows,), np.float32)
+    engine.reduce.sum(dx, z, rows, dim, 1)
     ref = x.astype(np.float64).sum(axis=1)
     quads = np.zeros((rows, -(-dim // 4) * 4), np.float32)
     quads[:, :dim] = x
@@ -375,8 +375,8 @@ def test_ragged_column_sums_error(hip, outer, dim, inner):
     further from 64 bits than four interleaved runs of rows added in fp32 (3%
     for the two orders' scatter)."""
     x = SplitMix64(0xC0E + dim).normal((outer, dim, inner), 0.5, 1.0)
-    z = DeviceArray((outer, inner), np.float32)
-    engine.reduce.sum(DeviceArray.from_numpy(x), z, outer, dim, inner)
+    dx, z = DeviceArray.from_numpy(x), DeviceArray((outer, inner), np.float32)
+    engine.reduce.sum(dx, z, outer, dim, inner)
     ref = x.astype(np.float64).sum(axis=1)
     runs = [np.zeros((outer, inner), np.float32) for _ in range(4)]
     for r in range(dim):
