@@ -817,7 +817,8 @@ __device__ __forceinline__ void xent_loss(float nll, float *loss, size_t b, unsi
     if (threadIdx.x == 0) loss[0] = t / static_cast<float>(b);
 }
 
-// c < 4: one thread per row.
+// c < 4, or more rows than the lanes of the other forms can number: one
+// thread per row.
 __global__ __launch_bounds__(kBlock) void k_xent_few(const float *__restrict__ logits,
                                                      const int32_t *__restrict__ labels, float *__restrict__ loss,
                                                      float *__restrict__ dl, size_t b, size_t c, float inv_b, unsigned blocks,
@@ -1244,12 +1245,16 @@ int cxm_softmax_xent_f32(const float *logits, const int32_t *labels, float *loss
     if (!logits || !labels || !loss || !dlogits || b == 0 || c == 0) return CXM_E_INVALID;
     if (c > 0x7fffffffu) return CXM_E_TOO_LARGE;
     // lanes per row: the fewest whose one float4 each covers it, then more
-    // float4 per lane of a whole wave, then a workgroup per row
+    // float4 per lane of a whole wave, then a workgroup per row; a thread per
+    // row where that makes a grid of 2^32 threads or more (2^26 rows of more
+    // than 128 classes, 2^30 of up to 16)
     const size_t v4 = (c + 3) / 4;
-    const size_t rpb = c < 4 ? kBlock : v4 <= 4 ? 64 : v4 <= 8 ? 32 : v4 <= 16 ? 16 : v4 <= 32 ? 8
-                       : c <= kWaveRowMax ? 4 : 1;
+    size_t rpb = c < 4 ? kBlock : v4 <= 4 ? 64 : v4 <= 8 ? 32 : v4 <= 16 ? 16 : v4 <= 32 ? 8 : c <= kWaveRowMax ? 4 : 1;
+    constexpr size_t kMaxGrid = 0xffffffffu / kBlock;
+    const bool few = c < 4 || (b + rpb - 1) / rpb > kMaxGrid;
+    if (few) rpb = kBlock;
     const size_t blocks = (b + rpb - 1) / rpb;
-    if (blocks > 0x7fffffffu) return CXM_E_TOO_LARGE;
+    if (blocks > kMaxGrid) return CXM_E_TOO_LARGE;
     Workspace ws;
     int rc = get_workspace(st, kXentGroups + 1, blocks * sizeof(float), &ws);
     if (rc) return rc;
@@ -1262,7 +1267,7 @@ int cxm_softmax_xent_f32(const float *logits, const int32_t *labels, float *loss
 #define CXM_XENT(G, NV)                                                                                              \
     hipLaunchKernelGGL((k_xent_rows<G, NV>), grid, dim3(kBlock), 0, s, logits, labels, loss, dlogits, b, ci, inv_b, nb,  \
                        part, ws.counters)
-    if (c < 4)
+    if (few)
         hipLaunchKernelGGL(k_xent_few, grid, dim3(kBlock), 0, s, logits, labels, loss, dlogits, b, c, inv_b, nb, part,
                            ws.counters);
     else if (v4 <= 4) CXM_XENT(4, 1);

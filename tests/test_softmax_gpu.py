@@ -445,3 +445,26 @@ def test_ragged_rows_one_rounding(hip, rows, cols, in_place):
         return np.sqrt(np.mean(((a.astype(np.float64) - ref) / ref) ** 2))
 
     assert error(y.numpy()) <= (1.05 if cols <= 4096 else 1.08) * error(quotient), (error(y.numpy()), error(quotient))
+
+
+def test_xent_of_more_rows_than_lanes_can_number(hip):
+    """2^30 + 64 rows of 4 classes: four lanes per row would need a grid of
+    more than 2^32 threads, so a thread takes a row.  All logits equal, label
+    0: dlogits are -3/4 and 1/4 over the row count, exact but for the last
+    product's rounding; the loss is log 4 to the rounding of 2^14 partials
+    added in turn."""
+    from cortexmind_amd.device import DeviceArray
+
+    b, c = (1 << 30) + 64, 4
+    logits, labels = DeviceArray((b * c,), np.float32), DeviceArray((b,), np.int32)
+    dl, loss = DeviceArray((b * c,), np.float32), DeviceArray((1,), np.float32)
+    logits.fill_bytes(0)
+    labels.fill_bytes(0)
+    dl.fill_bytes(0xFF)
+    engine.train.softmax_xent(logits, labels, loss, dl, b, c)
+    assert abs(loss.numpy()[0] / np.log(4.0) - 1.0) <= 2.0**14 * 2.0**-24
+    want = np.tile(np.array([-0.75, 0.25, 0.25, 0.25], np.float32) * np.float32(1.0 / b), 256)
+    for row in (0, 1 << 29, b - 256):
+        got = np.empty(1024, np.float32)
+        call("cxm_memcpy_d2h", got.ctypes.data, dl.ptr + 16 * row, 4096, None)
+        assert np.allclose(got, want, rtol=2.0**-23, atol=0.0)
