@@ -6,22 +6,27 @@
 // reduce.hpp:49-329, reduce.cpp:17-621).  Semantics the
 // kernels keep from it are listed in include/cxm_hip.h.
 //
-// Two kernels cover every shape:
-//  * k_rows: inner == 1 (row reductions, and the flat form as one row).
-//    Each row is cut into `segs` segments; one 256-thread workgroup reduces
-//    a segment with 128-bit loads (an unaligned head and a ragged tail of
-//    fewer than 4 elements each are folded in by segment 0), several in
-//    flight per thread, then a DPP wave reduce and a 4-entry LDS combine.
-//    With segs > 1 the segment results are combined in segment order: by
-//    the row's last workgroup (ticket) or, for a flat reduction, by one
-//    reader workgroup that polls tagged slots.
-//  * k_cols: inner > 1.  A workgroup owns 256 adjacent columns of one outer
-//    slice and a chunk of the reduced rows; each thread keeps one float4 of
-//    columns, the four waves take interleaved rows and meet in LDS.  Chunks
-//    are combined in chunk order by the last workgroup of the column tile.
-//    Narrow slices (see kFlatInner) are read flat instead (k_cols_flat): every
-//    thread's float4s lie a whole number of rows apart, so it keeps four
-//    columns whatever the row length.
+// Kernels, and when each runs:
+//  * k_rows_short: rows (inner == 1, more than one) of 4 to 4096 floats, 4 to 64
+//    lanes each, in registers; k_rows_whole instead for at least 2048 whole
+//    aligned rows of one batch of its loads;
+//  * k_rows: longer rows, and the flat form as one row.  Each row is cut into
+//    `segs` segments; one 256-thread workgroup reduces a segment with 128-bit
+//    loads (an unaligned head and a ragged tail of fewer than 4 elements each
+//    are folded in by segment 0), several in flight per thread, then a DPP
+//    wave reduce and a 4-entry LDS combine.  With segs > 1 the segment results
+//    are combined in segment order: by the row's last workgroup (ticket) or,
+//    for a flat reduction, by one reader workgroup that polls tagged slots;
+//  * k_rows_bytes: rows whose base is not 4-byte aligned;
+//  * k_cols: slices of more than kFlatInner columns.  A workgroup owns up to
+//    256 adjacent columns of one outer slice and a chunk of the reduced rows;
+//    each thread keeps one float4 of columns, the waves take interleaved rows
+//    and meet in LDS.  Chunks are combined by the last workgroups of the
+//    column tile; k_cols_whole instead for whole aligned tiles and chunks;
+//  * k_cols_flat: narrower slices, read flat: every thread's float4s lie a
+//    whole number of rows apart, so it keeps four columns whatever the row
+//    length;
+//  * k_cols_few: rows, or whole slices, of fewer than four floats.
 #include <atomic>
 #include <mutex>
 #include <type_traits>
@@ -1017,7 +1022,7 @@ bool use_whole(const float *x, size_t rows, size_t dim) {
 // workgroup-per-row form, 8.8 here).  A single row is the flat form's.
 template <class Op>
 bool use_short(const float *x, size_t rows, size_t dim) {
-    return rows > 1 && dim >= 4 && dim <= 4096 && rows <= 0x7fffffffu && !use_whole<Op>(x, rows, dim);
+    return rows > 1 && dim >= 4 && dim <= 4096 && !use_whole<Op>(x, rows, dim);
 }
 
 // Row plan: each row cut into `segs` segments of seg4 float4s (a multiple
@@ -1042,6 +1047,8 @@ int run_rows(const float *x, size_t rows, size_t dim, OutDesc out, cxm_stream_t 
     }
     if (use_short<Op>(x, rows, dim)) {
         const int d = static_cast<int>(dim);
+        const size_t lanes = v4 <= 4 ? 4 : v4 <= 8 ? 8 : v4 <= 16 ? 16 : v4 <= 32 ? 32 : 64;
+        if (rows > (0xffffffffu - kBlock) / lanes) return CXM_E_TOO_LARGE;  // 32-bit thread count of a grid
 #define CXM_SHORT(G, NV)                                                                                            \
     hipLaunchKernelGGL((k_rows_short<Op, G, NV>), dim3(static_cast<unsigned>((rows + kBlock / G - 1) / (kBlock / G))), \
                        dim3(kBlock), 0, hs, x, rows, d, out)

@@ -388,3 +388,22 @@ def test_ragged_column_sums_error(hip, outer, dim, inner):
         return np.sqrt(np.mean((a - ref) ** 2))
 
     assert error(z.numpy()) <= 1.03 * error(four), (error(z.numpy()), error(four))
+
+
+def test_more_rows_than_lanes_can_number(hip):
+    """2^26 rows of 129 floats, a wave each, would be a grid of 2^32 threads:
+    CXM_E_TOO_LARGE from the host, with operands of that size; a few rows
+    fewer are reduced (the first and last of them, of zeros but for one
+    element, checked)."""
+    from cortexmind_amd._lib import E_TOO_LARGE
+
+    rows, dim = 1 << 26, 129
+    x, z = DeviceArray((rows * dim,), np.float32), DeviceArray((rows,), np.float32)
+    assert lib().cxm_reduce_sum_f32(x.ptr, z.ptr, rows, dim, 1, None) == E_TOO_LARGE
+    x.fill_bytes(0)
+    one = np.ones(1, np.float32)
+    n = rows - 16
+    call("cxm_memcpy_h2d", x.ptr + 4 * ((n - 1) * dim + 7), one.ctypes.data, 4, None)
+    call("cxm_reduce_sum_f32", x.ptr, z.ptr, n, dim, 1, None)
+    got = z.numpy()[:n]
+    assert got[-1] == 1.0 and not np.any(got[:-1])
