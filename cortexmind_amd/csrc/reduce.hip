@@ -290,7 +290,20 @@ __device__ __forceinline__ typename Op::T row_segment(const float *__restrict__ 
 #pragma unroll
         for (int u = 0; u < UNR; ++u) fold4<Op>(acc, v[u], off + static_cast<int>(4 * (j + u * kBlock)), 1, k4);
     }
-    for (; j < n4; j += kBlock) fold4<Op>(acc, ld4_stream_at(sb, 16u * j), off + static_cast<int>(4 * j), 1, k4);
+    // What is left, fewer than UNR loads per thread: one clamped batch where
+    // they are many (one at a time, 7 of them took as long as the 16 before:
+    // [300, 24000] sum 8.6 -> 6.6 us), in turn where they are few.
+    if (const unsigned left = n4 % (UNR * kBlock); j < n4 && left > UNR / 4 * kBlock) {
+        float4 v[UNR];
+#pragma unroll
+        for (int u = 0; u < UNR; ++u) v[u] = ld4_stream_at(sb, 16u * (j + u * kBlock < n4 ? j + u * kBlock : n4 - 1));
+        __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+        for (int u = 0; u < UNR; ++u)
+            if (j + u * kBlock < n4) fold4<Op>(acc, v[u], off + static_cast<int>(4 * (j + u * kBlock)), 1, k4);
+    } else {
+        for (; j < n4; j += kBlock) fold4<Op>(acc, ld4_stream_at(sb, 16u * j), off + static_cast<int>(4 * j), 1, k4);
+    }
     if (seg == 0) {
         // head elements to threads 0..h-1, tail elements to threads 4..4+t-1
         int i = -1;
@@ -1068,7 +1081,8 @@ int run_rows(const float *x, size_t rows, size_t dim, OutDesc out, cxm_stream_t 
     // split rows only where there are too few of them: a workgroup per row ran
     // [1500, 5000] in 6.4 us against 10.1 in two segments, [688, 10698] in 7.0
     // against 8.2, [1000, 65536] in 38 against 44, but [300, 200000] in 45
-    // against 41
+    // against 41; at the edge (sum, unsplit / split) [256, 4100] 3.4 / 4.8,
+    // [256, 24000] 5.5 / 6.3, [300, 24000] 6.6 / 6.8, [384, 32768] 8.9 / 10.7
     if (rows < 256 || (rows < 512 && dim > 32768)) {
         const size_t want = (kTargetBlocks + rows - 1) / rows;
         const size_t max_segs = (v4 + 255) / 256;
