@@ -1192,7 +1192,9 @@ FlatPlan flat_plan(size_t outer, size_t dim, size_t inner, size_t elem) {
     // about four 256-thread workgroups per CU, each with a batch of loads at
     // least ([100000, 10] sum: 6.0 us with 512 workgroups in all, 5.7 with 1024)
     size_t chunks = outer < 1024 ? 1024 / outer : 1;
-    const size_t most = (steps + kFlatUnr - 1) / kFlatUnr;
+    // (a wave's slice of up to 2 K floats stays whole: in two chunks argmax of
+    // [1, 40, 33] took 5.2 us, 3.5 whole)
+    const size_t most = f.nt == 64 ? 1 : (steps + kFlatUnr - 1) / kFlatUnr;
     if (chunks > most) chunks = most;
     while (chunks > 1 && outer * chunks * inner * elem > kColPartBytes) --chunks;
     const size_t per = (steps + chunks - 1) / chunks;
@@ -1244,6 +1246,17 @@ int run_cols_flat(const float *x, size_t outer, size_t dim, size_t inner, OutDes
 // / 10.0, [7000, 130] 12.2 / 6.6: a tile's 256 columns are combined by as many
 // workgroups as there are tiles, a flat slice's by one.
 constexpr size_t kFlatInner = 64;
+
+// Few slices of many of those columns take the tiles all the same where the
+// flat form would cut them into a few chunks: the chunks of a tile have
+// sixteen waves' loads in flight at once and meet by fewer barriers.  Measured
+// (us, tiles / flat): sum [1, 200, 48] 4.0 / 4.7, [8, 400, 64] 4.1 / 4.8,
+// argmax [1, 356, 48] 5.2 / 6.6, [8, 900, 16] 5.6 / 6.4, but sum [1, 500, 33]
+// 4.9 / 4.8, [1, 1500, 48] 4.6 / 4.7, [1, 2500, 48] 5.3 / 4.6.
+template <class T>
+bool few_wide_slices(size_t outer, size_t dim, size_t inner) {
+    return outer <= 32 && dim <= 1000 && dim * inner > 8192 && inner >= (std::is_same_v<T, ArgPair> ? 16 : 40);
+}
 
 constexpr size_t kColWaves = 16;  // waves per k_cols workgroup
 constexpr size_t kFewRows = 64;
@@ -1334,7 +1347,8 @@ int run_cols(const float *x, size_t outer, size_t dim, size_t inner, OutDesc out
                            static_cast<unsigned>(inner), out);
         return launch_status();
     }
-    if (inner <= kFlatInner) return run_cols_flat<Op>(x, outer, dim, inner, out, s, fixed);
+    if (inner <= kFlatInner && !few_wide_slices<typename Op::T>(outer, dim, inner))
+        return run_cols_flat<Op>(x, outer, dim, inner, out, s, fixed);
     const size_t tiles = (inner + kColTile - 1) / kColTile * outer;
     return run_cols_plan<Op>(x, outer, dim, inner, out, col_plan(tiles, dim), s, fixed);
 }

@@ -407,3 +407,22 @@ def test_more_rows_than_lanes_can_number(hip):
     call("cxm_reduce_sum_f32", x.ptr, z.ptr, n, dim, 1, None)
     got = z.numpy()[:n]
     assert got[-1] == 1.0 and not np.any(got[:-1])
+
+
+@pytest.mark.parametrize("outer,dim,inner", [(1, 205, 40), (1, 204, 40), (32, 1000, 64), (33, 1000, 64), (2, 1001, 48),
+                                             (3, 513, 16), (3, 512, 16), (5, 900, 17), (1, 40, 33), (7, 62, 33), (1, 31, 66)])
+def test_narrow_columns_routes(hip, outer, dim, inner):
+    """Narrow columns at the edges of the flat form, the column tiles and the
+    flat form's single chunk: sum and variance against float64, the index of
+    the maximum exactly (the first of equal ones)."""
+    x = SplitMix64(0x2A4 + dim * inner).normal((outer, dim, inner), 0.5, 1.0)
+    x[:, dim // 2] = x[:, dim // 3]
+    dx = DeviceArray.from_numpy(x)
+    z, zi = DeviceArray((outer, inner), np.float32), DeviceArray((outer, inner), np.int32)
+    x64 = x.astype(np.float64)
+    engine.reduce.sum(dx, z, outer, dim, inner)
+    assert np.all(np.abs(z.numpy() - x64.sum(1)) <= 1e-6 * np.abs(x64).sum(1))
+    engine.reduce.var(dx, z, outer, dim, inner)
+    assert np.allclose(z.numpy(), x64.var(1), rtol=1e-6)
+    engine.reduce.argmax(dx, zi, outer, dim, inner)
+    assert np.array_equal(zi.numpy(), x.argmax(1))
