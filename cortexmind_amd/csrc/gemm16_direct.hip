@@ -299,18 +299,28 @@ int launch_direct16(const uint16_t *A, const uint16_t *B, uint16_t *C, size_t M,
 //    18.5 / 29.9, but 2048x1024x1024 15.2 / 11.9); with A stored [K, M], which
 //    they transpose first, from 600 (1024^3 7.9 / 14.8, 2048x1024x1024 12.2 /
 //    17.0, 1536x1024x1536 16.4 / 17.6, 4096x1024x1024 20.8 / 21.5);
-//  * 256x256 staged tiles on 200 CUs and more when both operands' rows allow
-//    128-bit loads (4000x1000x4000 123 / 60; 3000x500x3008 27 / 40);
-//  * A B^T, whose operands both come as 32 strided rows per load here, on 180
-//    128x128 staged tiles and more when 16-byte aligned (2000x1000x3000 63 / 26,
-//    1296x720x1296 14 / 19), and on 380 with odd K, where the direct loads are
-//    only 2-byte aligned (3001x777x2003 99 / 89; 3000x500x3008 46 / 135).
+//  * where both operands' rows allow 128-bit loads, 256x256 staged tiles on 200
+//    CUs and more (4000x1000x4000 123 / 60), and else whichever estimate is
+//    the lower: direct 64x64 tiles by their number times K (A B^T, whose operands
+//    both come as 32 strided rows per load, by rounds of 256 of them), staged
+//    ones by rounds times K (A B 3000x1600x3000 108 / 77, 3000x520x3000 38 / 43,
+//    2504x1000x2504 54 / 49; A^T B 3000x1600x3000 94 / 78, 2600x1600x2600 72 /
+//    116; A B^T 1456x1600x1684 46 / 28, 900x1600x1700 33 / 28, 900x520x1700
+//    10.5 / 13.1);
+//  * A B^T of odd K, where the direct loads are only 2-byte aligned, on 380
+//    128x128 tiles and more (3001x777x2003 99 / 89; 3000x500x3008 46 / 135).
 bool staged_faster(size_t M, size_t K, size_t N, bool ta, bool tb, bool ring, bool vec) {
     const size_t t64 = ((M + 63) / 64) * ((N + 63) / 64), t128 = ((M + 127) / 128) * ((N + 127) / 128),
                  t256 = ((M + 255) / 256) * ((N + 255) / 256);
     if (ring) return t64 > (ta ? 600 : 128);
-    if (vec && t256 >= 200) return true;
-    return tb && ((vec && t128 >= 180) || (K % 2 != 0 && t128 >= 380));
+    if (!vec) return tb && K % 2 != 0 && t128 >= 380;
+    if (t256 >= 200 || (tb && t128 >= 180)) return true;
+    if (t64 < 180) return false;
+    const double k = static_cast<double>(K);
+    if (tb) return 3.0 + (t64 + 255) / 256 * (0.6 + 0.0088 * k) > (t64 > 512 ? 1.0 : 1.05) * (7.0 + 0.014 * k);
+    const double direct = 3.0 + (ta ? 26e-6 : 29.5e-6) * t64 * k;
+    if (t256 >= 128) return direct > 27.0 + 0.0315 * k;
+    return !ta && direct > (t128 <= 256 ? 10.0 + 0.0268 * k : 11.5 + 0.038 * k);
 }
 
 template <int DT>

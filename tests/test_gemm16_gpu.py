@@ -219,3 +219,26 @@ def test_direct_products(hip, orc, shape, ta, tb, dt):
     a[m // 2, k - 1] = 0x7fff  # NaN in either type
     got = orc.convert(product(a, 0).ravel(), dt, DT_F32).reshape(m, n)
     assert np.all(np.isnan(got[m // 2])) and not np.any(np.isnan(np.delete(got, m // 2, axis=0)))
+
+
+@pytest.mark.parametrize("m,k,n,ta,tb,staged", [(3000, 1600, 3000, 0, 0, 1), (2504, 1600, 2504, 0, 0, 0),
+                                                (1456, 1600, 1688, 0, 1, 0), (3000, 1600, 3000, 1, 0, 1),
+                                                (3000, 304, 3000, 0, 0, None), (904, 520, 1704, 0, 1, None),
+                                                (1800, 1600, 1800, 1, 0, None)], ids=lambda v: str(v))
+def test_direct_or_staged(hip, orc, m, k, n, ta, tb, staged):
+    """Aligned products of a longer K that fill the chip are left to the staged
+    kernels (up to 70% faster there), the others run on the direct tiles: told
+    apart by the bits, since these sum k in another order.  Right either way."""
+    g = SplitMix64(0xD6 + m + 3 * k + 7 * n)
+    a16, a64 = rand16(g, (k, m) if ta else (m, k), DT_BF16, orc)
+    b16, b64 = rand16(g, (n, k) if tb else (k, n), DT_BF16, orc)
+    got = run(a16, b16, m, k, n, DT_BF16, ta, tb)
+    same = []
+    try:
+        for kern in (0, 1):
+            _kernel(kern)
+            same.append(np.array_equal(run(a16, b16, m, k, n, DT_BF16, ta, tb), got))
+    finally:
+        _kernel(-1)
+    assert any(same) == (staged is not None)  # (the staged kernels agree bit for bit)
+    check(got, a64.T if ta else a64, b64.T if tb else b64, DT_BF16, orc)
