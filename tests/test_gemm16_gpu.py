@@ -210,7 +210,7 @@ def test_direct_products(hip, orc, shape, ta, tb, dt):
         call("cxm_gemm_t", da.ptr, db.ptr, c.ptr, m, k, n, ta, tb, dt, None)
         full = c.base.numpy()
         s = 4 + off
-        assert np.all(full[s + m * n:] == 0x1234)
+        assert np.all(full[:s] == 0) and np.all(full[s + m * n:] == 0x1234)  # dev() puts zeros before the view
         return full[s:s + m * n].reshape(m, n)
 
     for off in (0, 1):

@@ -73,7 +73,8 @@ def test_gemm_full_size_float64(hip, m, k, n):
 @pytest.mark.parametrize("m,k,n", [(4096, 256, 4096), (4100, 300, 4095)])
 @pytest.mark.parametrize("ta,tb", [(0, 0), (1, 0), (0, 1), (1, 1)])
 def test_gemm_large_grid_float64(hip, m, k, n, ta, tb):
-    """Grids of >= 1024 tiles take the four-wave kernel; ragged edges included."""
+    """Products of more than 1024 128x128 tiles, ragged edges included: the
+    ring, the direct tiles and, for A^T B^T, the four-wave kernel."""
     g = SplitMix64(m + 3 * k + 7 * n + 11 * ta + 13 * tb)
     a = g.normal((m, k))
     b = g.normal((k, n))
@@ -210,7 +211,7 @@ def test_direct_products(hip, m, k, n, ta, tb, off):
                     act=ACT_RELU if kind == "bias_relu" else ACT_NONE, gate=dev(gate, off) if kind == "gate" else None)
         full = c.base.numpy()
         got = full[4 + off:4 + off + m * n].reshape(m, n)
-        assert np.all(full[4:4 + off] == 7.0) and np.all(full[4 + off + m * n:] == 7.0)
+        assert np.all(full[:4] == 0.0) and np.all(full[4:4 + off] == 7.0) and np.all(full[4 + off + m * n:] == 7.0)
         want = np.maximum(ref + bias, 0.0) if kind == "bias_relu" else np.where(gate > 0, ref, 0.0) if kind == "gate" else ref
         assert np.all(np.abs(got - want) <= lim)
     a[m // 2, k - 1] = np.nan
@@ -267,3 +268,32 @@ def test_direct_or_staged(hip, m, k, n, ta, tb, variant):
         _pin(-1)
     assert any(same.values()) == (variant is not None)
     assert variant is None or same[variant]
+
+
+@pytest.mark.parametrize("m,k,n", [(130, 260, 140), (133, 517, 131), (300, 1100, 261)], ids=lambda v: str(v))
+@pytest.mark.parametrize("ta,tb", [(0, 0), (1, 0), (0, 1), (1, 1)])
+@pytest.mark.parametrize("variant", [0, 1, 2, 3, 4, 5, 6])
+def test_pinned_staged_kernels(hip, m, k, n, ta, tb, variant):
+    """Every register-staged kernel that can be pinned, with 128-bit and
+    element loads, K whole and split, partial tiles in each direction."""
+    g = SplitMix64(0x91D + m + 3 * k + 7 * n + ta + 2 * tb)
+    a, b, bias = g.normal((m, k)), g.normal((k, n)), g.normal((n,), 0.0, 0.5)
+    try:
+        _pin(variant)
+        got = run(a, b, ta, tb, bias=bias, act=ACT_RELU)
+    finally:
+        _pin(-1)
+    ref = np.maximum(a.astype(np.float64) @ b.astype(np.float64) + bias.astype(np.float64), 0.0)
+    assert np.all(np.abs(got - ref) <= bound(a, b) + 1e-6 * np.abs(bias)[None, :])
+
+
+@pytest.mark.parametrize("m,k,n", [(1, 4099, 300), (1, 2051, 17), (300, 4099, 1), (1, 5003, 1), (257, 1030, 1)],
+                         ids=lambda v: str(v))
+@pytest.mark.parametrize("ta,tb", [(0, 0), (1, 0), (0, 1), (1, 1)])
+def test_one_row_or_column(hip, m, k, n, ta, tb):
+    """One row or one column and a ragged K long enough to be split: what the
+    thin kernels refuse and, stored across k, the direct tiles too."""
+    g = SplitMix64(0x1C0 + m + 3 * k + 7 * n + ta + 2 * tb)
+    a, b = g.normal((m, k)), g.normal((k, n))
+    got = run(a, b, ta, tb)
+    assert np.all(np.abs(got - a.astype(np.float64) @ b.astype(np.float64)) <= bound(a, b))

@@ -296,20 +296,24 @@ def test_xent_bad_label_gives_nan(hip):
 
 
 @pytest.mark.parametrize("shape,same_path", [((64, 1024), True), ((16, 40000), False), ((8, 600000), True),
-                                              ((5, 37), True)])
+                                              ((5, 37), True), ((7, 3), True), ((9, 130), True), ((5, 8194), False),
+                                              ((3, 4097), False), ((3, 600001), True)])
 @pytest.mark.parametrize("log", [False, True])
-def test_in_place(hip, orc, shape, same_path, log):
+@pytest.mark.parametrize("off", [0, 1])
+def test_in_place(hip, orc, shape, same_path, log, off):
     """y == x (forward) and dx == dy / dx == y (backward) against the oracle,
-    on every path: the wave kernel, the single-pass long-row shape (which in
-    place runs the two-pass kernels instead), the two-pass shape and the
-    unaligned kernel.  Where the path is the same as out of place, the bits
-    are too."""
+    on every path: rows in registers, aligned, ragged and on a base that is
+    only 4-byte aligned; the single-pass long-row shapes (which in place run
+    the two-pass kernels instead), aligned and ragged, with last segments of
+    1 and 2 floats, whose loads reach back into what another workgroup
+    overwrites; the two-pass shapes; and the wave per row of fewer than 4
+    columns.  Where the path is the same as out of place, the bits are too."""
     g = SplitMix64(0x1A1A + shape[1])
     x = g.normal(shape, 0.0, 4.0)
     dy_h = g.normal(shape, 0.0, 1.0)
     r, c = shape
-    sep = fwd(x, log)
-    buf = dev(x)
+    sep = fwd(x, log, off)
+    buf = dev(x, off)
     engine.softmax.forward(buf, buf, r, c, log=log)
     got = buf.numpy()
     # past F64_COLS columns the oracle's own fp32 row sums drift beyond the
@@ -317,10 +321,10 @@ def test_in_place(hip, orc, shape, same_path, log):
     check_fwd(x, got, orc.softmax_fwd(x, log) if c <= F64_COLS else f64_fwd(x, log), log)
     if same_path:
         assert np.array_equal(got.view(np.uint32), sep.view(np.uint32))
-    want = bwd(sep, dy_h, log)
+    want = bwd(sep, dy_h, log, off)
     ref = orc.softmax_bwd(sep, dy_h, log) if c <= F64_COLS else f64_bwd(sep, dy_h, log)
     for alias in ("dy", "y"):
-        dy_d, dg = dev(sep), dev(dy_h)
+        dy_d, dg = dev(sep, off), dev(dy_h, off)
         out = dg if alias == "dy" else dy_d
         engine.softmax.backward(dy_d, dg, out, r, c, log=log)
         got = out.numpy()
@@ -382,7 +386,7 @@ def test_ragged_and_narrow_rows(hip, cols, off):
     def check_guard(v):
         full = v.base.numpy()
         s = (v.ptr - v.base.ptr) // 4
-        assert np.all(full[:s][4 + off:] == 7.0) and np.all(full[s + n:] == 7.0)
+        assert np.all(full[:s] == 0.0) and np.all(full[s + n:] == 7.0)  # dev() puts zeros before the view
         return full[s:s + n].reshape(rows, cols)
 
     for log in (False, True):
