@@ -91,7 +91,9 @@ __device__ __forceinline__ float4 sm_quot4(float4 e, float s, float inv) {
 // G lanes per row, NV float4 per lane: cols <= 4 G NV; a 128-thread
 // workgroup takes 128 / G rows (measured on [512, 1024] as 3.35 us per launch
 // against 3.5-3.8 us with four or eight waves per workgroup: more workgroups
-// spread the rows over more CUs).  AL: 16-byte aligned rows (G = 64 only);
+// spread the rows over more CUs).  AL: 16-byte aligned rows, non-temporal stores
+// (narrow ones at dword alignment with temporal stores: [60000, 128] backward
+// 18.0 us, 13.7 so; forward 12.1 and 10.5);
 // otherwise dword-aligned 128-bit accesses with a masked tail (tail_off).
 // The ragged forms replaced three sweeps of dword loads by a wave per row:
 // [5000, 1003] forward and backward 36.4 -> 20.4 us (20 bytes per element: 4.9 TB/s).  Rows of up to 128 columns share a
@@ -100,7 +102,6 @@ constexpr int kSmThreads = 128;
 template <int G, int NV, bool LOG, bool AL>
 __global__ __launch_bounds__(kSmThreads) void k_sm_fwd_rows(const float *__restrict__ x, float *__restrict__ y,
                                                             size_t rows, size_t cols) {
-    static_assert(G == kWave || !AL, "narrow rows take the dword-aligned form");
     const size_t r = static_cast<size_t>(blockIdx.x) * (kSmThreads / G) + threadIdx.x / G;
     if (G == kWave && r >= rows) return;  // whole waves leave together
     const size_t row = r < rows ? r : rows - 1;  // lanes past the last row re-read it
@@ -171,7 +172,6 @@ __device__ __forceinline__ float4 sm_dx4(float4 y, float4 g, float r) {
 template <int G, int NV, bool LOG, bool AL>
 __global__ __launch_bounds__(kSmThreads) void k_sm_bwd_rows(const float *__restrict__ y, const float *__restrict__ dy,
                                                             float *__restrict__ dx, size_t rows, size_t cols) {
-    static_assert(G == kWave || !AL, "narrow rows take the dword-aligned form");
     const size_t rw = static_cast<size_t>(blockIdx.x) * (kSmThreads / G) + threadIdx.x / G;
     if (G == kWave && rw >= rows) return;
     const size_t row = rw < rows ? rw : rows - 1;
@@ -979,10 +979,10 @@ int sm_fwd_rows(const float *x, float *y, size_t rows, size_t cols, hipStream_t 
 #define CXM_SM(G, NV, A)                                                                                          \
     hipLaunchKernelGGL((k_sm_fwd_rows<G, NV, LOG, A>), dim3(ceil_div(rows, kSmThreads / G)), dim3(kSmThreads), 0, s, \
                        x, y, rows, cols)
-    if (v4 <= 4) CXM_SM(4, 1, false);
-    else if (v4 <= 8) CXM_SM(8, 1, false);
-    else if (v4 <= 16) CXM_SM(16, 1, false);
-    else if (v4 <= 32) CXM_SM(32, 1, false);
+    if (v4 <= 4) CXM_SM(4, 1, AL);
+    else if (v4 <= 8) CXM_SM(8, 1, AL);
+    else if (v4 <= 16) CXM_SM(16, 1, AL);
+    else if (v4 <= 32) CXM_SM(32, 1, AL);
     else if (v4 <= 64) CXM_SM(64, 1, AL);
     else if (v4 <= 128) CXM_SM(64, 2, AL);
     else if (v4 <= 256) CXM_SM(64, 4, AL);
@@ -998,10 +998,10 @@ int sm_bwd_rows(const float *y, const float *dy, float *dx, size_t rows, size_t 
 #define CXM_SM(G, NV, A)                                                                                          \
     hipLaunchKernelGGL((k_sm_bwd_rows<G, NV, LOG, A>), dim3(ceil_div(rows, kSmThreads / G)), dim3(kSmThreads), 0, s, \
                        y, dy, dx, rows, cols)
-    if (v4 <= 4) CXM_SM(4, 1, false);
-    else if (v4 <= 8) CXM_SM(8, 1, false);
-    else if (v4 <= 16) CXM_SM(16, 1, false);
-    else if (v4 <= 32) CXM_SM(32, 1, false);
+    if (v4 <= 4) CXM_SM(4, 1, AL);
+    else if (v4 <= 8) CXM_SM(8, 1, AL);
+    else if (v4 <= 16) CXM_SM(16, 1, AL);
+    else if (v4 <= 32) CXM_SM(32, 1, AL);
     else if (v4 <= 64) CXM_SM(64, 1, AL);
     else if (v4 <= 128) CXM_SM(64, 2, AL);
     else if (v4 <= 256) CXM_SM(64, 4, AL);
