@@ -1250,12 +1250,13 @@ constexpr size_t kFlatInner = 64;
 // Few slices of many of those columns take the tiles all the same where the
 // flat form would cut them into a few chunks: the chunks of a tile have
 // sixteen waves' loads in flight at once and meet by fewer barriers.  Measured
-// (us, tiles / flat): sum [1, 200, 48] 4.0 / 4.7, [8, 400, 64] 4.1 / 4.8,
-// argmax [1, 356, 48] 5.2 / 6.6, [8, 900, 16] 5.6 / 6.4, but sum [1, 500, 33]
+// (us, tiles / flat): sum [1, 200, 48] 4.0 / 4.7, [20, 552, 16] 4.3 / 5.0,
+// argmax [1, 356, 48] 5.2 / 6.6, [20, 552, 15] 5.6 / 7.0, but sum [1, 500, 33]
 // 4.9 / 4.8, [1, 1500, 48] 4.6 / 4.7, [1, 2500, 48] 5.3 / 4.6.
 template <class T>
 bool few_wide_slices(size_t outer, size_t dim, size_t inner) {
-    return outer <= 32 && dim <= 1000 && dim * inner > 8192 && inner >= (std::is_same_v<T, ArgPair> ? 16 : 40);
+    return outer <= 32 && dim <= 1000 && dim * inner > 8192 &&
+           inner >= (std::is_same_v<T, ArgPair> ? 8 : inner % 4 == 0 ? 16 : 40);
 }
 
 constexpr size_t kColWaves = 16;  // waves per k_cols workgroup

@@ -410,7 +410,7 @@ def test_more_rows_than_lanes_can_number(hip):
 
 
 @pytest.mark.parametrize("outer,dim,inner", [(1, 205, 40), (1, 204, 40), (32, 1000, 64), (33, 1000, 64), (2, 1001, 48),
-                                             (3, 513, 16), (3, 512, 16), (5, 900, 17), (1, 40, 33), (7, 62, 33), (1, 31, 66)])
+                                             (3, 513, 16), (3, 512, 16), (5, 900, 17), (4, 1000, 9), (2, 993, 20), (1, 40, 33), (7, 62, 33), (1, 31, 66)])
 def test_narrow_columns_routes(hip, outer, dim, inner):
     """Narrow columns at the edges of the flat form, the column tiles and the
     flat form's single chunk: sum and variance against float64, the index of
